@@ -567,7 +567,7 @@ static int placement(loader *ld) {
     return 0;
 }
 
-/* The prefill GEMM's tiled copies of the layer matrices (Q4_K / Q6_K, sdy_mat_gemm_layout): a second
+/* The many-token kernels' tiled copies of the layer matrices (quantized types, sdy_mat_gemm_layout): a second
  * copy of those weights, from which the GEMM's loads read whole cache lines. They only make prompts
  * faster (without one the GEMM reads the planes, with the same results), so they are made where the
  * device has room: the attention and dense FFN matrices of every layer first, then the expert stacks

@@ -966,19 +966,38 @@ __global__ void k_gemm_check(GemmArgs g, int *bad) {
 
 // =============================================================================== host
 
-// Offsets and sizes of the planes of the GEMM's copy of a matrix of `rows` rows (tiles of 32 rows:
-// the 16-byte unit records [tile][unit][32], the per-super-block records [tile][super-block][32]).
-static size_t gemm_layout_planes(int type, int n_in, long rows, size_t off[5], size_t sz[5]) {
-    const size_t tiles = (size_t)(rows + 31) / 32, T = (size_t)n_in / 64, nb = (size_t)n_in / 256;
-    const size_t unit = tiles * T * 512, sbk = tiles * nb * 32;
-    const size_t s4[5] = {unit, unit, sbk * 16, 0, 0}, s6[5] = {unit, unit, unit, sbk * 16, sbk * 2};
+// The planes of the tiled copy of a matrix of `rows` rows (tiles of 32 rows: records [tile][unit][32], the
+// K-quants' per-super-block records [tile][super-block][32]): offsets, sizes, and each plane's records per row and
+// record bytes. Returns the copy's bytes, 0 for types without one.
+static size_t gemm_layout_planes(int type, int n_in, long rows, size_t off[5], size_t sz[5], int nrec[5], int rsz[5]) {
+    const int T = (n_in + 63) / 64, nb = n_in / 256;
+    static const int bytes[5][5] = {
+        {16, 16, 16, 0, 0}, {16, 16, 16, 16, 2}, {16, 16, 16, 16, 4}, {16, 16, 0, 0, 4}, {16, 16, 8, 0, 4}};
+    int k;  // row of the table
+    switch (type) {
+    case SDY_Q4_K: k = 0; break;
+    case SDY_Q6_K: k = 1; break;
+    case SDY_Q8_0: k = 2; break;
+    case SDY_Q4_0: k = 3; break;
+    case SDY_Q5_0: k = 4; break;
+    default: return 0;
+    }
+    const size_t tiles = (size_t)(rows + 31) / 32;
     size_t o = 0;
     for (int i = 0; i < 5; i++) {
-        sz[i] = type == SDY_Q4_K ? s4[i] : s6[i];
+        rsz[i] = bytes[k][i];
+        nrec[i] = (k == 0 && i == 2) || (k == 1 && i >= 3) ? nb : T;
+        sz[i] = tiles * nrec[i] * 32 * rsz[i];
         off[i] = o;
         o += (sz[i] + 255) & ~(size_t)255;
     }
     return o;
+}
+
+extern "C" size_t sdy_gemm_layout_planes(int type, int n_in, long rows, size_t off[5]) {
+    size_t sz[5];
+    int nrec[5], rsz[5];
+    return gemm_layout_planes(type, n_in, rows, off, sz, nrec, rsz);
 }
 
 // The kernel arguments of m; with its GEMM copy (k_gemm3) when it has one and `layout` is set.
@@ -995,7 +1014,8 @@ static GemmArgs gemm_args(const sdy_mat *m, bool layout = false) {
                     m->type == SDY_Q4_K ? 0 : sbk * 2};
     if (layout && m->gbase) {
         size_t off[5];
-        gemm_layout_planes(m->type, m->n_in, m->grows, off, sz);
+        int nrec[5], rsz[5];
+        gemm_layout_planes(m->type, m->n_in, m->grows, off, sz, nrec, rsz);
         for (int i = 0; i < 5; i++) g.p[i] = (const uint8_t *)m->gbase + off[i];
         g.blk = 1;
         g.grow0 = m->grow0;
@@ -1005,7 +1025,7 @@ static GemmArgs gemm_args(const sdy_mat *m, bool layout = false) {
     return g;
 }
 
-// Plane record r = row * n_rec + j (rs bytes, rs 16 or 2) into the tiled copy: [row / 32][j][row % 32].
+// Plane record r = row * n_rec + j (rs bytes: 16, 8, 4 or 2) into the tiled copy: [row / 32][j][row % 32].
 __global__ __launch_bounds__(256) void k_gemm_layout(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
                                                      long n_rows, int n_rec, int rs) {
     const long i = blockIdx.x * 256L + threadIdx.x;
@@ -1013,35 +1033,42 @@ __global__ __launch_bounds__(256) void k_gemm_layout(const uint8_t *__restrict__
     const long row = i / n_rec;
     const int j = (int)(i - row * n_rec);
     const size_t o = (((size_t)(row >> 5) * n_rec + j) * 32 + (row & 31)) * rs;
-    if (rs == 16) *reinterpret_cast<uint4 *>(dst + o) = *reinterpret_cast<const uint4 *>(src + (size_t)i * 16);
-    else *reinterpret_cast<uint16_t *>(dst + o) = *reinterpret_cast<const uint16_t *>(src + (size_t)i * 2);
+    const uint8_t *r = src + (size_t)i * rs;
+    if (rs == 16) *reinterpret_cast<uint4 *>(dst + o) = *reinterpret_cast<const uint4 *>(r);
+    else if (rs == 8) *reinterpret_cast<uint2 *>(dst + o) = *reinterpret_cast<const uint2 *>(r);
+    else if (rs == 4) *reinterpret_cast<uint32_t *>(dst + o) = *reinterpret_cast<const uint32_t *>(r);
+    else *reinterpret_cast<uint16_t *>(dst + o) = *reinterpret_cast<const uint16_t *>(r);
+}
+
+// whether m can have a tiled copy: a quantised matrix in device memory (the kernels that multiply many
+// tokens read one in host memory in place)
+static bool gemm_layout_ok(const sdy_mat *m) {
+    if (!m || !m->base || m->hbase) return false;
+    if (m->type == SDY_Q4_K || m->type == SDY_Q6_K) return m->gemm_ok != 0;
+    return m->type == SDY_Q8_0 || m->type == SDY_Q4_0 || m->type == SDY_Q5_0;
 }
 
 extern "C" size_t sdy_mat_gemm_layout_bytes(const sdy_mat *m) {
-    if (!m || !m->base || m->hbase || (m->type != SDY_Q4_K && m->type != SDY_Q6_K) || !m->gemm_ok || m->gbase)
-        return 0;
-    size_t off[5], sz[5];
-    return gemm_layout_planes(m->type, m->n_in, m->n_rows, off, sz);
+    if (!gemm_layout_ok(m) || m->gbase) return 0;
+    size_t off[5];
+    return sdy_gemm_layout_planes(m->type, m->n_in, m->n_rows, off);
 }
 
 extern "C" int sdy_mat_gemm_layout(sdy_mat *m, sdy_stream s) {
-    // (a matrix in host memory keeps no copy: the GEMM reads its planes in place)
-    if (!m || !m->base || m->hbase || (m->type != SDY_Q4_K && m->type != SDY_Q6_K) || !m->gemm_ok) return 0;
+    if (!gemm_layout_ok(m)) return 0;
     if (m->grow0 != 0 || (m->gbase && m->grows != m->n_rows))
         return sdy_fail(-1, "gemm_layout: made for a whole matrix, not a row view");
     size_t off[5], sz[5];
-    const size_t bytes = gemm_layout_planes(m->type, m->n_in, m->n_rows, off, sz);
+    int nrec[5], rsz[5];
+    const size_t bytes = gemm_layout_planes(m->type, m->n_in, m->n_rows, off, sz, nrec, rsz);
     int rc;
     if (!m->gbase) {
         if ((rc = sdy_malloc(&m->gbase, bytes))) return rc;
         m->gbytes = bytes;
         m->grows = m->n_rows;
-        // the padding rows of the last tile: zero (never read: the GEMM clamps its rows)
+        // the padding rows of the last tile: zero (never read: the kernels clamp their rows)
         if ((rc = sdy_memset(m->gbase, 0, bytes, s))) return rc;
     }
-    const int T = m->n_units, nb = m->n_in / 256;
-    const int nrec[5] = {T, T, m->type == SDY_Q4_K ? nb : T, nb, nb};
-    const int rsz[5] = {16, 16, 16, 16, 2};
     for (int i = 0; i < 5; i++) {
         if (!sz[i]) continue;
         const long total = m->n_rows * (long)nrec[i];

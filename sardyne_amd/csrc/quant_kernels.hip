@@ -2608,6 +2608,15 @@ static int launch_mv(const sdy_mat *m, const sdy_mv_args *a, int n_tok, const ui
 
 template <int WT>
 static int mv_type(const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
+    // Five and more tokens of the 32-element types: the matrix cores (mm_blocks.hip). With 3 or 4 tokens the 4-token
+    // matvec below is still the faster one on small matrices (2048 x 2048: 11.1 us against 12.1; the 8-token one takes
+    // 15.2 against 12.3).
+    if constexpr (!is_k(WT)) {
+        if (a->n_tok >= 5) {
+            const int rc = sdy_mm_blocks(m, a, (sdy_stream)st);
+            if (rc <= 0) return rc;
+        }
+    }
     size_t xrow = sdy_raw_row_bytes(is_k(WT) ? SDY_Q8_K : SDY_Q8_0, m->n_in);
     const int T = m->n_units, nb = n_blocks(WT, m->n_in);
     // largest token capacity (8, 4, 2, 1) whose LDS fits; tokens are processed in chunks of it

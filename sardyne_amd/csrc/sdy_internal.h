@@ -3,6 +3,8 @@
 #include <stddef.h>
 #include <string.h>
 
+#include "sdy_shim.h"
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -16,6 +18,10 @@ int sdy_lds_limit(const void *fn, size_t bytes, size_t *granted);
 int sdy_attn_split_scratch_setup(void);
 /* Bytes of one row in the GGUF layout. */
 size_t sdy_raw_row_bytes(int type, int n_in);
+/* Offsets of the planes of a matrix' tiled copy (sdy_mat_gemm_layout) of `rows` rows; returns its bytes. */
+size_t sdy_gemm_layout_planes(int type, int n_in, long rows, size_t off[5]);
+/* Many tokens of a Q8_0 / Q4_0 / Q5_0 matrix (mm_blocks.hip): 0, 1 when it does not take the call, or an error. */
+int sdy_mm_blocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s);
 #ifdef __cplusplus
 }
 /* The host function of the last matvec / GEMM / attention kernel launched by this thread (the name

@@ -66,7 +66,7 @@ typedef struct {
     size_t plane_off[5];
     int gemm_ok;    /* Q4_K / Q6_K: 1 when the GEMM's one-fragment scheme is exact for every block,
                        2 when some block needs the wide variant (Q6_K: twice the MFMA work); 0 other types */
-    void *gbase;    /* the GEMM's copy of the planes (sdy_mat_gemm_layout) or NULL: rows in tiles of 32,
+    void *gbase;    /* the many-token kernels' copy of the planes (sdy_mat_gemm_layout) or NULL: rows in tiles of 32,
                        each tile's records unit-major ([tile][unit][32 rows][16 bytes], the per-super-block
                        records [tile][super-block][32 rows]) */
     size_t gbytes;
@@ -98,9 +98,10 @@ int sdy_mat_from_device(sdy_mat *m, int type, int n_in, long n_rows, const void 
  * synchronisation, no exactness check). */
 int sdy_mat_repack_async(sdy_mat *m, long r0, long n, long step, long grp, long gstride, const void *dev_raw,
                          sdy_stream s);
-/* The GEMM's copy of a Q4_K / Q6_K matrix (gbase), made from its planes after the last upload, for
- * the prefill GEMM's loads (a load instruction then reads whole cache lines). Another upload into
- * the matrix frees it (the GEMM reads the planes until it is made again). Other types: no-op. */
+/* The many-token kernels' copy of a quantized matrix (gbase), made from its planes after the last upload
+ * (a load instruction of the K-quants' GEMM, or of the block types' MFMA matvec, then reads whole
+ * cache lines). Another upload into the matrix frees it (those kernels read the planes until it is made again,
+ * with the same results). Float types and matrices in host memory: no-op. */
 int sdy_mat_gemm_layout(sdy_mat *m, sdy_stream s);
 /* Bytes sdy_mat_gemm_layout would allocate for m (0: no copy for this type or matrix). */
 size_t sdy_mat_gemm_layout_bytes(const sdy_mat *m);

@@ -1395,6 +1395,66 @@ def test_matrix_in_host_memory_same_bits(kind):
         L.sdy_mat_free(ctypes.byref(host))
 
 
+@pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
+@pytest.mark.parametrize("n_in,n_out,n_tok", [(32, 33, 5), (96, 31, 31), (544, 130, 64), (2048, 129, 33), (2080, 66, 32),
+                                              (4064, 96, 65), (11008, 70, 255), (11008, 200, 256), (2048, 2600, 517)])
+def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
+    """Five and more tokens of the 32-element types (int8 MFMA), around the edges of its row, token and
+    block tiles and of its wave splits, against float64: the integer dots and the scale products are exact, each
+    output is a sum over the row's nb blocks whose longest chain is 8 + nb / 16 + 4 additions, each rounding by
+    at most 2^-24 of a partial sum (itself at most the sum of the terms' magnitudes). The tiled copy, the
+    planes, a row range and rows at 2 bytes' alignment give the same bits; so does the SwiGLU epilogue."""
+    t, w, xq = _matvec_case(kind, n_in, n_out, n_tok, seed=n_in + n_tok)
+    nb = n_in // 32
+    # some scales subnormal in f16
+    wb = w.reshape(n_out, nb, -1)
+    wb[::3, ::2, 0:2] = np.array([7], np.uint16).view(np.uint8)
+    xb = xq.reshape(n_tok, nb, 34)
+    xb[::2, ::5, 0:2] = np.array([300], np.uint16).view(np.uint8)
+    wd = O.dequant(w, t, n_in * n_out).astype(np.float64).reshape(n_out, nb, 32)
+    xd = xb[:, :, 2:].copy().view(np.int8).astype(np.float64) * xb[:, :, :2].copy().view(np.float16).astype(np.float64)
+    exp, mag = np.zeros((n_tok, n_out)), np.zeros((n_tok, n_out))
+    for b in range(nb):
+        p = xd[:, b] @ wd[:, b].T
+        exp += p
+        mag += np.abs(p)
+    L = lib()
+    off = 2  # bytes before the second copy of the rows
+    dq = capi.DeviceBuffer.from_array(np.concatenate([xq.reshape(-1), np.zeros(off + xq.size % 2, np.uint8)]))
+    dq2 = capi.DeviceBuffer.from_array(np.concatenate([np.zeros(off, np.uint8), xq.reshape(-1)]))
+
+    def run(m, q, r0=0, r1=n_out, epilogue=capi.EPI_NONE, **kw):
+        cols = n_out if epilogue == capi.EPI_NONE else (r1 - r0) // 2
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, cols), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=q, n_tok=n_tok, out=out.ptr, out_stride=cols, row0=r0, row1=r1, epilogue=epilogue, **kw)
+        capi.check(L.sdy_matvec(ctypes.byref(m.m), ctypes.byref(a), None))
+        return out.to_array(np.float32, (n_tok, cols))
+
+    tiled, planes = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=False)
+    assert tiled.m.gbase and not planes.m.gbase
+    got = run(tiled, dq.ptr)
+    assert b"k_mm_blocks" in L.sdy_last_kernel()
+    assert np.all(np.abs(got - exp) <= (12 + nb / 16) * 2.0 ** -24 * mag + 1e-45)
+    assert np.array_equal(bits(run(planes, dq.ptr)), bits(got))
+    assert np.array_equal(bits(run(tiled, dq2.ptr + off)), bits(got))
+    part = run(planes, dq.ptr, 3, n_out - 2)
+    assert np.array_equal(bits(part[:, 3:n_out - 2]), bits(got[:, 3:n_out - 2]))
+    assert np.all(np.isnan(part[:, :3])) and np.all(np.isnan(part[:, n_out - 2:]))
+    view = L.sdy_mat_rows(ctypes.byref(tiled.m), 5, n_out - 5)  # the copy addressed by rows of the whole matrix
+    out = capi.DeviceBuffer(n_tok * (n_out - 5) * 4)
+    a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out - 5, row0=0, row1=n_out - 5)
+    capi.check(L.sdy_matvec(ctypes.byref(view), ctypes.byref(a), None))
+    assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out - 5))), bits(got[:, 5:]))
+    rng = np.random.default_rng(3)
+    bias, resid = rng.standard_normal(n_out).astype(np.float32), rng.standard_normal((n_tok, n_out)).astype(np.float32)
+    db, dr = capi.DeviceBuffer.from_array(bias), capi.DeviceBuffer.from_array(resid)
+    assert np.array_equal(bits(run(tiled, dq.ptr, bias=db.ptr, resid=dr.ptr)), bits(resid + (got + bias)))
+    even = n_out & ~1
+    gate, up = np.ascontiguousarray(got[:, 0:even:2]), np.ascontiguousarray(got[:, 1:even:2])
+    L.op_silu_mul(ptr(gate), ptr(up), gate.size)
+    assert np.array_equal(bits(run(tiled, dq.ptr, 0, even, capi.EPI_SWIGLU)), bits(gate))
+
+
 @pytest.mark.parametrize("variant", ["11", "12", "13", "14", "15", "16", "17", "18", "19", "20"])
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 def test_gemm_tile_variants_bit_exact(kind, variant, monkeypatch):
