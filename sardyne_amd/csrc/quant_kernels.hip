@@ -2617,6 +2617,17 @@ static int mv_type(const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
             if (rc <= 0) return rc;
         }
     }
+    // Several tokens of the K-quants: the matrix cores too (mm_superblocks.hip), with the same bits. Q4_K from two
+    // tokens (22016 x 2048: 10.7 us against 17.0 with the quantiser's launch; 2048 x 2048: 7.3 against 7.7); Q6_K,
+    // whose super-blocks take the kernel longer, from two on matrices of up to 4096 rows (2048 x 11008: 17.6 against
+    // 18.4) and from five on larger ones (151936 x 2048: 84 us whatever the tokens, against 57, 74, 85 and 100
+    // for 2, 3, 4 and 5).
+    if constexpr (is_k(WT)) {
+        if (a->n_tok >= (WT == SDY_Q4_K || a->row1 - a->row0 <= 4096 ? 2 : 5)) {
+            const int rc = sdy_mm_superblocks(m, a, (sdy_stream)st);
+            if (rc <= 0) return rc;
+        }
+    }
     size_t xrow = sdy_raw_row_bytes(is_k(WT) ? SDY_Q8_K : SDY_Q8_0, m->n_in);
     const int T = m->n_units, nb = n_blocks(WT, m->n_in);
     // largest token capacity (8, 4, 2, 1) whose LDS fits; tokens are processed in chunks of it

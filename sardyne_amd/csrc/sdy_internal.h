@@ -22,6 +22,8 @@ size_t sdy_raw_row_bytes(int type, int n_in);
 size_t sdy_gemm_layout_planes(int type, int n_in, long rows, size_t off[5]);
 /* Many tokens of a Q8_0 / Q4_0 / Q5_0 matrix (mm_blocks.hip): 0, 1 when it does not take the call, or an error. */
 int sdy_mm_blocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s);
+/* Several tokens of a Q4_K / Q6_K matrix (mm_superblocks.hip): 0, 1 when it does not take the call, or an error. */
+int sdy_mm_superblocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s);
 #ifdef __cplusplus
 }
 /* The host function of the last matvec / GEMM / attention kernel launched by this thread (the name

@@ -1455,6 +1455,53 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
     assert np.array_equal(bits(run(tiled, dq.ptr, 0, even, capi.EPI_SWIGLU)), bits(gate))
 
 
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("n_in,n_out,n_tok", [(256, 3, 2), (2304, 33, 5), (2048, 16, 15), (4096, 130, 16), (11008, 31, 7),
+                                              (2048, 8300, 3), (1024, 4200, 6), (768, 70, 33)])
+def test_superblock_mfma_few_tokens(kind, n_in, n_out, n_tok):
+    """Several tokens of the K-quants (int8 MFMA) around the edges of the row, token and super-block tiles, with scales
+    and quants over their whole range and a token of one sign: the oracle's bits, from the tiled copy and the planes,
+    over a row range and a row view, with bias and residual, and with the SwiGLU epilogue."""
+    t = TYPES[kind]
+    w = _full_range_blocks(kind, n_out, n_in, n_in + n_tok)
+    x = np.random.default_rng(n_tok).standard_normal((n_tok, n_in)).astype(np.float32)
+    x[0] = np.abs(x[0])
+    xq = O.quantize(x, O.Q8_K)
+    exp = O.matmul_q(w, t, xq, n_in, simd=1)
+    L = lib()
+    dq = capi.DeviceBuffer.from_array(xq)
+
+    def run(m, r0=0, r1=n_out, epilogue=capi.EPI_NONE, **kw):
+        cols = n_out if epilogue == capi.EPI_NONE else (r1 - r0) // 2
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, max(cols, 1)), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=cols, row0=r0, row1=r1, epilogue=epilogue, **kw)
+        capi.check(L.sdy_matvec(ctypes.byref(m.m), ctypes.byref(a), None))
+        return out.to_array(np.float32, (n_tok, cols))
+
+    tiled, planes = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=False)
+    assert np.array_equal(bits(run(tiled)), bits(exp))
+    assert (b"k_mm_superblocks" in L.sdy_last_kernel()) == (kind == "Q4_K" or n_out <= 4096 or n_tok >= 5)
+    assert np.array_equal(bits(run(planes)), bits(exp))
+    rng = np.random.default_rng(3)
+    bias, resid = rng.standard_normal(n_out).astype(np.float32), rng.standard_normal((n_tok, n_out)).astype(np.float32)
+    db, dr = capi.DeviceBuffer.from_array(bias), capi.DeviceBuffer.from_array(resid)
+    assert np.array_equal(bits(run(tiled, bias=db.ptr, resid=dr.ptr)), bits(resid + (exp + bias)))
+    if n_out < 4:
+        return
+    part = run(planes, 3, n_out - 1)
+    assert np.array_equal(bits(part[:, 3:n_out - 1]), bits(exp[:, 3:n_out - 1]))
+    assert np.all(np.isnan(part[:, :3])) and np.all(np.isnan(part[:, n_out - 1:]))
+    view = L.sdy_mat_rows(ctypes.byref(tiled.m), 2, n_out - 2)
+    out = capi.DeviceBuffer(n_tok * (n_out - 2) * 4)
+    a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out - 2, row0=0, row1=n_out - 2)
+    capi.check(L.sdy_matvec(ctypes.byref(view), ctypes.byref(a), None))
+    assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out - 2))), bits(exp[:, 2:]))
+    even = n_out & ~1
+    gate, up = np.ascontiguousarray(exp[:, 0:even:2]), np.ascontiguousarray(exp[:, 1:even:2])
+    L.op_silu_mul(ptr(gate), ptr(up), gate.size)
+    assert np.array_equal(bits(run(tiled, 0, even, capi.EPI_SWIGLU)), bits(gate))
+
+
 @pytest.mark.parametrize("variant", ["11", "12", "13", "14", "15", "16", "17", "18", "19", "20"])
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 def test_gemm_tile_variants_bit_exact(kind, variant, monkeypatch):
