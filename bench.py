@@ -657,7 +657,7 @@ def gemm_gate_up_ms(spec, n_tok, reps):
     def launch(_):
         capi.check(L.sdy_gemm(ctypes.byref(m.m), ctypes.byref(a), ws.ptr, st))
 
-    launch(0)  # makes the activations' f16 expansion in ws; the timed launches reuse it (GEMM alone)
+    launch(0)  # makes the activations' expansion in ws; the timed launches reuse it (GEMM alone)
     a.ws_ready = 1
     for i in range(2):
         launch(i)
@@ -782,7 +782,7 @@ def main():
     ap.add_argument("--layers", type=int, default=0, help="override the layer count (smoke runs only)")
     ap.add_argument("--scales", default="workload", choices=["workload", "file"],
                     help="K-quant scale distribution of the prefill model: the workload's, or the "
-                         "normalised scales of quantized model files (the GEMM's wide variant)")
+                         "normalised scales of quantized model files")
     ap.add_argument("--no-decode", action="store_true",
                     help="default workload: leave out the decode_3b / decode_moe sub-objects")
     args = ap.parse_args()

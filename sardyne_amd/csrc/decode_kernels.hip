@@ -11,7 +11,7 @@
 namespace {
 
 // VT = SDY_Q8_K, SDY_Q8_0 or SDY_F32 (normalise only). xb (f32 result) may be null for the
-// quantising variants; with e.y16 set, Q8_K also writes the GEMM's expansion of its blocks. Grid: one 256-thread block per row. For Q8_K rows of up to 4096 elements
+// quantising variants; with e.y8 set, Q8_K also writes the GEMM's expansion of its blocks. Grid: one 256-thread block per row. For Q8_K rows of up to 4096 elements
 // the row is read once: the float4 chunks of the sum of squares are the elements each lane
 // quantises (superblock wave + 4k, elements 4 lane .. 4 lane + 3).
 template <int VT>
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void k_norm_quant(const float *__restrict__ x,
                 *reinterpret_cast<uint32_t *>(ob + 4 + 4 * lane) = r[k].packed;
                 if ((lane & 3) == 0) *reinterpret_cast<int16_t *>(ob + 260 + 2 * (lane >> 2)) = (int16_t)r[k].gsum;
                 if (lane == 0) *reinterpret_cast<float *>(ob) = r[k].d;
-                if (e.y16) e.put(r[k], lane, (size_t)t * nb + wave + 4 * k);
+                if (e.y8) e.put(r[k], lane, (size_t)t * nb + wave + 4 * k);
             }
         for (int s = wave + 4 * NREG; s < nb; s += 4) {
             const float4 o = values(s, from_mem(s), *reinterpret_cast<const float4 *>(w + 256 * s + 4 * lane));
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void k_norm_quant(const float *__restrict__ x,
             *reinterpret_cast<uint32_t *>(ob + 4 + 4 * lane) = r1.packed;
             if ((lane & 3) == 0) *reinterpret_cast<int16_t *>(ob + 260 + 2 * (lane >> 2)) = (int16_t)r1.gsum;
             if (lane == 0) *reinterpret_cast<float *>(ob) = r1.d;
-            if (e.y16) e.put(r1, lane, (size_t)t * nb + s);
+            if (e.y8) e.put(r1, lane, (size_t)t * nb + s);
         }
     } else if constexpr (VT == SDY_Q8_0) {
         const int nblk = n / 32, l = lane & 31;

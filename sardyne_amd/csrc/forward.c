@@ -134,13 +134,13 @@ void sdy_engine_release(engine_ctx *c) {
 }
 
 /* Every write of c->xq[] comes with this call: the quantisation cache forgets its sources, and the GEMM
- * workspace's f16 expansion of the activations (recorded with the epoch it was made in) goes stale. */
+ * workspace's expansion of the activations (recorded with the epoch it was made in) goes stale. */
 static void xq_forget(engine_ctx *c) {
     c->xq_src[0] = c->xq_src[1] = NULL;
     c->xq_epoch++;
 }
 
-/* gemm_ws now holds the f16 expansion of xq (n_tok rows of n_in), made after the last write of xq[] */
+/* gemm_ws now holds the expansion of xq (n_tok rows of n_in), made after the last write of xq[] */
 static void gemm_record(engine_ctx *c, const void *xq, int n_tok, int n_in) {
     c->gemm_ready = 1;
     c->gemm_epoch = c->xq_epoch;
@@ -173,7 +173,7 @@ static int mm_epi(engine_ctx *c, float *out, const float *x, const dmat *w, int 
     } else {
         int s = vt == SDY_Q8_0 ? 0 : 1;
         if (c->xq_src[s] != x || c->xq_n_tok[s] != n_tok || c->xq_n_in[s] != w->n_in) {
-            /* for the GEMM the quantiser also writes the f16 expansion it reads */
+            /* for the GEMM the quantiser also writes the expansion it reads */
             const int gemm = vt == SDY_Q8_K && use_gemm(w, n_tok);
             if (gemm) TRY(sdy_quantize_gemm(x, c->xq[s], w->n_in, n_tok, c->gemm_ws, c->st));
             else TRY(sdy_quantize(vt, x, c->xq[s], w->n_in, n_tok, c->st));
@@ -186,7 +186,7 @@ static int mm_epi(engine_ctx *c, float *out, const float *x, const dmat *w, int 
         a.xq = c->xq[s];
         /* many tokens of a K-quant matrix: the MFMA GEMM (same bits as the matvec) */
         if (use_gemm(w, n_tok)) {
-            /* q, k and v (gate and up) read one quantised input: its f16 expansion is made once */
+            /* q, k and v (gate and up) read one quantised input: its expansion is made once */
             a.ws_ready = c->gemm_ready && c->gemm_epoch == c->xq_epoch && c->gemm_xq == a.xq &&
                          c->gemm_n_tok == n_tok && c->gemm_n_in == w->n_in;
             c->gemm_ready = 0;
@@ -246,7 +246,7 @@ static int norm_for(engine_ctx *c, const float *x, const float *wn, const dmat *
     xq_forget(c);
     if (vt == SDY_F32) return sdy_norm_quant(x, wn, in->norm_eps, in->dim, n, c->xb, SDY_F32, NULL, c->st);
     const int s = vt == SDY_Q8_0 ? 0 : 1;
-    if (vt == SDY_Q8_K && use_gemm(next, n)) { /* with the GEMM's f16 expansion of the rows */
+    if (vt == SDY_Q8_K && use_gemm(next, n)) { /* with the GEMM's expansion of the rows */
         TRY(sdy_norm_quant_gemm(x, wn, in->norm_eps, in->dim, n, c->xb, c->xq[s], c->gemm_ws, c->st));
         gemm_record(c, c->xq[s], n, in->dim);
     } else {

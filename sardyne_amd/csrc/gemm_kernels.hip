@@ -1,26 +1,26 @@
-// Quantized-weight GEMM for prefill (many tokens) on gfx950 MFMA, bit-exact with the reference's
-// integer-dot path (csrc/quant.c:191-235, csrc/quant.h:84-91; the reference's 4-token micro-kernels
-// csrc/quant_avx2.c:290-385 give the same bits as its one-token dots).
+// Prompt GEMM of Q4_K / Q6_K weights on the int8 matrix cores, bit-exact with the reference's integer-dot path
+// (csrc/quant.c:191-235, csrc/quant.h:84-91; the reference's 4-token micro-kernels csrc/quant_avx2.c:290-385 give
+// the same bits as its one-token dots).
 //
-// Per 256-element super-block the reference computes an exact integer isum = sum_k (sc_g q_k) y_k
-// (and for Q4_K msum = sum_j m_j bsum_j), then combines acc + (yd*d*isum - yd*dmin*msum) in f32.
-// Here every wave dequantises its weight fragments in registers as f16 w' = sc * q (Q4_K) or
-// sc * (q - 32) (Q6_K) — exact small integers — and multiplies them with the Q8_K activations as
-// f16 (exact int8 values) on v_mfma_f32_32x32x16_f16, accumulating one super-block at a time in
-// f32. The products are exact and every partial sum stays below 2^24 when
-// 127 * sum_k |w'_k| < 2^24 and |w'| <= 2048 for each row and super-block, so the accumulator
-// holds isum exactly. Matrices with a block beyond that (real Q6_K files store int8 scales down to
-// -128) take the wide variant, exact for every block the formats can hold: Q6_K splits each scale,
-// sc = 16 sh + sl with 0 <= sl < 16, into two fragments with two accumulators, isum = 16 ihi + ilo;
-// Q4_K centres its quants, isum = sum sc (q - 8) y + sum_j 8 sc_j bsum_j. Each part's partial sums
-// stay below 2^24 and the two are added in f32 with one rounding, that of (float)isum. The check
-// runs once per matrix at upload. The Q4_K min term is one more MFMA of the mins against
-// the 16-element bsums. The f32 combine then follows the reference's expression and super-block
-// order, so each output has the reference's bits.
+// v_mfma_i32_32x32x32_i8 multiplies a 32-element Q4_K sub-block of 32 rows with 32 tokens (Q6_K, whose sub-blocks
+// have 16 elements: v_mfma_i32_32x32x16_i8). A lane holds one row of the 32 x 32 products, so a sub-block's scale
+// is the lane's own: one 24-bit multiply-add per product sums them over the super-block, exactly, for every block
+// the formats can hold. The Q4_K mins and the Q6_K quants' offset 32 are one f16 matrix instruction against the
+// activations' 16-element sums (exact integers below 2^24), the f32 scale products an f32 outer product (one
+// rounding, the VALU multiply's; a zero product may be +0 where the multiply gives -0, which no sum keeps), and
+// the combine is the reference's expression, super-blocks in order.
 //
-// The activations are expanded to f16 by k_gemm_prep, once per call unless the caller says the
-// workspace already holds them (ws_ready: q, k and v of one input).
+// What bounds it: the VALU. Per super-block and 32 x 32 outputs Q4_K takes 315 VALU instructions (128 multiply-adds,
+// 96 of the combine) and the f32 outer product's 64 cycles, Q6_K about 500; the matrix cores' 290 and 540 cycles run
+// beside them. The weights dequantised to f16 (sc * q, one fragment, two for the scales of real Q6_K files) summed
+// whole super-blocks on the matrix cores with fewer VALU instructions, but its registers and LDS left two waves
+// to a SIMD that waited for each other; here three or more keep the VALU busy. With the quantiser's launch, f16
+// form -> this: 22016 x 2048 Q4_K, 512 tokens 90.6 -> 82.0 us (565 TFLOP/s; VALU busy 65 %), 128 tokens 40.4 -> 29.0;
+// 2048 x 11008 Q6_K, 203 tokens 69.4 -> 46.7, 64 tokens 66.3 -> 31.6 (on mm_superblocks.hip); 151936 x 2048 Q6_K, 32
+// tokens 110 -> 79, 64 tokens 127 -> 125.
 #include <stdlib.h>
+
+#include <type_traits>
 
 #include "sdy_device.h"
 #include "sdy_internal.h"
@@ -29,260 +29,82 @@
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float16v __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 struct GemmArgs {
-    const uint8_t *p[5];  // weight planes (quant_kernels.hip layout)
-    uint32_t psz[5];      // their sizes in bytes (bounds of the buffer resources)
+    const uint8_t *p[5];  // planes (quant_kernels.hip), or the tiled copy's (blk, grow0)
     int n_in, T, nb;      // elements, 64-element units and super-blocks per row
-    long row0, n_rows;    // rows row0 .. row0 + n_rows of the planes
+    int blk;              // records [row / 32][record][row % 32]; row r is row grow0 + r there
+    long grow0;
+    long row0, n_rows;    // rows row0 .. row0 + n_rows
+    SdyGemmExp e;         // the activations' expansion
     int n_tok;
-    const _Float16 *y16;  // [n_tok][n_in] activations (the Q8_K int8 values)
-    const float *yd;      // [n_tok][nb] Q8_K scales
-    const _Float16 *bs16; // [n_tok][nb][16] Q8_K bsums
     float *out;
     long out_stride;
     const float *bias, *resid;
     int swiglu;
-    // grouped launch (k_gemm3 only; grp_tile null: one matrix): group e (a routed expert) multiplies
-    // weight rows row0 + e * grp_rows + [0, n_rows) with activation rows grp_tok[e] .. grp_tok[e + 1]
-    // - 1; its token tiles are grp_tile[e] .. grp_tile[e + 1] - 1 of the grid. out_row (or null)
-    // sends activation row t's outputs to output row out_row[t].
-    const int *grp_tile, *grp_tok, *out_row;
-    const int *act_row;  // or null: the activation (expansion) row of row t of the tile
+    // grouped (grp_tile set): group e (a routed expert) multiplies weight rows row0 + e * grp_rows + [0, n_rows) with
+    // rows grp_tok[e] .. grp_tok[e + 1] - 1 on token tiles grp_tile[e] .. grp_tile[e + 1] - 1 of the grid; row t reads
+    // expansion row act_row[t] and writes output row out_row[t] (either may be null: t)
+    const int *grp_tile, *grp_tok, *out_row, *act_row;
     long grp_rows;
     int n_grp;
-    int wide;  // host-side: the wide variant is needed (k_gemm3 only)
-    // k_gemm3: p holds the GEMM's copy of the planes (sdy_mat_gemm_layout: rows in tiles of 32,
-    // records unit- or super-block-major within a tile); row r of the matrix is row grow0 + r there
-    int blk;
-    long grow0;
-    int exp_rows;  // rows of the activations' expansion (y16, yd, bs16)
 };
 
-SDY_DEV u32x2 ld8(const uint8_t *p) { return *reinterpret_cast<const u32x2 *>(p); }
-
-// f16 pairs (1024 + b0, 1024 + b1) from byte lanes 0,1 (sel lo) or 2,3 (hi) of v: the magic
-// exponent 0x64 put above each byte by v_perm_b32.
-SDY_DEV uint32_t magic_lo(uint32_t v) { return __builtin_amdgcn_perm(0x64646464u, v, 0x05010400u); }
-SDY_DEV uint32_t magic_hi(uint32_t v) { return __builtin_amdgcn_perm(0x64646464u, v, 0x05030402u); }
-
-SDY_DEV half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-
-// 8 Q4_K quants q (one per byte of n.x, n.y) times sc as f16 with one fused multiply-add per
-// pair: (1024 + q) * sc - 1024 * sc. The exact result q * sc <= 945 is representable, so the single
-// rounding of the fma is exact (1024 * sc <= 64512 is exact too).
-SDY_DEV half8 frag_q4(u32x2 n, half2v sc2, half2v nsc2) {
-    half8 r;
-    const uint32_t w[4] = {magic_lo(n.x), magic_hi(n.x), magic_lo(n.y), magic_hi(n.y)};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const half2v t = __builtin_elementwise_fma(as_h2(w[i]), sc2, nsc2);
-        r[2 * i] = t[0];
-        r[2 * i + 1] = t[1];
-    }
-    return r;
+SDY_DEV __amdgpu_buffer_rsrc_t rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, -1, 0x00020000);
 }
-SDY_DEV uint32_t as_u(half2v v) { return __builtin_bit_cast(uint32_t, v); }
-
-// 8 small unsigned integers (one per byte of n.x, n.y) times sc as f16: ((1024 + q) - 1024) * sc,
-// every step exact (q <= 63, |q * sc| <= 2048).
-SDY_DEV half8 frag_scaled(u32x2 n, half2v off, half2v sc2) {
-    half8 r;
-    const uint32_t w[4] = {magic_lo(n.x), magic_hi(n.x), magic_lo(n.y), magic_hi(n.y)};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const half2v t = (as_h2(w[i]) + off) * sc2;
-        r[2 * i] = t[0];
-        r[2 * i + 1] = t[1];
-    }
-    return r;
+SDY_DEV long as_long(u32x2 v) { return __builtin_bit_cast(long, v); }
+SDY_DEV u32x2 bload8(__amdgpu_buffer_rsrc_t r, uint32_t v, int s) {
+    const auto x = __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0);
+    return u32x2{(uint32_t)x[0], (uint32_t)x[1]};
 }
 
-template <int WT>
-SDY_DEV void load_unit(const GemmArgs &g, long row, int u, int h, u32x2 (&q)[3]) {
-    const size_t ou = ((size_t)row * g.T + u) * 16 + 8 * h;
-    if constexpr (WT == SDY_Q4_K) {
-        q[0] = ld8(g.p[0] + ou);  // QA
-        q[1] = ld8(g.p[1] + ou);  // QB
-    } else {
-        q[0] = ld8(g.p[0] + ou);  // N0
-        q[1] = ld8(g.p[1] + ou);  // N1
-        q[2] = ld8(g.p[2] + ou);  // HB
-    }
-}
+template <int RW, int KS>
+constexpr size_t gemm_lds_bytes() { return 2 * (size_t)(32 * 292 * KS) + (KS > 1 ? RW * KS * 16 * 64 * 4 : 0); }
 
-// The weights of one super-block for one lane: its A row's quants for k-half h of the 4 units, the
-// scale record (Q4_K: d, dmin and the 12 packed scale/min bytes; Q6_K: the 16 int8 scales) and
-// the Q6_K d.
-struct SbRegs {
-    u32x2 q[4][3];
-    u32x4 hd;
-    uint32_t d6;
-};
-
-template <int WT>
-SDY_DEV void load_sb(const GemmArgs &g, long row, int sb, int h, SbRegs &r) {
-#pragma unroll
-    for (int un = 0; un < 4; un++) load_unit<WT>(g, row, 4 * sb + un, h, r.q[un]);
-    if constexpr (WT == SDY_Q4_K) {
-        r.hd = *reinterpret_cast<const u32x4 *>(g.p[2] + ((size_t)row * g.nb + sb) * 16);
-        r.d6 = 0;
-    } else {
-        r.hd = *reinterpret_cast<const u32x4 *>(g.p[3] + ((size_t)row * g.nb + sb) * 16);
-        r.d6 = *reinterpret_cast<const uint16_t *>(g.p[4] + ((size_t)row * g.nb + sb) * 2);
-    }
-}
-
-// k_gemm3's weights of one super-block for one lane: the quants of its units (all 16 bytes of each
-// plane's record: both k-halves), the scale record and the Q6_K d.
-struct SbRegs3 {
-    u32x4 q[2][3];
-    u32x4 hd;
-    uint32_t d6;
-};
-
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-SDY_DEV uint32_t lds_addr(const float *p) {
-    return (uint32_t)(size_t)(const __attribute__((address_space(3))) float *)p;
-}
-
-// Four 16-byte LDS reads at a, a + 32, a + 64, a + 96 and four at b, b + 32, ... as one asm block
-// that waits for them itself. The compiler then does not see LDS loads here: it would otherwise
-// make them wait for every activation DMA in flight (it cannot tell that they do not alias).
-SDY_DEV void lds_read8(uint32_t a, uint32_t b, f32x4 &a0, f32x4 &a1, f32x4 &a2, f32x4 &a3, f32x4 &b0, f32x4 &b1,
-                       f32x4 &b2, f32x4 &b3) {
-    __asm__ volatile(
-        "ds_read_b128 %0, %8\n"
-        "ds_read_b128 %1, %8 offset:32\n"
-        "ds_read_b128 %2, %8 offset:64\n"
-        "ds_read_b128 %3, %8 offset:96\n"
-        "ds_read_b128 %4, %9\n"
-        "ds_read_b128 %5, %9 offset:32\n"
-        "ds_read_b128 %6, %9 offset:64\n"
-        "ds_read_b128 %7, %9 offset:96\n"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(b0), "=&v"(b1), "=&v"(b2), "=&v"(b3)
-        : "v"(a), "v"(b)
-        : "memory");
-}
-
-// Two 16-byte LDS reads at a, a + 32 and two at b, b + 32, as lds_read8.
-SDY_DEV void lds_read4(uint32_t a, uint32_t b, f32x4 &a0, f32x4 &a1, f32x4 &b0, f32x4 &b1) {
-    __asm__ volatile(
-        "ds_read_b128 %0, %4\n"
-        "ds_read_b128 %1, %4 offset:32\n"
-        "ds_read_b128 %2, %5\n"
-        "ds_read_b128 %3, %5 offset:32\n"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(a0), "=&v"(a1), "=&v"(b0), "=&v"(b1)
-        : "v"(a), "v"(b)
-        : "memory");
-}
-
-// The s_waitcnt immediate that waits for at most n (< 64) vector memory operations outstanding and
-// lgkm (0 or 15: every LDS access, or none) LDS and scalar ones (vmcnt in bits 3:0 and 15:14,
-// expcnt at its maximum, lgkmcnt in bits 11:8).
-constexpr int sdy_vmcnt_imm(int n, int lgkm = 0) { return (n & 15) | (((n >> 4) & 3) << 14) | (7 << 4) | (lgkm << 8); }
-
-// SIZE bytes per lane from buffer r at vo + so into LDS at dst + SIZE * lane (the host pass of this
-// file does not know the builtin: it has no body there)
-template <int SIZE>
-SDY_DEV void buf_to_lds(__amdgpu_buffer_rsrc_t r, lds_ptr_t dst, uint32_t vo, int so) {
-    static_assert(SIZE == 4 || SIZE == 16, "dword or dwordx4");
-#if __HIP_DEVICE_COMPILE__
-    if constexpr (SIZE == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, vo, so, 0, 0);
-    else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 4, vo, so, 0, 0);
-#endif
-}
-
-SDY_DEV __amdgpu_buffer_rsrc_t plane_rsrc(const uint8_t *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)bytes, 0x00020000);
-}
-
-// The MFMA GEMM with the activations staged by LDS DMA. A workgroup of WM waves covers 32*MT*WM
-// rows x 32*NT tokens; each wave owns 32*MT rows (MT MFMA row tiles, dequantised in registers
-// from buffer loads whose per-super-block advance is a scalar offset) and shares the staged
-// activations of all the workgroup's tokens. The two lanes of a row split its units, each loading
-// whole 16-byte records (lane half h: units 2h, 2h+1), so that a load instruction reads 32 bytes
-// of each of its 32 rows (the vector L1 looks up a cache line per row and instruction); a step's
-// MFMA k-slots are then the lane halves' own units, and the activation fragments are read to
-// match (the integer sums do not depend on the k order). Per super-block and stage the activations are
-// copied global -> LDS with global_load_lds (no registers): LDS chunk p (16 bytes) holds token
-// p / 32, chunk (p % 32) ^ (token % 8), so that the fragment reads of 8 consecutive lanes hit
-// distinct banks. Two stages: super-block s + 1 is in flight while s is multiplied; one
-// s_waitcnt + barrier per super-block. The per-row d (and dmin) are converted once per row into a
-// per-wave LDS table.
-//
-// KS = 2 splits each super-block's four 64-element units between the two waves of a pair that own
-// the same rows (units 0-1 and 2-3): each wave sums its units' integer products, the pair exchanges
-// half of its accumulator through LDS at the super-block's barrier, and each wave completes and
-// combines its half of the tile (D registers 0-7 or 8-15). Integer partial sums add exactly, so the
-// bits are KS 1's; a grid has twice the waves (for shapes with one wave per SIMD otherwise: the
-// 2048-row down and attention projections of a prompt).
-//
-// PF = 2 keeps two super-blocks in flight (three register sets and three stage buffers): the wave
-// waits by count for the loads of the next super-block only, and the workgroup barrier orders LDS
-// alone. For grids of one wave per SIMD, whose super-blocks otherwise each wait a full memory round
-// trip.
-//
-// The body below takes the workgroup's place in its grid (bx, by of gx, gy: a pair launch gives
-// each matrix a part of one grid) and its LDS: the stages (dynamic), the per-wave d table and the
-// KS 2 exchange (static objects of the kernel, sized by gemm3_dtab_floats / gemm3_xch_floats).
-template <int MT, int WM>
-constexpr int gemm3_dtab_floats() { return WM * 64 * MT; }
-template <int WT, int MT, int NT, int WM, bool WIDE, int KS>
-constexpr int gemm3_xch_floats() { return KS == 2 ? 2 * WM * (WIDE && WT == SDY_Q6_K ? 2 : 1) * MT * NT * 8 * 64 : 1; }
-
-template <int WT, int MT, int NT, int WM, bool WIDE, int KS, int PF>
-SDY_DEV void gemm3_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_t *lds, float *dtab_all,
-                        float *xch) {
-    static_assert(KS == 1 || (KS == 2 && WM % 2 == 0), "unit split");
-    static_assert(PF == 1 || PF == 2, "prefetch depth");
-    constexpr int UN = 4 / KS, PAIRS = WM / KS;  // units per wave, row tiles per workgroup
-    constexpr int BN = 32 * NT, NTH = 64 * WM;
-    constexpr int YDN = BN < 64 ? 64 : BN;                  // yd slots (one DMA dword per lane)
-    // PF 2: every wave issues the same loads (so that its waits can be counted): each copies the yd
-    // row into a slot of its own and a 1/WM share of the bsums, as dwords
-    constexpr int YDOFF = BN * 512, BSOFF = YDOFF + (PF == 2 ? WM : 1) * YDN * 4;
-    constexpr int BUF = BSOFF + BN * 32;                    // bytes of one stage
-    constexpr int NBSW = BN * 8 / (64 * WM);                // PF 2: bsum dword loads per wave
-    static_assert(PF == 1 || (BN * 8) % (64 * WM) == 0, "PF 2: the bsums in whole dword loads per wave");
-    constexpr int NI = BN * 32 / NTH;                       // activation DMA chunks per lane per stage
-    static_assert((BN * 32) % NTH == 0 && NI >= 1, "tile");
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h = lane >> 5,
-              lr = lane & 31;
-    // token tiles of a row tile on one XCD (workgroups are dealt round-robin to the 8 XCDs)
-    const int n_tt = gx;
-    const long n_rt = gy, L = (long)by * n_tt + bx;
+// A workgroup of RW * KS waves computes 32 RW rows x 32 tokens; a wave owns a row tile and, with KS > 1, every KS-th
+// super-block: its f32 terms go through LDS to the tile's waves, each adding up a part of the outputs over the KS
+// super-blocks in order. The activations are shared through LDS in stages of KS super-blocks, requested a stage ahead
+// into registers, 16-byte chunk c of a token's 256 at slot c ^ (token % 16) (16 tokens' reads of one chunk then hit all
+// 64 banks once). The weights go straight to registers, each lane (row lr, k-half h) loading its own records, and
+// are reloaded for the next stage as they are used: from the tiled copy a load instruction reads runs of 512
+// bytes. The workgroup's place in the grid is (bx, by) of (gx, gy): a pair launch gives each matrix a part of one grid.
+template <int WT, int RW, int KS>
+SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_t *lds) {
+    constexpr bool Q4 = WT == SDY_Q4_K;
+    constexpr int BM = 32 * RW, BN = 32, NTH = 64 * RW * KS;
+    constexpr int NA = BN * 16 * KS / NTH;             // 16-byte chunks of activations per thread and stage
+    constexpr int NS = (BN * 2 * KS + NTH - 1) / NTH;  // of their 16-element sums
+    constexpr int NY = (BN * KS + NTH - 1) / NTH;      // and scales
+    static_assert(BN * 16 * KS % NTH == 0, "whole chunks per thread");
+    constexpr int OFF_B = BN * 256 * KS, OFF_Y = OFF_B + BN * 32 * KS, STAGE = OFF_Y + BN * 4 * KS;
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, lr = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave % KS, rw = wave / KS;
+    // token tiles of a row tile on one XCD (workgroups are dealt to the 8 XCDs in turn)
+    const long n_tt = gx, n_rt = gy, L = (long)by * n_tt + bx;
     long rti, tti;
-    {
-        const long grp = 8L * n_tt, full = n_rt / 8 * grp;
-        if (L < full) {
-            const long gq = L / grp, w = L - gq * grp;
-            rti = gq * 8 + (w & 7);
-            tti = w >> 3;
-        } else {
-            const long w = L - full;
-            rti = n_rt / 8 * 8 + w / n_tt;
-            tti = w - (w / n_tt) * n_tt;
-        }
+    if (L < n_rt / 8 * 8 * n_tt) {
+        const long gq = L / (8 * n_tt), w = L - gq * 8 * n_tt;
+        rti = gq * 8 + (w & 7);
+        tti = w >> 3;
+    } else {
+        const long w = L - n_rt / 8 * 8 * n_tt;
+        rti = n_rt / 8 * 8 + w / n_tt;
+        tti = w % n_tt;
     }
-    const int pw = __builtin_amdgcn_readfirstlane(wave / KS);  // the wave's row tile
-    const int ks = __builtin_amdgcn_readfirstlane(wave - pw * KS);  // and unit share
-    const long rt = rti * (32 * MT * PAIRS) + 32 * MT * pw;
     int t0 = (int)tti * BN, t_end = g.n_tok;
     long row0 = g.row0;
     if (g.grp_tile) {
-        // the group of this token tile: the last e with grp_tile[e] <= tti (empty groups share
-        // their successor's start, so the last one is the group that owns the tile)
+        // the group of this token tile: the last e with grp_tile[e] <= tti (empty groups share their successor's
+        // start, so the last one is the group that owns the tile)
         if (tti >= g.grp_tile[g.n_grp]) return;  // past the routed tokens (uniform over the workgroup)
         int lo = 0, hi = g.n_grp - 1;
         while (lo < hi) {
@@ -294,639 +116,261 @@ SDY_DEV void gemm3_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8
         t_end = g.grp_tok[lo + 1];
         row0 += (long)lo * g.grp_rows;
     }
-    const int nb = g.nb;
-    auto tok_of = [&](int t) { return t0 + t < t_end ? t0 + t : t_end - 1; };
-    // the expansion rows the stages read: this lane's rows of the tile, looked up once
-    auto act_of = [&](int t) { return g.act_row ? g.act_row[tok_of(t)] : tok_of(t); };
-    int ar_st[NI], ar_yd[YDN / 64], ar_bs[BN / 32 > 0 ? BN / 32 : 1], ar_b2[PF == 2 && NBSW > 0 ? NBSW : 1];
-#pragma unroll
-    for (int j = 0; j < NI; j++) ar_st[j] = act_of(((j * WM + wave) * 64 + lane) >> 5);
-#pragma unroll
-    for (int i = 0; i < YDN / 64; i++) ar_yd[i] = act_of(64 * i + lane);
-#pragma unroll
-    for (int i = 0; i < BN / 32; i++) ar_bs[i] = act_of(32 * i + (lane >> 1));
-    if constexpr (PF == 2 && WT == SDY_Q4_K) {
-#pragma unroll
-        for (int i = 0; i < NBSW; i++) ar_b2[i] = act_of(((i * WM + wave) * 64 + lane) >> 3);
-    }
-    // the stage's loads as buffer loads to LDS: the lanes' byte offsets are fixed, the super-block
-    // advance is a scalar offset (no per-super-block address arithmetic)
-    const __amdgpu_buffer_rsrc_t ry = plane_rsrc(reinterpret_cast<const uint8_t *>(g.y16), (uint32_t)g.exp_rows * g.n_in * 2u),
-                                 ryd = plane_rsrc(reinterpret_cast<const uint8_t *>(g.yd), (uint32_t)g.exp_rows * nb * 4u),
-                                 rbs = plane_rsrc(reinterpret_cast<const uint8_t *>(g.bs16), (uint32_t)g.exp_rows * nb * 32u);
-    uint32_t vst[NI], vyd[YDN / 64], vbs[BN / 32 > 0 ? BN / 32 : 1], vb2[PF == 2 && NBSW > 0 ? NBSW : 1];
-#pragma unroll
-    for (int j = 0; j < NI; j++) {
-        const int p = (j * WM + wave) * 64 + lane, t = p >> 5, c = (p & 31) ^ (t & 7);
-        vst[j] = ((uint32_t)ar_st[j] * (uint32_t)g.n_in + 8u * (uint32_t)c) * 2u;
-    }
-#pragma unroll
-    for (int i = 0; i < YDN / 64; i++) vyd[i] = (uint32_t)ar_yd[i] * (uint32_t)nb * 4u;
-#pragma unroll
-    for (int i = 0; i < BN / 32; i++) vbs[i] = (uint32_t)ar_bs[i] * (uint32_t)nb * 32u + 16u * (uint32_t)(lane & 1);
-    if constexpr (PF == 2 && WT == SDY_Q4_K) {
-#pragma unroll
-        for (int i = 0; i < NBSW; i++) vb2[i] = (uint32_t)ar_b2[i] * (uint32_t)nb * 32u + 4u * (uint32_t)(lane & 7);
-    }
+    const int nb = g.nb, T = g.T, ns = (nb + KS - 1) / KS;
 
-    // weight buffer resources and this lane's per-row offsets
-    __amdgpu_buffer_rsrc_t rq[3], rh, rd;
-#pragma unroll
-    for (int i = 0; i < 3; i++) rq[i] = plane_rsrc(g.p[i], g.psz[i]);
-    rh = plane_rsrc(g.p[WT == SDY_Q4_K ? 2 : 3], g.psz[WT == SDY_Q4_K ? 2 : 3]);
-    rd = plane_rsrc(g.p[4], g.psz[4]);
-    // the lane's units of each super-block: ub + uu, uu < UN / 2
-    constexpr int UL = UN / 2;
-    const int ub = ks * UN + h * UL;
-    // the lane's LDS byte offsets in a stage of its activation fragments' chunks k = 2 s + hh of unit ub
-    uint32_t rbo[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) rbo[k] = 16u * (uint32_t)(lr * 32 + 8 * ub + (k ^ (lr & 7)));
-    // per-lane offsets of the row's records, and the scalar strides of a unit and a super-block:
-    // planes row-major, or the GEMM copy (tiles of 32 rows, the tile's 32 records of one unit or
-    // super-block adjacent: a load instruction reads 512 contiguous bytes per half-wave)
-    uint32_t oq[MT], oh[MT], od[MT];
-    const uint32_t ust = g.blk ? 512u : 16u, hst = g.blk ? 512u : 16u, dst2 = g.blk ? 64u : 2u;
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const long ri = rt + 32 * mt + lr;
-        const uint32_t row = (uint32_t)(row0 + (ri < g.n_rows ? ri : g.n_rows - 1));
-        if (g.blk) {
-            const uint32_t R = (uint32_t)g.grow0 + row, tb = R >> 5, r = R & 31u;
-            oq[mt] = (tb * (uint32_t)g.T * 32u + r) * 16u + 512u * (uint32_t)(h * UL);
-            oh[mt] = (tb * (uint32_t)nb * 32u + r) * 16u;
-            od[mt] = (tb * (uint32_t)nb * 32u + r) * 2u;
+    // Weights: buffers from the first record of the wave's rows (of its first tile of 32 in the copy), the lane's
+    // offsets from there, and a unit's (super-block's) scalar one.
+    const long rt = rti * BM + 32 * rw, ri = rt + lr;
+    const long rfirst = row0 + (rt < g.n_rows ? rt : g.n_rows - 1), rc = row0 + (ri < g.n_rows ? ri : g.n_rows - 1);
+    const long t32 = (g.grow0 + rfirst) >> 5;
+    const size_t ub = g.blk ? (size_t)t32 * T * 32 : (size_t)rfirst * T, sb0 = g.blk ? (size_t)t32 * nb * 32 : (size_t)rfirst * nb;
+    const uint32_t dt = (uint32_t)(((g.grow0 + rc) >> 5) - t32), r32 = (uint32_t)(g.grow0 + rc) & 31u, dr = (uint32_t)(rc - rfirst);
+    const uint32_t vu = (g.blk ? dt * (uint32_t)T * 32u + r32 : dr * (uint32_t)T) * 16u;
+    const uint32_t vs = g.blk ? dt * (uint32_t)nb * 32u + r32 : dr * (uint32_t)nb;
+    const int us = g.blk ? 512 : 16, ss = g.blk ? 32 : 1;
+    const __amdgpu_buffer_rsrc_t r0 = rsrc(g.p[0] + ub * 16), r1 = rsrc(g.p[1] + ub * 16),
+                                 r2 = rsrc(g.p[2] + (Q4 ? sb0 : ub) * 16), r3 = rsrc(g.p[3] + sb0 * 16), r4 = rsrc(g.p[4] + sb0 * 2);
+    // (Q4_K: lane half h reads plane h; Q6_K: bytes 8 h .. of each plane's record)
+    const uint32_t vq = vu + (Q4 ? (h ? (uint32_t)(g.p[1] - g.p[0]) : 0u) : 8u * (uint32_t)h);
+    u32x4 w4[Q4 ? 4 : 1], sc;
+    u32x2 w6[Q4 ? 1 : 4][3];
+    uint32_t d6 = 0;
+    auto sb_of = [&](int s) { return s * KS + ks < nb ? s * KS + ks : nb - 1; };  // (past the end: not added)
+    auto load_u = [&](int s, int u) {
+        const int so = (4 * sb_of(s) + u) * us;
+        if constexpr (Q4) {
+            w4[u] = __builtin_amdgcn_raw_buffer_load_b128(r0, vq, so, 0);
         } else {
-            oq[mt] = row * (uint32_t)g.T * 16u + 16u * (uint32_t)(h * UL);
-            oh[mt] = row * (uint32_t)nb * 16u;
-            od[mt] = row * (uint32_t)nb * 2u;
-        }
-    }
-    auto load_sb3 = [&](int sb, SbRegs3 (&R)[MT]) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-            for (int uu = 0; uu < UL; uu++) {  // units ub + uu (h UL in the lane's offset)
-                const int so = (4 * sb + ks * UN + uu) * (int)ust;
-                R[mt].q[uu][0] = __builtin_amdgcn_raw_buffer_load_b128(rq[0], oq[mt], so, 0);
-                R[mt].q[uu][1] = __builtin_amdgcn_raw_buffer_load_b128(rq[1], oq[mt], so, 0);
-                if constexpr (WT == SDY_Q6_K) R[mt].q[uu][2] = __builtin_amdgcn_raw_buffer_load_b128(rq[2], oq[mt], so, 0);
-            }
-            R[mt].hd = __builtin_amdgcn_raw_buffer_load_b128(rh, oh[mt], sb * (int)hst, 0);
-            R[mt].d6 = WT == SDY_Q6_K ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rd, od[mt], sb * (int)dst2, 0) : 0u;
+            w6[u][0] = bload8(r0, vq, so);
+            w6[u][1] = bload8(r1, vq, so);
+            w6[u][2] = bload8(r2, vq, so);
         }
     };
-    // activation stage of super-block sb into buffer buf (asynchronous; completes at s_waitcnt)
-    auto stage = [&](int sb, int buf) {
-        uint8_t *base = lds + buf * BUF;
-#pragma unroll
-        for (int j = 0; j < NI; j++) {
-            const int blk = j * WM + wave;  // 64-chunk block written by this wave instruction
-            buf_to_lds<16>(ry, (lds_ptr_t)(base + blk * 1024), vst[j], sb * 512);
-        }
-        if constexpr (PF == 2) {
-#pragma unroll
-            for (int i = 0; i < YDN / 64; i++)
-                buf_to_lds<4>(ryd, (lds_ptr_t)(base + YDOFF + wave * (YDN * 4) + 256 * i), vyd[i], sb * 4);
-            if constexpr (WT == SDY_Q4_K) {
-#pragma unroll
-                for (int i = 0; i < NBSW; i++)  // bsum dword p = (i WM + wave) 64 + lane: token p / 8, bytes 4 (p % 8)
-                    buf_to_lds<4>(rbs, (lds_ptr_t)(base + BSOFF + 256 * (i * WM + wave)), vb2[i], sb * 32);
-            }
-        } else {
-            if (wave == 0) {
-#pragma unroll
-                for (int i = 0; i < YDN / 64; i++)
-                    buf_to_lds<4>(ryd, (lds_ptr_t)(base + YDOFF + 256 * i), vyd[i], sb * 4);
-            }
-        }
-        if constexpr (WT == SDY_Q4_K && PF == 1) {
-            if (wave == (WM > 1 ? 1 : 0)) {
-#pragma unroll
-                for (int i = 0; i < BN / 32; i++)
-                    buf_to_lds<16>(rbs, (lds_ptr_t)(base + BSOFF + 1024 * i), vbs[i], sb * 32);
-            }
-        }
+    auto load_s = [&](int s) {
+        sc = __builtin_amdgcn_raw_buffer_load_b128(Q4 ? r2 : r3, vs * 16u, sb_of(s) * ss * 16, 0);
+        if constexpr (!Q4) d6 = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r4, vs * 2u, sb_of(s) * ss * 2, 0);
     };
-    // PF 1: the barrier's release fence waits for every load of the wave, the DMA of the stage included.
-    // PF 2: the loads of the iteration's super-block sb + 2 stay in flight: wait until at most as
-    // many as the wave issued for it are outstanding (loads complete in order), then a barrier that
-    // orders the LDS accesses (the activations DMA'd by every wave, the exchange)
-    constexpr int NWL = MT * (UL * (WT == SDY_Q6_K ? 3 : 2) + (WT == SDY_Q6_K ? 2 : 1));  // load_sb3's loads
-    constexpr int NSL = NI + YDN / 64 + (WT == SDY_Q4_K ? NBSW : 0);                     // PF 2: stage()'s
-    static_assert(PF == 1 || NWL + NSL < 64, "wait count");
-    auto wait_stage = [&]() {
-        if constexpr (PF == 1) {
-            __syncthreads();
-        } else {
-            // s_waitcnt vmcnt(NWL + NSL) lgkmcnt(0) (the compiler's own wait tracking sees it), then the
-            // barrier as a compiler memory barrier too (a fence would wait for the DMA in flight: it
-            // writes LDS)
-            __builtin_amdgcn_s_waitcnt(sdy_vmcnt_imm(NWL + NSL));
-            __asm__ volatile("s_barrier" ::: "memory");
+    // Activations: this thread's chunks of a stage, of fixed tokens, super-block of the stage and place in it.
+    const __amdgpu_buffer_rsrc_t ry = rsrc(g.e.y8), rb = rsrc(g.e.bs16), rd = rsrc(g.e.yd);
+    auto act_of = [&](int t) {
+        const int r = t0 + t < t_end ? t0 + t : t_end - 1;
+        return (uint32_t)(g.act_row ? g.act_row[r] : r);
+    };
+    const int ac = tid % 16, ak = tid / 16 % KS, at0 = tid / (16 * KS), bk = tid / 2 % KS, yk = tid % KS;
+    constexpr int AS = NTH / (16 * KS);  // tokens between a thread's chunks
+    // (fewer sums and scales than threads: the threads past them repeat one, with the same values)
+    auto bt = [&](int i) { return (tid + NTH * i) / (2 * KS) % BN; };
+    auto yt = [&](int i) { return (tid + NTH * i) / KS % BN; };
+    uint32_t ao[NA], bo[NS], yo[NY];
+#pragma unroll
+    for (int i = 0; i < NA; i++) ao[i] = act_of(at0 + AS * i) * (uint32_t)g.n_in + 16u * (uint32_t)ac;
+#pragma unroll
+    for (int i = 0; i < NS; i++) bo[i] = act_of(bt(i)) * (uint32_t)nb * 32u + 16u * (uint32_t)(tid & 1);
+#pragma unroll
+    for (int i = 0; i < NY; i++) yo[i] = act_of(yt(i)) * (uint32_t)nb * 4u;
+    u32x4 av[NA], bv[NS];
+    uint32_t yv[NY];
+    auto load_a = [&](int s) {
+        auto blk = [&](int k) { return s * KS + k < nb ? s * KS + k : nb - 1; };
+#pragma unroll
+        for (int i = 0; i < NA; i++) av[i] = __builtin_amdgcn_raw_buffer_load_b128(ry, ao[i] + 256u * (uint32_t)blk(ak), 0, 0);
+#pragma unroll
+        for (int i = 0; i < NS; i++) bv[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, bo[i] + 32u * (uint32_t)blk(bk), 0, 0);
+#pragma unroll
+        for (int i = 0; i < NY; i++) yv[i] = __builtin_amdgcn_raw_buffer_load_b32(rd, yo[i] + 4u * (uint32_t)blk(yk), 0, 0);
+    };
+    auto store_a = [&](uint8_t *buf) {
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            const int t = at0 + AS * i;
+            *reinterpret_cast<u32x4 *>(buf + (ak * BN + t) * 256 + 16 * (ac ^ (t & 15))) = av[i];
         }
+#pragma unroll
+        for (int i = 0; i < NS; i++) *reinterpret_cast<u32x4 *>(buf + OFF_B + (bk * BN + bt(i)) * 32 + 16 * (tid & 1)) = bv[i];
+#pragma unroll
+        for (int i = 0; i < NY; i++) *reinterpret_cast<uint32_t *>(buf + OFF_Y + (yk * BN + yt(i)) * 4) = yv[i];
     };
 
-    constexpr int RH = 16 / KS;  // D registers (of 16) that a wave completes: RH ks .. RH ks + RH - 1
-    float acc[MT][NT][RH];
+    constexpr int NF = 16 / KS;  // the outputs a wave adds up: registers NF ks .. of the tile's 16
+    float acc[NF];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
+    for (int i = 0; i < NF; i++) acc[i] = 0.0f;
+    float *xch = reinterpret_cast<float *>(lds + 2 * STAGE);
+    // isum += scale(j) * products j = 0 .. n - 1, each issued a step ahead of its use
+    auto sums = [&](auto issue, auto scale, auto n, i32x16 &isum) {
+        i32x16 p[2];
+        issue(0, p[0]);
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
+        for (int j = 0; j < n(); j++) {
+            if (j + 1 < n()) issue(j + 1, p[(j + 1) & 1]);
+            const int f = scale(j);
 #pragma unroll
-            for (int i = 0; i < RH; i++) acc[mt][nt][i] = 0.0f;
-    const half2v off6 = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-    const half2v off4c = {(_Float16)-1032.0f, (_Float16)-1032.0f};  // centred Q4_K quants q - 8
-    // per-wave d[32 MT] then dmin[32 MT] as f32 (static LDS: a separate object from the DMA target,
-    // so its reads need not wait for the activation loads in flight)
-    float *dtab = dtab_all + wave * (64 * MT);
-    // KS 2: the half accumulators a wave hands its partner (xch), [parity][wave][sum][mt][nt][8][64]
-    constexpr int NXS = WIDE && WT == SDY_Q6_K ? 2 : 1;
-
-    constexpr int NBUF = PF + 1;  // stage buffers
-    // one super-block: sb's weights in A, the loads of sb + PF issued into An (clamped to the last
-    // super-block, so that every iteration issues the same weight loads)
-    auto iter = [&](int sb, SbRegs3(&A)[MT], SbRegs3(&An)[MT]) {
-        const int cur = sb & 1;
-        // issue priorities over a super-block (the SIMD's other wave is at another point of its own):
-        // the next super-block's weight loads and activation DMA first (2), then the fragment reads
-        // and MFMA loop (1), the combine (VALU only) last (0). 3B prefill +1.4 % and +4.6 % on two
-        // boxes for the MFMA loop's 1, +0.7 % more for the loads' 2; the priority around the MFMA
-        // instructions alone changed nothing
-        __builtin_amdgcn_s_setprio(2);
-        load_sb3(sb + PF < nb ? sb + PF : nb - 1, An);
-        // PF 2 stages the last super-block again past the end (into the buffer of sb - 1, which is
-        // read no more), so that every iteration issues the same loads
-        if constexpr (PF == 2) {
-            stage(sb + PF < nb ? sb + PF : nb - 1, (sb + PF) % NBUF);
-            // already true (the previous iteration waited for sb's loads): stated so that the
-            // compiler's wait tracking, which loses count at the loop head, knows A complete
-            __builtin_amdgcn_s_waitcnt(sdy_vmcnt_imm(2 * (NWL + NSL), 15));
-        } else if (sb + PF < nb) {
-            stage(sb + PF, (sb + PF) % NBUF);
+            for (int i = 0; i < 16; i++) isum[i] += __mul24(f, p[j & 1][i]);  // |p| <= 32 * 15 * 128 or 16 * 63 * 128
+            // hide where the sums come from: the compiler then keeps one multiply-add per product (it would add
+            // the products of two sub-blocks at once, in three instructions and with both products' registers)
+            __asm__ volatile("" : "+v"(isum));
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_s_setprio(1);
-        // d (and dmin) of the lane's row (lr, the same in both lane halves) as f32
-        float drow[MT], mrow[MT];
+    };
+    // the wave's super-block of stage s, and its weights' reload for the next stage
+    auto compute = [&](int s, const uint8_t *buf) {
+        const uint8_t *ab = buf + (ks * BN + lr) * 256;
+        i32x16 isum = {};
+        f16x8 gw;  // the mins (Q4_K) or scales (Q6_K) of the lane's 16-element groups 8 h .. 8 h + 7
+        float dl;  // d, and for Q4_K dmin in lane half 1
+        if constexpr (Q4) {
+            // 6-bit scales and mins of the 8 sub-blocks as bytes (csrc/quant.h:72-80)
+            const uint32_t A = sc.y, B = sc.z, C = sc.w;
+            const uint32_t sw[2] = {A & 0x3F3F3F3Fu, (C & 0x0F0F0F0Fu) | ((A >> 2) & 0x30303030u)};
+            const uint32_t mw = h ? ((C >> 4) & 0x0F0F0F0Fu) | ((B >> 2) & 0x30303030u) : B & 0x3F3F3F3Fu;
+            dl = sdy_h2f((uint16_t)(h ? sc.x >> 16 : sc.x & 0xFFFFu));
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const uint32_t dp = WT == SDY_Q4_K ? A[mt].hd.x : A[mt].d6;
-            drow[mt] = sdy_h2f((uint16_t)(dp & 0xFFFFu));
-            mrow[mt] = WT == SDY_Q4_K ? sdy_h2f((uint16_t)(dp >> 16)) : 0.0f;
+            for (int e = 0; e < 8; e++) gw[e] = (_Float16)(float)((mw >> (8 * (e >> 1))) & 255u);
+            load_s(s + 1);
+            auto issue = [&](int j, i32x16 &p) {  // sub-block j: the low or high nibbles of unit j / 2, 16 to a lane half
+                const u32x4 w = w4[j >> 1];
+                const i32x4 wf = __builtin_bit_cast(i32x4, ((j & 1) ? w >> 4u : w) & 0x0F0F0F0Fu);
+                if (j & 1) load_u(s + 1, j >> 1);
+                const i32x4 a = *reinterpret_cast<const i32x4 *>(ab + 16 * ((2 * j + h) ^ (lr & 15)));
+                p = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, wf, i32x16{}, 0, 0, 0);
+            };
+            sums(issue, [&](int j) { return (int)((sw[j >> 2] >> (8 * (j & 3))) & 255u); }, std::integral_constant<int, 8>{}, isum);
+        } else {
+            const u32x4 scv = sc;
+            dl = sdy_h2f((uint16_t)d6);
+            const uint32_t g0 = h ? scv.z : scv.x, g1 = h ? scv.w : scv.y;
+#pragma unroll
+            for (int e = 0; e < 8; e++) gw[e] = (_Float16)(float)(int8_t)(((e < 4 ? g0 : g1) >> (8 * (e & 3))) & 255u);
+            load_s(s + 1);
+            auto issue = [&](int j, i32x16 &p) {  // sub-block j = 4 u + k: elements 16 k .. of unit u, stored 32 too high
+                const int u = j >> 2, k = j & 3;
+                const u32x2 nn = w6[u][k & 1], hb = w6[u][2];
+                const u32x2 lo = (k & 2) ? (nn >> 4u) & 0x0F0F0F0Fu : nn & 0x0F0F0F0Fu;
+                const u32x2 hi = k == 0 ? (hb & 0x03030303u) << 4u : k == 1 ? (hb & 0x0C0C0C0Cu) << 2u
+                                 : k == 2 ? hb & 0x30303030u : (hb >> 2u) & 0x30303030u;
+                if (k == 3) load_u(s + 1, u);
+                const long a = *reinterpret_cast<const long *>(ab + 16 * (j ^ (lr & 15)) + 8 * h);
+                p = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, as_long(lo | hi), i32x16{}, 0, 0, 0);
+            };
+            sums(issue, [&](int j) { return (int)(int8_t)((scv[j >> 2] >> (8 * (j & 3))) & 255u); }, std::integral_constant<int, 16>{}, isum);
         }
-        // KS 1: the combine's scale products from the matrix cores (outer products, below); KS 2 keeps
-        // them on the VALU from a per-wave LDS table (the MFMA form's registers cost the unit split's
-        // grids an occupancy step)
-        constexpr bool OUTER = KS == 1;
-        if constexpr (!OUTER) {
-            if (h == 0) {
+        const float yd = *reinterpret_cast<const float *>(buf + OFF_Y + (ks * BN + lr) * 4);
+        const f16x8 bs = *reinterpret_cast<const f16x8 *>(buf + OFF_B + (ks * BN + lr) * 32 + 16 * h);
+        const f32x16 off = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, gw, f32x16{}, 0, 0, 0);
+        // yd d in registers 0 .. 15 and (Q4_K) yd dmin in 16 .. 31: block b takes its factors from lane half b
+        const f32x32 sd = __builtin_amdgcn_mfma_f32_32x32x1f32(yd, dl, f32x32{}, 0, 0, 0);
+        float *xw = xch + (size_t)wave * (16 * 64) + lane;
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    dtab[32 * mt + lr] = drow[mt];
-                    if constexpr (WT == SDY_Q4_K) dtab[32 * MT + 32 * mt + lr] = mrow[mt];
-                }
-            }
-        }
-        const uint8_t *bbuf = lds + (sb % NBUF) * BUF;
-        // WIDE (any block the formats can hold):
-        //   Q6_K: each scale sc = 16 sh + sl (sl in [0, 16), sh in [-8, 7]) is applied in two exact
-        //         fragments with their own integer sums, isum = 16 ihi + ilo; the partial sums stay
-        //         below 2^24 (127 * 256 * 32 * 15 and 127 * 256 * 32 * 8);
-        //   Q4_K: the quants are centred, isum = sum sc (q - 8) y + sum_j 8 sc_j bsum_j: the first sum
-        //         below 127 * 256 * 63 * 8 < 2^24, the second one more MFMA against the bsums.
-        constexpr bool SPLIT6 = WIDE && WT == SDY_Q6_K;
-        float16v isum[MT][NT], ihi[SPLIT6 ? MT : 1][SPLIT6 ? NT : 1];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) isum[mt][nt] = float16v{};
-        if constexpr (SPLIT6) {
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) ihi[mt][nt] = float16v{};
-        }
-        // the lane's scales for its units, once per super-block. Q4_K: the 6-bit scales of sub-blocks
-        // 2 ub .. 2 ub + 2 UL - 1 as bytes (sub-blocks 0-3 from the low bits of the first word, 4-7
-        // from the third word and the top bits of the first); Q6_K: the int8 scale words of units ub + uu
-        uint32_t scw[MT][UL];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            if constexpr (WT == SDY_Q4_K) {
-                const uint32_t Aw = A[mt].hd.y, Cw = A[mt].hd.w;
-                const uint32_t f1 = Aw & 0x3F3F3F3Fu, f2 = (Cw & 0x0F0F0F0Fu) | ((Aw >> 2) & 0x30303030u);
-                scw[mt][0] = (ub >= 2 ? f2 : f1) >> (16 * (ub & 1));
+        for (int i = 0; i < 16; i++) {
+            float term;
+            if constexpr (Q4) {
+                const float t1 = sd[i] * (float)isum[i], t2 = sd[16 + i] * off[i];
+                term = t1 - t2;
             } else {
-#pragma unroll
-                for (int uu = 0; uu < UL; uu++) {
-                    const int w = ub + uu;
-                    const uint32_t lo = (w & 1) ? A[mt].hd.y : A[mt].hd.x, hi2 = (w & 1) ? A[mt].hd.w : A[mt].hd.z;
-                    scw[mt][uu] = (w & 2) ? hi2 : lo;
-                }
+                term = sd[i] * (float)(isum[i] - 32 * (int)off[i]);
             }
-        }
-        // step sl = 8 uu + 4 hh + s of the lane: k-half hh of unit ub + uu, quarter s (its 16-element
-        // chunk 8 (ub + uu) + 2 s + hh of each token), read from LDS one step ahead of its MFMAs
-        half8 bf[2][NT];
-        // chunk 8 (ub + uu) + k of token 32 nt + lr sits at bbuf + rbo[k] + 128 uu + 16384 nt (the swizzle
-        // only permutes the low three bits of the chunk index: k ^ (lr & 7))
-        const uint8_t *rbp[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) rbp[k] = bbuf + rbo[k];
-        auto read_b = [&](int sl, half8 (&dst)[NT]) {
-            const int k = 2 * (sl & 3) + ((sl >> 2) & 1), uu = sl >> 3;
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) dst[nt] = *reinterpret_cast<const half8 *>(rbp[k] + 128 * uu + 16384 * nt);
-        };
-        read_b(0, bf[0]);
-#pragma unroll
-        for (int uu = 0; uu < UL; uu++) {
-#pragma unroll
-            for (int hh = 0; hh < 2; hh++)
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const int sl = 8 * uu + 4 * hh + s;  // the lane's step
-                if (sl + 1 < 4 * UN) read_b(sl + 1, bf[(sl + 1) & 1]);
-                __builtin_amdgcn_sched_barrier(0);  // the next step's reads go out before this step's work
-                half8 a[MT], ah[SPLIT6 ? MT : 1];
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    auto half_of = [&](const u32x4 &v) { return hh ? u32x2{v.z, v.w} : u32x2{v.x, v.y}; };
-                    if constexpr (WT == SDY_Q4_K) {
-                        // sub-block 2 (ub + uu) + s / 2
-                        const int sc = (int)((scw[mt][0] >> (8 * (2 * uu + (s >> 1)))) & 255u);
-                        const u32x2 src = half_of((s & 1) ? A[mt].q[uu][1] : A[mt].q[uu][0]);
-                        const u32x2 nib = (s & 2) ? ((src >> 4u) & 0x0F0F0F0Fu) : (src & 0x0F0F0F0Fu);
-                        if constexpr (WIDE) {
-                            const _Float16 f = (_Float16)(float)sc;
-                            a[mt] = frag_scaled(nib, off4c, half2v{f, f});
-                        } else {
-                            const _Float16 f = (_Float16)(float)sc, nf = (_Float16)(float)(-1024 * sc);
-                            a[mt] = frag_q4(nib, half2v{f, f}, half2v{nf, nf});
-                        }
-                    } else {
-                        const int sc = (int)(int8_t)((scw[mt][uu] >> (8 * s)) & 255u);
-                        const u32x2 src = half_of((s & 1) ? A[mt].q[uu][1] : A[mt].q[uu][0]);
-                        const u32x2 lo = (s & 2) ? ((src >> 4u) & 0x0F0F0F0Fu) : (src & 0x0F0F0F0Fu);
-                        const u32x2 hi = ((half_of(A[mt].q[uu][2]) >> (unsigned)(2 * s)) & 0x03030303u) << 4u;
-                        if constexpr (SPLIT6) {
-                            const int sl6 = sc & 15, sh = sc >> 4;
-                            const _Float16 fl = (_Float16)(float)sl6, fh = (_Float16)(float)sh;
-                            a[mt] = frag_scaled(lo | hi, off6, half2v{fl, fl});
-                            ah[mt] = frag_scaled(lo | hi, off6, half2v{fh, fh});
-                        } else {
-                            const _Float16 f = (_Float16)(float)sc;
-                            a[mt] = frag_scaled(lo | hi, off6, half2v{f, f});
-                        }
-                    }
-                }
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-#pragma unroll
-                    for (int mt = 0; mt < MT; mt++) {
-                        isum[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt], bf[sl & 1][nt], isum[mt][nt], 0, 0, 0);
-                        if constexpr (SPLIT6)
-                            ihi[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[mt], bf[sl & 1][nt], ihi[mt][nt], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        __builtin_amdgcn_s_setprio(0);
-        // combine in the reference's order: acc + (yd*d*isum - yd*dmin*msum)
-        float ydn[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-            ydn[nt] = *reinterpret_cast<const float *>(bbuf + YDOFF + (PF == 2 ? wave * (YDN * 4) : 0) + 4 * (32 * nt + lr));
-        // Q4_K, row tile mt: msum = sum_j m_j bsum_j and, WIDE, cw = sum_j 8 sc_j bsum_j (below 16 * 504 *
-        // 2032 < 2^24), both exact, from the staged bsums
-        auto bsum_mfma = [&](int mt, float16v(&msum)[NT], float16v(&cw)[NT]) {
-            const uint32_t Aw = A[mt].hd.y, Bw = A[mt].hd.z, Cw = A[mt].hd.w;
-            half8 a2, a3;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int j = 4 * h + (e >> 1);  // sub-block of 16-group 8h + e
-                const int m = j < 4 ? (int)((Bw >> (8 * j)) & 63)
-                                    : (int)(((Cw >> (8 * (j - 4) + 4)) & 15) | (((Bw >> (8 * (j - 4) + 6)) & 3) << 4));
-                a2[e] = (_Float16)(float)m;
-                if constexpr (WIDE) {
-                    const int sc = j < 4 ? (int)((Aw >> (8 * j)) & 63)
-                                         : (int)(((Cw >> (8 * (j - 4))) & 15) | (((Aw >> (8 * (j - 4) + 6)) & 3) << 4));
-                    a3[e] = (_Float16)(float)(8 * sc);
-                }
-            }
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const half8 b2 = *reinterpret_cast<const half8 *>(bbuf + BSOFF + 32 * (32 * nt + lr) + 16 * h);
-                msum[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b2, float16v{}, 0, 0, 0);
-                if constexpr (WIDE) cw[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a3, b2, float16v{}, 0, 0, 0);
-            }
-        };
-        // acc += yd d isum - yd dmin msum over the wave's D registers of row tile mt: register RH ks + i
-        // holds row 8 q + 4 h + (i & 3) of the tile, q = (RH ks + i) / 4
-        auto combine = [&](int mt, const float(&tot)[NT][RH], const float(&ms)[NT][RH]) {
-            if constexpr (OUTER) {
-                // yd*d and yd*dmin of the tile's (row, token) pairs as the outer products of an f32 MFMA
-                // with k = 1: one rounding of a single product, the bits of the VALU's multiply (a zero
-                // product may come out +0 where the multiply gives -0; acc starts at +0 and sums of
-                // zeros of either sign keep it +0, so the results are the same). Two blocks: token
-                // tiles 2p and 2p + 1 from lane halves 0 and 1 (past the last tile, block 1 repeats it
-                // and is not read); the D register r of block b holds the row and token that isum's
-                // register r holds.
-#pragma unroll
-                for (int pr = 0; pr < (NT + 1) / 2; pr++) {
-                    const float ydb = h && 2 * pr + 1 < NT ? ydn[2 * pr + 1] : ydn[2 * pr];
-                    const f32x32 da = __builtin_amdgcn_mfma_f32_32x32x1f32(drow[mt], ydb, f32x32{}, 0, 0, 0);
-                    f32x32 dmv = {};
-                    if constexpr (WT == SDY_Q4_K)
-                        dmv = __builtin_amdgcn_mfma_f32_32x32x1f32(mrow[mt], ydb, f32x32{}, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < RH; i++) {
-#pragma unroll
-                        for (int b = 0; b < 2; b++) {
-                            const int nt = 2 * pr + b;
-                            if (nt >= NT) continue;
-                            const int r = 16 * b + RH * ks + i;
-                            if constexpr (WT == SDY_Q4_K) {
-                                const float t1 = da[r] * tot[nt][i], t2 = dmv[r] * ms[nt][i];
-                                acc[mt][nt][i] = acc[mt][nt][i] + (t1 - t2);
-                            } else {
-                                acc[mt][nt][i] = acc[mt][nt][i] + da[r] * tot[nt][i];
-                            }
-                        }
-                    }
-                }
-                return;
-            }
-            float dv[RH], dm[RH];
-            const uint32_t da = lds_addr(dtab + 32 * mt + 4 * h + 8 * (RH / 4) * ks);
-            if constexpr (KS == 1) {
-                f32x4 d0, d1, d2, d3, m0, m1, m2, m3;
-                lds_read8(da, da + 4 * 32 * MT, d0, d1, d2, d3, m0, m1, m2, m3);
-                const f32x4 dq[4] = {d0, d1, d2, d3}, mq[4] = {m0, m1, m2, m3};
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        dv[4 * q + i] = dq[q][i];
-                        dm[4 * q + i] = WT == SDY_Q4_K ? mq[q][i] : 0.0f;
-                    }
-            } else {
-                f32x4 d0, d1, m0, m1;
-                lds_read4(da, da + 4 * 32 * MT, d0, d1, m0, m1);
-                const f32x4 dq[2] = {d0, d1}, mq[2] = {m0, m1};
-#pragma unroll
-                for (int q = 0; q < 2; q++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        dv[4 * q + i] = dq[q][i];
-                        dm[4 * q + i] = WT == SDY_Q4_K ? mq[q][i] : 0.0f;
-                    }
-            }
-#pragma unroll
-            for (int i = 0; i < RH; i++) {
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    if constexpr (WT == SDY_Q4_K) {
-                        const float dall = ydn[nt] * dv[i], dmn = ydn[nt] * dm[i];
-                        const float t1 = dall * tot[nt][i], t2 = dmn * ms[nt][i];
-                        acc[mt][nt][i] = acc[mt][nt][i] + (t1 - t2);
-                    } else {
-                        const float ydd = ydn[nt] * dv[i];
-                        acc[mt][nt][i] = acc[mt][nt][i] + ydd * tot[nt][i];
-                    }
-                }
-            }
-        };
-        if constexpr (KS == 1) {
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                float16v msum[NT], cw[NT];
-                if constexpr (WT == SDY_Q4_K) bsum_mfma(mt, msum, cw);
-                float tot[NT][16], ms[NT][16];
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        float v = isum[mt][nt][r];
-                        // SPLIT6: isum = 16 ihi + ilo, 16 ihi exact, one rounding of the sum (that of (float)isum)
-                        if constexpr (SPLIT6) v = 16.0f * ihi[mt][nt][r] + v;
-                        if constexpr (WT == SDY_Q4_K && WIDE) v = v + cw[nt][r];  // one rounding
-                        tot[nt][r] = v;
-                        ms[nt][r] = WT == SDY_Q4_K ? msum[nt][r] : 0.0f;
-                    }
-                combine(mt, tot, ms);
-            }
-            wait_stage();
-        } else {
-            // before the barrier (after it the stage buffer is refilled): the bsum products, and the half
-            // of the integer sums that the partner completes into its slot
-            float ms[MT][NT][RH], cws[MT][NT][RH];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                float16v msum[NT], cw[NT];
-                if constexpr (WT == SDY_Q4_K) {
-                    bsum_mfma(mt, msum, cw);
-#pragma unroll
-                    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                        for (int i = 0; i < RH; i++) {
-                            ms[mt][nt][i] = ks ? msum[nt][RH + i] : msum[nt][i];
-                            if constexpr (WIDE) cws[mt][nt][i] = ks ? cw[nt][RH + i] : cw[nt][i];
-                        }
-                }
-            }
-            float *xw = xch + (size_t)(cur * WM + wave) * (NXS * MT * NT * 512);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                    for (int i = 0; i < RH; i++) {
-                        const int o = ((mt * NT + nt) * 8 + i) * 64 + lane;
-                        xw[o] = ks ? isum[mt][nt][i] : isum[mt][nt][RH + i];
-                        if constexpr (SPLIT6) xw[MT * NT * 512 + o] = ks ? ihi[mt][nt][i] : ihi[mt][nt][RH + i];
-                    }
-            wait_stage();
-            const float *xr = xch + (size_t)(cur * WM + (wave ^ 1)) * (NXS * MT * NT * 512);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                float tot[NT][RH], msh[NT][RH];
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                    for (int i = 0; i < RH; i++) {
-                        const int o = ((mt * NT + nt) * 8 + i) * 64 + lane;
-                        // the unit halves' sums are integers below 2^24: their sum is isum exactly
-                        float v = (ks ? isum[mt][nt][RH + i] : isum[mt][nt][i]) + xr[o];
-                        if constexpr (SPLIT6) {
-                            const float hi = (ks ? ihi[mt][nt][RH + i] : ihi[mt][nt][i]) + xr[MT * NT * 512 + o];
-                            v = 16.0f * hi + v;
-                        }
-                        if constexpr (WT == SDY_Q4_K && WIDE) v = v + cws[mt][nt][i];
-                        tot[nt][i] = v;
-                        msh[nt][i] = WT == SDY_Q4_K ? ms[mt][nt][i] : 0.0f;
-                    }
-                combine(mt, tot, msh);
-            }
+            if constexpr (KS == 1) acc[i] = acc[i] + term;
+            else xw[i * 64] = term;
         }
     };
-    if constexpr (PF == 1) {
-        SbRegs3 A[MT];
-        load_sb3(0, A);
-        stage(0, 0);
-        __syncthreads();
-        for (int sb = 0; sb < nb; sb++) {
-            SbRegs3 An[MT];
-            iter(sb, A, An);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) A[mt] = An[mt];
-        }
-    } else {
-        // a ring of three register sets, rotated by name
-        SbRegs3 S0[MT], S1[MT], S2[MT];
-        load_sb3(0, S0);
-        stage(0, 0);
-        load_sb3(nb > 1 ? 1 : 0, S1);
-        if (nb > 1) stage(1, 1);
-        __syncthreads();
-        // whole rounds of three, then the rest (no exit inside a round: the compiler's wait tracking
-        // would merge such exits into the loop's back edge, with the next set still pending)
-        int sb = 0;
-        for (; sb + 3 <= nb; sb += 3) {
-            iter(sb, S0, S2);
-            iter(sb + 1, S1, S0);
-            iter(sb + 2, S2, S1);
-        }
-        if (sb < nb) {
-            iter(sb, S0, S2);
-            if (sb + 1 < nb) iter(sb + 1, S1, S0);
-        }
-    }
-    // store (bias, residual, or the SwiGLU pair of rows 2i, 2i+1 held by this lane). The output rows,
-    // bias and residual values are all requested before the first store (one memory round trip);
-    // tokens and rows past the ends read the last valid ones and store nothing.
-    int orow[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const int tok = t0 + 32 * nt + lr;
-        orow[nt] = tok < t_end ? tok : t_end - 1;
-    }
-    if (g.out_row) {
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) orow[nt] = g.out_row[orow[nt]];
-    }
-    auto row_of = [&](int mt, int i) {  // the matrix row of D register RH ks + i of row tile mt (clamped)
-        const int r = RH * ks + i;
-        const long ri = rt + 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
-        return ri < g.n_rows ? ri : g.n_rows - 1;
+    // orders LDS only: the weights in flight stay in flight
+    auto barrier = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-    // the SwiGLU exponential's table in a register (its lane reads need every lane: the values are
-    // computed before the stores' branches)
+    load_a(0);
+    load_s(0);
+#pragma unroll
+    for (int u = 0; u < 4; u++) load_u(0, u);
+    store_a(lds);
+    barrier();
+    for (int s = 0; s < ns; s++) {
+        load_a(s + 1);  // (past the last stage the loads are clamped, their values not used)
+        compute(s, lds + (s & 1) * STAGE);
+        store_a(lds + ((s + 1) & 1) * STAGE);
+        barrier();
+        if constexpr (KS > 1) {
+            const float *xr = xch + (size_t)(rw * KS) * (16 * 64) + NF * ks * 64 + lane;
+            const int left = nb - s * KS;
+            float v[KS][NF];
+#pragma unroll
+            for (int k = 0; k < KS; k++)
+#pragma unroll
+                for (int i = 0; i < NF; i++) v[k][i] = xr[k * (16 * 64) + i * 64];
+#pragma unroll
+            for (int k = 0; k < KS; k++)
+#pragma unroll
+                for (int i = 0; i < NF; i++) acc[i] = k < left ? acc[i] + v[k][i] : acc[i];
+            barrier();  // the terms are read before the next stage's overwrite them
+        }
+    }
+    // register f of the tile's 16 (this wave's: NF ks + i) holds token 8 (f / 4) + 4 h + f % 4, row lr. The residuals and
+    // output rows are requested before the first store.
     const uint32_t etab = sdy_expf_tab_lane(lane);
-    float bv[MT][RH], rv[MT][NT][RH];
-    if (g.bias) {
+    const bool on_row = ri < g.n_rows;
+    const long row = g.grp_tile ? ri : g.row0 + ri;
+    const float bias = g.bias && on_row ? g.bias[row] : 0.0f;
+    int orow[NF];
+    bool on[NF];
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int i = 0; i < RH; i++) bv[mt][i] = g.bias[g.row0 + row_of(mt, i)];
+    for (int i = 0; i < NF; i++) {
+        const int f = NF * ks + i, t = t0 + 8 * (f >> 2) + 4 * h + (f & 3), tc = t < t_end ? t : t_end - 1;
+        on[i] = on_row && t < t_end;
+        orow[i] = g.out_row ? g.out_row[tc] : tc;
     }
-    if (g.resid) {
+    if (g.swiglu) {  // the pair's up row is in the next lane
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                for (int i = 0; i < RH; i++) rv[mt][nt][i] = g.resid[(size_t)orow[nt] * g.out_stride + g.row0 + row_of(mt, i)];
-    }
-    if (g.swiglu) {
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                for (int i = 0; i < RH; i += 2)
-                    acc[mt][nt][i] = sdy_silu_mul1_reg(acc[mt][nt][i], acc[mt][nt][i + 1], etab);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            if (t0 + 32 * nt + lr >= t_end) continue;
-            float *orp = g.out + (size_t)orow[nt] * g.out_stride;
-#pragma unroll
-            for (int i = 0; i < RH; i++) {
-                const int r = RH * ks + i;  // the D register
-                const long ri = rt + 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (ri >= g.n_rows) continue;
-                const long row = g.grp_tile ? ri : g.row0 + ri;
-                if (g.swiglu) {
-                    if ((i & 1) == 0) orp[ri >> 1] = acc[mt][nt][i];
-                } else {
-                    float v = acc[mt][nt][i];
-                    if (g.bias) v = v + bv[mt][i];
-                    if (g.resid) v = rv[mt][nt][i] + v;
-                    orp[row] = v;
-                }
-            }
+        for (int i = 0; i < NF; i++) {
+            const float up = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc[i]), 0xB1, 0xF, 0xF, false));
+            const float v = sdy_silu_mul1_reg(acc[i], up, etab);
+            if (on[i] && !(lr & 1)) g.out[(size_t)orow[i] * g.out_stride + (ri >> 1)] = v;
         }
+        return;
+    }
+    float rv[NF];
+#pragma unroll
+    for (int i = 0; i < NF; i++) rv[i] = g.resid && on[i] ? g.resid[(size_t)orow[i] * g.out_stride + row] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        float v = acc[i];
+        if (g.bias) v = v + bias;
+        if (g.resid) v = rv[i] + v;
+        if (on[i]) g.out[(size_t)orow[i] * g.out_stride + row] = v;
+    }
 }
 
-template <int WT, int MT, int NT, int WM, bool WIDE, int KS = 1, int PF = 1>
-__global__ __launch_bounds__(64 * WM) void k_gemm3(GemmArgs g) {
+template <int WT, int RW, int KS>
+__global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm(GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds[];
-    __shared__ __align__(16) float dtab_all[gemm3_dtab_floats<MT, WM>()];
-    __shared__ float xch[gemm3_xch_floats<WT, MT, NT, WM, WIDE, KS>()];
-    gemm3_body<WT, MT, NT, WM, WIDE, KS, PF>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds,
-                                             dtab_all, xch);
+    gemm_body<WT, RW, KS>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
 }
 
-// Two GEMMs on the same activations in one launch (a layer's q|k and a v of another type): row
-// tiles [0, gy1) of the grid multiply g1, the rest g2; both take the <MT, NT, WM, KS> tile form.
-template <int WT1, bool WIDE1, int WT2, bool WIDE2, int MT, int NT, int WM, int KS>
-__global__ __launch_bounds__(64 * WM) void k_gemm3_pair(GemmArgs g1, GemmArgs g2, int gy1) {
+// Two GEMMs on the same activations in one launch (a layer's q|k and a v of another type): row tiles [0, gy1) of
+// the grid multiply g1, the rest g2.
+template <int WT1, int WT2, int RW, int KS>
+__global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm_pair(GemmArgs g1, GemmArgs g2, int gy1) {
     extern __shared__ __align__(16) uint8_t lds[];
-    constexpr int X1 = gemm3_xch_floats<WT1, MT, NT, WM, WIDE1, KS>(), X2 = gemm3_xch_floats<WT2, MT, NT, WM, WIDE2, KS>();
-    __shared__ __align__(16) float dtab_all[gemm3_dtab_floats<MT, WM>()];
-    __shared__ float xch[X1 > X2 ? X1 : X2];
-    if ((int)blockIdx.y < gy1)
-        gemm3_body<WT1, MT, NT, WM, WIDE1, KS, 1>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds,
-                                                  dtab_all, xch);
-    else
-        gemm3_body<WT2, MT, NT, WM, WIDE2, KS, 1>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x,
-                                                  (int)gridDim.y - gy1, lds, dtab_all, xch);
+    if ((int)blockIdx.y < gy1) gemm_body<WT1, RW, KS>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds);
+    else gemm_body<WT2, RW, KS>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x, (int)gridDim.y - gy1, lds);
 }
 
-
-// Q8_K rows -> f16 values, f32 scales and f16 bsums for the GEMM (all exact: |q| <= 127, |bsum| <=
-// 2032). One thread per 16 values of a super-block (n_sb = n_tok * nb super-blocks in a row): four
-// 4-byte loads, two 16-byte stores, and the super-block's bsum number `part`; 256 threads.
-__global__ __launch_bounds__(256) void k_gemm_prep(const uint8_t *__restrict__ xq, long n_sb,
-                                                   _Float16 *__restrict__ y16, float *__restrict__ yd,
-                                                   _Float16 *__restrict__ bs16) {
-    const long g = blockIdx.x * 256L + threadIdx.x, sbg = g >> 4;
-    const int part = (int)(g & 15);
+// Q8_K rows -> the GEMM's expansion: int8 values, f32 scales and f16 sums in planes of their own (exact: |bsum| <=
+// 2032). One thread per 16 values of a super-block (n_sb = n_tok * nb super-blocks in a row); 256 threads.
+__global__ __launch_bounds__(256) void k_gemm_prep(const uint8_t *__restrict__ xq, long n_sb, SdyGemmExp e) {
+    const long i = blockIdx.x * 256L + threadIdx.x, sbg = i >> 4;
+    const int part = (int)(i & 15);
     if (sbg >= n_sb) return;
     const uint8_t *blk = xq + sbg * 292;
-    const uint32_t *q4 = reinterpret_cast<const uint32_t *>(blk + 4 + 16 * part);
-    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-    f16x8 o[2];
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-        const uint32_t v = q4[w];
-#pragma unroll
-        for (int e = 0; e < 4; e++) o[w >> 1][4 * (w & 1) + e] = (_Float16)(float)(int8_t)((v >> (8 * e)) & 255u);
-    }
-    f16x8 *dst = reinterpret_cast<f16x8 *>(y16 + sbg * 256 + 16 * part);
-    dst[0] = o[0];
-    dst[1] = o[1];
-    bs16[sbg * 16 + part] = (_Float16)(float)reinterpret_cast<const int16_t *>(blk + 260)[part];
-    if (part == 0) yd[sbg] = *reinterpret_cast<const float *>(blk);
+    const uint32_t *q = reinterpret_cast<const uint32_t *>(blk + 4 + 16 * part);
+    *reinterpret_cast<u32x4 *>(e.y8 + sbg * 256 + 16 * part) = u32x4{q[0], q[1], q[2], q[3]};
+    e.bs16[sbg * 16 + part] = (_Float16)(float)reinterpret_cast<const int16_t *>(blk + 260)[part];
+    if (part == 0) e.yd[sbg] = *reinterpret_cast<const float *>(blk);
 }
 
-// Which variant of the GEMM multiplies a K-quant matrix exactly: flags a row super-block whose
-// 127 * sum |w'| reaches 2^24 or (Q6_K) whose |sc * (q - 32)| exceeds 2048, which the one-fragment
-// scheme would round; the wide variant multiplies every block exactly. One thread per
-// (row, super-block) of rows [0, n_rows) of the planes.
+// What sdy_mat's gemm_ok says of a K-quant matrix: flags a row super-block whose 127 * sum |sc * q| reaches 2^24 or
+// (Q6_K) whose |sc * (q - 32)| exceeds 2048. (The GEMM multiplies either exactly.) One thread per (row,
+// super-block) of rows [0, n_rows) of the planes.
 template <int WT>
 __global__ void k_gemm_check(GemmArgs g, int *bad) {
     const long gid = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -1000,7 +444,7 @@ extern "C" size_t sdy_gemm_layout_planes(int type, int n_in, long rows, size_t o
     return gemm_layout_planes(type, n_in, rows, off, sz, nrec, rsz);
 }
 
-// The kernel arguments of m; with its GEMM copy (k_gemm3) when it has one and `layout` is set.
+// The kernel arguments of m; with its tiled copy when it has one and `layout` is set.
 static GemmArgs gemm_args(const sdy_mat *m, bool layout = false) {
     GemmArgs g;
     memset(&g, 0, sizeof(g));
@@ -1009,19 +453,13 @@ static GemmArgs gemm_args(const sdy_mat *m, bool layout = false) {
     g.T = m->n_units;
     g.nb = m->n_in / 256;
     g.n_rows = m->n_rows;
-    const size_t rows = (size_t)m->n_rows, unit = rows * g.T * 16, sbk = rows * g.nb;
-    size_t sz[5] = {unit, unit, m->type == SDY_Q4_K ? sbk * 16 : unit, m->type == SDY_Q4_K ? 0 : sbk * 16,
-                    m->type == SDY_Q4_K ? 0 : sbk * 2};
     if (layout && m->gbase) {
         size_t off[5];
-        int nrec[5], rsz[5];
-        gemm_layout_planes(m->type, m->n_in, m->grows, off, sz, nrec, rsz);
+        sdy_gemm_layout_planes(m->type, m->n_in, m->grows, off);
         for (int i = 0; i < 5; i++) g.p[i] = (const uint8_t *)m->gbase + off[i];
         g.blk = 1;
         g.grow0 = m->grow0;
     }
-    for (int i = 0; i < 5; i++) g.psz[i] = sz[i] < 0xFFFFFFFFu ? (uint32_t)sz[i] : 0xFFFFFFFFu;
-    g.wide = m->gemm_ok == 2;
     return g;
 }
 
@@ -1081,7 +519,7 @@ extern "C" int sdy_mat_gemm_layout(sdy_mat *m, sdy_stream s) {
     return 0;
 }
 
-// Flags (bad = 1) rows [r0, r0 + n) of m that the GEMM cannot multiply exactly. Synchronous.
+// Flags (bad = 1) rows [r0, r0 + n) of m with a block of gemm_ok 2. Synchronous.
 extern "C" int sdy_gemm_check_rows_async(const sdy_mat *m, long r0, long n, int *bad_dev, sdy_stream s) {
     if ((m->type != SDY_Q4_K && m->type != SDY_Q6_K) || m->hbase) return 0;  // (host memory: wide, unchecked)
     sdy_mat v = sdy_mat_rows(m, r0, n);
@@ -1115,84 +553,69 @@ extern "C" int sdy_gemm_check_rows(const sdy_mat *m, long r0, long n, int *bad_h
 
 extern "C" size_t sdy_gemm_ws_bytes(int n_tok, int n_in) {
     const size_t nb = (size_t)n_in / 256;
-    return (size_t)n_tok * n_in * 2 + (size_t)n_tok * nb * 4 + (size_t)n_tok * nb * 32 + 3 * 256;
+    return (size_t)n_tok * n_in + (size_t)n_tok * nb * 4 + (size_t)n_tok * nb * 32 + 3 * 256;
 }
 
 extern "C" int sdy_gemm_ok(const sdy_mat *m, int n_tok) {
-    // buffer resources address each plane with 32-bit offsets: planes below 4 GiB
     return (m->type == SDY_Q4_K || m->type == SDY_Q6_K) && m->gemm_ok && n_tok >= 2 &&
            (size_t)m->n_rows * m->n_units * 16 < 0xFFFFFFFFu;
 }
 
-template <int WT, int MT, int NT, int WM, bool WIDE, int KS, int PF>
-static int launch_gemm3_s(GemmArgs &g, hipStream_t st) {
-    constexpr int BN = 32 * NT, BM = 32 * MT * WM / KS, YDN = BN < 64 ? 64 : BN;
-    constexpr size_t lds = (PF + 1) * (size_t)(BN * 512 + (PF == 2 ? WM : 1) * YDN * 4 + BN * 32);
+// A Q4_K lane reaches both quant planes by one 32-bit offset from its row tile in the first. (A plane of 4 GiB: the
+// rows of one take the matvec.)
+static bool gemm_far(const GemmArgs &g) { return (size_t)(g.p[1] - g.p[0]) + (size_t)g.T * 4096 > 0xFFFFFFFFu; }
+
+template <int WT, int RW, int KS>
+static int launch_gemm(const GemmArgs &g, unsigned tok_tiles, hipStream_t st) {
+    constexpr size_t lds = gemm_lds_bytes<RW, KS>();
     static size_t granted = 0;
-    const void *fn = (const void *)k_gemm3<WT, MT, NT, WM, WIDE, KS, PF>;
-    int rc = sdy_lds_limit(fn, lds, &granted);
-    if (rc) return rc;
-    const unsigned tok_tiles = (unsigned)((g.n_tok + BN - 1) / BN), row_tiles = (unsigned)((g.n_rows + BM - 1) / BM);
-    SDY_NOTE_KERNEL((k_gemm3<WT, MT, NT, WM, WIDE, KS, PF>));
-    hipLaunchKernelGGL((k_gemm3<WT, MT, NT, WM, WIDE, KS, PF>), dim3(tok_tiles, row_tiles), dim3(64 * WM), lds, st, g);
+    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS>, lds, &granted)) return rc;
+    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS>));
+    hipLaunchKernelGGL((k_gemm<WT, RW, KS>), dim3(tok_tiles, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))), dim3(64 * RW * KS),
+                       lds, st, g);
     return sdy_check_launch("gemm");
 }
 
-// g.wide: the matrix has blocks that the one-fragment scheme cannot multiply exactly
-template <int WT, int MT, int NT, int WM, int KS = 1, int PF = 1>
-static int launch_gemm3(GemmArgs &g, hipStream_t st) {
-    return g.wide ? launch_gemm3_s<WT, MT, NT, WM, true, KS, PF>(g, st)
-                  : launch_gemm3_s<WT, MT, NT, WM, false, KS, PF>(g, st);
-}
-
-template <int WT, int MT, int NT, int WM, bool WIDE, int KS>
-static int launch_gemm3_grid_s(GemmArgs &g, unsigned tok_tiles, unsigned row_tiles, hipStream_t st) {
-    constexpr int BN = 32 * NT, YDN = BN < 64 ? 64 : BN;
-    constexpr size_t lds = 2 * (size_t)(BN * 512 + YDN * 4 + BN * 32);
-    static size_t granted = 0;
-    const void *fn = (const void *)k_gemm3<WT, MT, NT, WM, WIDE, KS>;
-    int rc = sdy_lds_limit(fn, lds, &granted);
-    if (rc) return rc;
-    SDY_NOTE_KERNEL((k_gemm3<WT, MT, NT, WM, WIDE, KS>));
-    hipLaunchKernelGGL((k_gemm3<WT, MT, NT, WM, WIDE, KS>), dim3(tok_tiles, row_tiles), dim3(64 * WM), lds, st, g);
-    return sdy_check_launch("gemm");
-}
-
-template <int WT, int MT, int NT, int WM, int KS>
-static int launch_gemm3_grid(GemmArgs &g, unsigned tok_tiles, unsigned row_tiles, hipStream_t st) {
-    return g.wide ? launch_gemm3_grid_s<WT, MT, NT, WM, true, KS>(g, tok_tiles, row_tiles, st)
-                   : launch_gemm3_grid_s<WT, MT, NT, WM, false, KS>(g, tok_tiles, row_tiles, st);
+// The forms of the GEMM, by the 32 x 32 tiles of its output: four waves to two tiles' super-blocks each (KS 4) while
+// the tiles alone are fewer than two to a CU, two up to eight (KS 2), one to a tile beyond (with the quantiser's
+// launch, forms KS 4, 2, 1: Q4_K 2048 x 2048, 130 tokens: 11.8, 13.6, 17.3 us; 512 tokens: 21.2, 18.5, 19.1;
+// 22016 x 2048, 64 tokens: 27.0, 20.8, 22.6; 128 tokens: 47.4, 33.4, 29.0).
+static int gemm_form(long n_rows, int n_tok) {
+    const long tiles = (n_rows + 31) / 32 * ((n_tok + 31) / 32);
+    return tiles < 512 ? 4 : tiles < 2048 ? 2 : 1;
 }
 
 template <int WT>
-static int gemm_type(GemmArgs &g, hipStream_t st) {
-    // SARDYNE_GEMM_VARIANT picks one tile shape (tests and tuning); default: by shape
+static int gemm_type(const GemmArgs &g, const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
+    // SARDYNE_GEMM_VARIANT picks one form (tests and tuning); default: by shape
     const char *ev = getenv("SARDYNE_GEMM_VARIANT");
-    const int variant = ev ? atoi(ev) : 1;
-    switch (variant) {
-    case 11: return launch_gemm3<WT, 1, 4, 8>(g, st);
-    case 12: return launch_gemm3<WT, 1, 2, 4>(g, st);
-    case 13: return launch_gemm3<WT, 1, 2, 8>(g, st);
-    case 14: return launch_gemm3<WT, 1, 1, 4>(g, st);
-    case 15: return launch_gemm3<WT, 1, 4, 4>(g, st);
-    case 16: return launch_gemm3<WT, 2, 2, 4>(g, st);
-    case 17: return launch_gemm3<WT, 1, 1, 4, 2>(g, st);
-    case 18: return launch_gemm3<WT, 1, 1, 8, 2>(g, st);
-    case 19: return launch_gemm3<WT, 1, 1, 4, 1, 2>(g, st);
-    case 20: return launch_gemm3<WT, 1, 1, 4, 2, 2>(g, st);
-    default: break;
+    const int variant = ev ? atoi(ev) : 0;
+    const unsigned tt = (unsigned)((g.n_tok + 31) / 32);
+    // Small grids: the 16 x 16 tiles of mm_superblocks.hip, up to 2.5 to a CU, and up to 16 tokens on more rows (with the
+    // quantiser's launch: Q4_K 2560 x 2048, 64 tokens: 10.0 us against 11.4, 128 tokens 12.7 against 11.8; 22016 x 2048,
+    // 16 tokens: 12.2 against 16.1, 24 tokens 18.1 against 16.3; Q6_K 2048 x 11008, 64 tokens 31.6 against 42.3, 128
+    // tokens 63.7 against 44.3; 151936 x 2048, 16 tokens: 88.4 against 72.5).
+    const long t16 = (g.n_rows + 15) / 16 * ((g.n_tok + 15) / 16);
+    const bool small = variant == 14 || (!variant && (t16 <= 640 || (g.n_tok <= 16 && t16 <= (WT == SDY_Q4_K ? 4096 : 1024))));
+    if (small) {
+        const int rc = sdy_mm_superblocks_exp(m, a, &g.e, (sdy_stream)st);
+        if (rc <= 0) return rc;
     }
-    // 128-row workgroup tiles (4 waves of 32 rows) of 64 tokens when there are enough row tiles to
-    // fill the GPU twice over with them; else 64-row tiles of 32 tokens, two waves to a row tile
-    // splitting each super-block's units (twice the waves for the grids of one wave per SIMD).
-    // Measured on the 256- to 22016-row matrices of a 512-token prefill.
-    const long r128 = (g.n_rows + 127) / 128, t64 = (g.n_tok + 63) / 64;
-    if (r128 * t64 >= 1024) return launch_gemm3<WT, 1, 2, 4>(g, st);
-    return launch_gemm3<WT, 1, 1, 4, 2>(g, st);
+    const int form = variant == 11 ? 1 : variant == 12 ? 2 : variant == 13 ? 4 : gemm_form(g.n_rows, g.n_tok);
+    if (form == 4) return launch_gemm<WT, 2, 4>(g, tt, st);
+    return form == 2 ? launch_gemm<WT, 2, 2>(g, tt, st) : launch_gemm<WT, 4, 1>(g, tt, st);
 }
 
-// out[t][row] for rows [a->row0, a->row1) and a->n_tok tokens of Q8_K activations a->xq, through
-// the MFMA GEMM; ws: sdy_gemm_ws_bytes(n_tok, n_in) bytes of device scratch.
+// The activations' expansion of one call in ws: made unless ws_ready.
+static int gemm_expand(const sdy_mv_args *a, int rows, int n_in, void *ws, SdyGemmExp &e, hipStream_t st) {
+    e = sdy_gemm_exp(ws, rows, n_in);
+    if (a->ws_ready) return 0;
+    const long n_sb = (long)rows * (n_in / 256);
+    SDY_NOTE_KERNEL(k_gemm_prep);
+    hipLaunchKernelGGL(k_gemm_prep, dim3((unsigned)((n_sb * 16 + 255) / 256)), dim3(256), 0, st, (const uint8_t *)a->xq, n_sb, e);
+    return sdy_check_launch("gemm_prep");
+}
+
 // The checks and kernel arguments of one sdy_gemm call; the activations' expansion is made first
 // unless ws_ready. *empty: an empty row range (nothing to launch).
 static int gemm_setup(const sdy_mat *m, const sdy_mv_args *a, void *ws, hipStream_t st, GemmArgs &g, bool *empty) {
@@ -1207,22 +630,10 @@ static int gemm_setup(const sdy_mat *m, const sdy_mv_args *a, void *ws, hipStrea
         return 0;
     }
     g = gemm_args(m, true);
-    const int nb = g.nb, n_tok = a->n_tok;
-    const SdyGemmExp e = sdy_gemm_exp(ws, n_tok, g.n_in);
-    g.exp_rows = n_tok;
-    g.y16 = e.y16;
-    g.yd = e.yd;
-    g.bs16 = e.bs16;
-    if (!a->ws_ready) {
-        const long n_sb = (long)n_tok * nb;
-        SDY_NOTE_KERNEL(k_gemm_prep);
-        hipLaunchKernelGGL(k_gemm_prep, dim3((unsigned)((n_sb * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const uint8_t *)a->xq, n_sb, (_Float16 *)g.y16, (float *)g.yd, (_Float16 *)g.bs16);
-        if (int rc = sdy_check_launch("gemm_prep")) return rc;
-    }
+    if (int rc = gemm_expand(a, a->n_tok, g.n_in, ws, g.e, st)) return rc;
     g.row0 = a->row0;
     g.n_rows = a->row1 - a->row0;
-    g.n_tok = n_tok;
+    g.n_tok = a->n_tok;
     g.out = a->out;
     g.out_stride = a->out_stride;
     g.bias = a->bias;
@@ -1232,63 +643,56 @@ static int gemm_setup(const sdy_mat *m, const sdy_mv_args *a, void *ws, hipStrea
     return 0;
 }
 
+// out[t][row] for rows [a->row0, a->row1) and a->n_tok tokens of Q8_K activations a->xq; ws:
+// sdy_gemm_ws_bytes(n_tok, n_in) bytes of device scratch.
 extern "C" int sdy_gemm(const sdy_mat *m, const sdy_mv_args *a, void *ws, sdy_stream s) {
     hipStream_t st = (hipStream_t)s;
     GemmArgs g;
     bool empty;
     if (int rc = gemm_setup(m, a, ws, st, g, &empty)) return rc;
     if (empty) return 0;
-    return m->type == SDY_Q4_K ? gemm_type<SDY_Q4_K>(g, st) : gemm_type<SDY_Q6_K>(g, st);
+    if (gemm_far(g)) return sdy_matvec(m, a, s);
+    return m->type == SDY_Q4_K ? gemm_type<SDY_Q4_K>(g, m, a, st) : gemm_type<SDY_Q6_K>(g, m, a, st);
 }
 
-// the small-grid tile form of gemm_type (64-row tiles of 32 tokens, the unit split)
-static bool gemm_small_grid(long n_rows, int n_tok) {
-    return ((n_rows + 127) / 128) * (long)((n_tok + 63) / 64) < 1024;
-}
-
-template <int WT1, bool WIDE1, int WT2, bool WIDE2>
-static int launch_gemm3_pair_s(GemmArgs &g1, GemmArgs &g2, hipStream_t st) {
-    constexpr int NT = 1, BN = 32 * NT, YDN = 64, BM = 64;
-    constexpr size_t lds = 2 * (size_t)(BN * 512 + YDN * 4 + BN * 32);
+template <int RW, int KS>
+static int launch_gemm_pair(const GemmArgs &g1, const GemmArgs &g2, hipStream_t st) {
+    constexpr size_t lds = gemm_lds_bytes<RW, KS>();
     static size_t granted = 0;
-    const void *fn = (const void *)k_gemm3_pair<WT1, WIDE1, WT2, WIDE2, 1, NT, 4, 2>;
-    int rc = sdy_lds_limit(fn, lds, &granted);
-    if (rc) return rc;
-    const unsigned tok_tiles = (unsigned)((g1.n_tok + BN - 1) / BN);
-    const int gy1 = (int)((g1.n_rows + BM - 1) / BM), gy2 = (int)((g2.n_rows + BM - 1) / BM);
-    SDY_NOTE_KERNEL((k_gemm3_pair<WT1, WIDE1, WT2, WIDE2, 1, NT, 4, 2>));
-    hipLaunchKernelGGL((k_gemm3_pair<WT1, WIDE1, WT2, WIDE2, 1, NT, 4, 2>), dim3(tok_tiles, (unsigned)(gy1 + gy2)),
-                       dim3(256), lds, st, g1, g2, gy1);
+    if (int rc = sdy_lds_limit((const void *)k_gemm_pair<SDY_Q4_K, SDY_Q6_K, RW, KS>, lds, &granted)) return rc;
+    const int gy1 = (int)((g1.n_rows + 32 * RW - 1) / (32 * RW)), gy2 = (int)((g2.n_rows + 32 * RW - 1) / (32 * RW));
+    SDY_NOTE_KERNEL((k_gemm_pair<SDY_Q4_K, SDY_Q6_K, RW, KS>));
+    hipLaunchKernelGGL((k_gemm_pair<SDY_Q4_K, SDY_Q6_K, RW, KS>), dim3((unsigned)((g1.n_tok + 31) / 32), (unsigned)(gy1 + gy2)),
+                       dim3(64 * RW * KS), lds, st, g1, g2, gy1);
     return sdy_check_launch("gemm2");
 }
 
-// Two GEMMs over the same activations (a layer's q|k and its v): one launch when the first matrix
-// is Q4_K and the second Q6_K, each on the small-grid tile form (the bits of two sdy_gemm calls);
-// otherwise, or with SARDYNE_GEMM_VARIANT set, two sdy_gemm calls.
+// Two GEMMs over the same activations (a layer's q|k and its v): one launch when the first matrix is Q4_K and the
+// second Q6_K and neither would fill the GPU by itself (the KS forms); otherwise, or with SARDYNE_GEMM_VARIANT set, two
+// sdy_gemm calls. The same bits either way.
 extern "C" int sdy_gemm2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat *m2, const sdy_mv_args *a2, void *ws,
                          sdy_stream s) {
     hipStream_t st = (hipStream_t)s;
     if (a2->xq != a1->xq || a2->n_tok != a1->n_tok || m2->n_in != m1->n_in)
         return sdy_fail(-1, "gemm2: the two GEMMs must read the same activation rows");
+    const long rows = (a1->row1 - a1->row0) + (a2->row1 - a2->row0);
     const bool pair = m1->type == SDY_Q4_K && m2->type == SDY_Q6_K && !getenv("SARDYNE_GEMM_VARIANT") &&
-                      a1->row1 > a1->row0 && a2->row1 > a2->row0 && gemm_small_grid(a1->row1 - a1->row0, a1->n_tok) &&
-                      gemm_small_grid(a2->row1 - a2->row0, a2->n_tok);
+                      a1->row1 > a1->row0 && a2->row1 > a2->row0 && gemm_form(rows, a1->n_tok) > 1;
+    sdy_mv_args b = *a2;
+    b.ws_ready = 1;  // the expansion the first call makes (or finds)
     if (!pair) {
         if (int rc = sdy_gemm(m1, a1, ws, s)) return rc;
-        sdy_mv_args b = *a2;
-        b.ws_ready = 1;  // the expansion the first call made (or found)
         return sdy_gemm(m2, &b, ws, s);
     }
     GemmArgs g1, g2;
     bool e1, e2;
-    sdy_mv_args b = *a2;
-    b.ws_ready = 1;
     if (int rc = gemm_setup(m1, a1, ws, st, g1, &e1)) return rc;  // (both ranges non-empty here)
     if (int rc = gemm_setup(m2, &b, ws, st, g2, &e2)) return rc;
-    if (g1.wide) return g2.wide ? launch_gemm3_pair_s<SDY_Q4_K, true, SDY_Q6_K, true>(g1, g2, st)
-                                : launch_gemm3_pair_s<SDY_Q4_K, true, SDY_Q6_K, false>(g1, g2, st);
-    return g2.wide ? launch_gemm3_pair_s<SDY_Q4_K, false, SDY_Q6_K, true>(g1, g2, st)
-                   : launch_gemm3_pair_s<SDY_Q4_K, false, SDY_Q6_K, false>(g1, g2, st);
+    if (gemm_far(g1)) {
+        if (int rc = sdy_matvec(m1, a1, s)) return rc;
+        return sdy_gemm(m2, &b, ws, s);
+    }
+    return gemm_form(rows, g1.n_tok) == 4 ? launch_gemm_pair<2, 4>(g1, g2, st) : launch_gemm_pair<2, 2>(g1, g2, st);
 }
 
 extern "C" int sdy_gemm_grouped_tile(void) { return 32; }
@@ -1310,19 +714,8 @@ extern "C" int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, cons
         return sdy_fail(-1, "gemm_grouped: activation rows by index read an expansion of n_act >= 1 rows that the "
                             "caller made (ws_ready)");
     GemmArgs g = gemm_args(m, true);
-    const SdyGemmExp e = sdy_gemm_exp(ws, act_row ? n_act : n_tok, g.n_in);
-    g.exp_rows = act_row ? n_act : n_tok;
-    g.y16 = e.y16;
-    g.yd = e.yd;
-    g.bs16 = e.bs16;
-    int rc;
-    if (!a->ws_ready) {
-        const long n_sb = (long)n_tok * g.nb;
-        SDY_NOTE_KERNEL(k_gemm_prep);
-        hipLaunchKernelGGL(k_gemm_prep, dim3((unsigned)((n_sb * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const uint8_t *)a->xq, n_sb, (_Float16 *)g.y16, (float *)g.yd, (_Float16 *)g.bs16);
-        if ((rc = sdy_check_launch("gemm_prep"))) return rc;
-    }
+    if (int rc = gemm_expand(a, act_row ? n_act : n_tok, g.n_in, ws, g.e, st)) return rc;
+    if (gemm_far(g)) return sdy_fail(-1, "gemm_grouped: quant planes of 4 GiB");
     g.row0 = 0;
     g.n_rows = grp_rows;
     g.n_tok = n_tok;
@@ -1337,13 +730,11 @@ extern "C" int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, cons
     g.act_row = act_row;
     g.grp_rows = grp_rows;
     g.n_grp = n_grp;
-    // token tiles: at most one partial tile per group beyond the full ones (the grid's extra
-    // workgroups return at once)
-    // (128-row tiles, one wave to a row tile: the unit split of the dense GEMM's small grids measured
-    // slower here, 38.5 against 36.3 ms for the 30B-A3B-shaped 1024-token prefill)
-    constexpr int BN = 32;
-    const unsigned tok_tiles = (unsigned)((n_tok + BN - 1) / BN + n_grp - 1);
-    const unsigned row_tiles = (unsigned)((grp_rows + 127) / 128);
-    return m->type == SDY_Q4_K ? launch_gemm3_grid<SDY_Q4_K, 1, 1, 4, 1>(g, tok_tiles, row_tiles, st)
-                               : launch_gemm3_grid<SDY_Q6_K, 1, 1, 4, 1>(g, tok_tiles, row_tiles, st);
+    // token tiles: at most one partial tile per group beyond the full ones (the grid's extra workgroups return at once)
+    const unsigned tok_tiles = (unsigned)((n_tok + 31) / 32 + n_grp - 1);
+    const char *ev = getenv("SARDYNE_GEMM_VARIANT");
+    const int v = ev ? atoi(ev) : 0;
+    if (v == 12) return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 2, 2>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 2, 2>(g, tok_tiles, st);
+    if (v == 13) return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 2, 4>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 2, 4>(g, tok_tiles, st);
+    return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 4, 1>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 4, 1>(g, tok_tiles, st);
 }

@@ -31,7 +31,8 @@ struct SbArgs {
     int blk;              // records [row / 32][record][row % 32]; row r is row grow0 + r there
     long grow0;
     long row0, n_rows;
-    const uint8_t *xq;    // Q8_K rows, nb blocks of 292 bytes
+    const uint8_t *xq;    // Q8_K rows, nb blocks of 292 bytes,
+    SdyGemmExp e;         // or the GEMM's expansion of them
     int n_tok;
     float *out;
     long out_stride;
@@ -54,7 +55,7 @@ SDY_DEV void opaque(i32x4 &v) { __asm__ volatile("" : "+v"(v)); }
 
 constexpr int KS = 8;  // waves, super-blocks of a round
 
-template <int WT, int MT>
+template <int WT, int MT, bool EXP>
 __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     constexpr bool Q4 = WT == SDY_Q4_K;
     constexpr int OUT = MT * 256, NTH = 64 * KS;  // outputs of the workgroup, threads
@@ -77,13 +78,15 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
         vs[m] = g.blk ? ((R >> 5) * (uint32_t)nb * 32u + (R & 31u)) : (uint32_t)rc * (uint32_t)nb;
     }
     const int ss = g.blk ? 32 : 1;  // super-block records from one to the next
-    const __amdgpu_buffer_rsrc_t r0 = rsrc(g.p[0]), r2 = rsrc(g.p[2]), r3 = rsrc(g.p[3]), r4 = rsrc(g.p[4]), rx = rsrc(g.xq);
+    const __amdgpu_buffer_rsrc_t r0 = rsrc(g.p[0]), r2 = rsrc(g.p[2]), r3 = rsrc(g.p[3]), r4 = rsrc(g.p[4]),
+                                 rx = rsrc(EXP ? (const uint8_t *)g.e.y8 : g.xq), ry = rsrc((const uint8_t *)g.e.yd), rb = rsrc((const uint8_t *)g.e.bs16);
     // token n's row for the products, tokens 4 q + i for the scales of the results
-    auto tok_row = [&](int t) { return (uint32_t)(t0 + t < g.n_tok ? t0 + t : g.n_tok - 1) * (uint32_t)nb * 292u; };
-    const uint32_t va = tok_row(n);
+    constexpr uint32_t XB = EXP ? 256u : 292u, YB = EXP ? 4u : 292u;
+    auto tok_sb = [&](int t) { return (uint32_t)(t0 + t < g.n_tok ? t0 + t : g.n_tok - 1) * (uint32_t)nb; };
+    const uint32_t va = tok_sb(n) * XB, vb = tok_sb(n) * 32u;
     uint32_t vy[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) vy[i] = tok_row(4 * q + i);
+    for (int i = 0; i < 4; i++) vy[i] = tok_sb(4 * q + i) * YB;
 
     struct Regs {
         u32x2 w[MT][4], hb[Q4 ? 1 : MT][4];
@@ -93,12 +96,13 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
         float yd[4];
     };
     auto load = [&](int sb, Regs &r) {
-        const int xb = sb * 292;
+        const int xb = sb * (int)XB;
 #pragma unroll
-        for (int i = 0; i < 4; i++) r.yd[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, vy[i], xb, 0));
-        r.bs = bload8(rx, va + 8u * (uint32_t)q, xb + 260);
+        for (int i = 0; i < 4; i++)
+            r.yd[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(EXP ? ry : rx, vy[i], sb * (int)YB, 0));
+        r.bs = EXP ? bload8(rb, vb + 8u * (uint32_t)q, sb * 32) : bload8(rx, va + 8u * (uint32_t)q, xb + 260);
 #pragma unroll
-        for (int j = 0; j < 8; j++) r.a[j] = bload8(rx, va + 8u * (uint32_t)q, xb + 4 + 32 * j);
+        for (int j = 0; j < 8; j++) r.a[j] = bload8(rx, va + 8u * (uint32_t)q, xb + (EXP ? 0 : 4) + 32 * j);
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             r.sc[m] = __builtin_amdgcn_raw_buffer_load_b128(Q4 ? r2 : r3, vs[m] * 16u, sb * ss * 16, 0);
@@ -113,8 +117,12 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     // the super-block's f32 terms of the lane's outputs (token 4 q + i, row n), as the matvec forms them
     auto compute = [&](const Regs &r, float *dst) {
         f16x4 bsf;
+        if constexpr (EXP) {
+            bsf = __builtin_bit_cast(f16x4, r.bs);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++) bsf[e] = (_Float16)(float)(int16_t)(r.bs[e >> 1] >> (16 * (e & 1)));
+            for (int e = 0; e < 4; e++) bsf[e] = (_Float16)(float)(int16_t)(r.bs[e >> 1] >> (16 * (e & 1)));
+        }
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             i32x4 isum = {};
@@ -239,23 +247,20 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     }
 }
 
-template <int WT, int MT>
+template <int WT, int MT, bool EXP>
 int launch_sb(const SbArgs &g, hipStream_t st) {
-    SDY_NOTE_KERNEL((k_mm_superblocks<WT, MT>));
-    hipLaunchKernelGGL((k_mm_superblocks<WT, MT>),
+    SDY_NOTE_KERNEL((k_mm_superblocks<WT, MT, EXP>));
+    hipLaunchKernelGGL((k_mm_superblocks<WT, MT, EXP>),
                        dim3((unsigned)((g.n_tok + 15) / 16), (unsigned)((g.n_rows + 16 * MT - 1) / (16 * MT))), dim3(64 * KS), 0, st, g);
     return sdy_check_launch("matvec (super-block MFMA)");
 }
 
-}  // namespace
-
-// The tokens of a->xq through rows [a->row0, a->row1) of m (Q4_K, Q6_K), with the bits of sdy_matvec. Returns 1,
-// launching nothing, when the kernel's 32-bit offsets do not reach every byte of the matrix or the activations.
-extern "C" int sdy_mm_superblocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s) {
+template <bool EXP>
+int run_sb(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, hipStream_t st) {
     const int nb = m->n_in / 256;
     const size_t lim = 0xFFFFFFFFu;
     const long n_rows = a->row1 - a->row0;
-    if (m->bytes >= lim || m->gbytes >= lim || (size_t)nb * 292 * a->n_tok >= lim || ((uintptr_t)a->xq & 3) ||
+    if (m->bytes >= lim || m->gbytes >= lim || (size_t)nb * 292 * a->n_tok >= lim || (!EXP && ((uintptr_t)a->xq & 3)) ||
         (n_rows + 15) / 16 > 65535)
         return 1;
     SbArgs g = {};
@@ -271,17 +276,33 @@ extern "C" int sdy_mm_superblocks(const sdy_mat *m, const sdy_mv_args *a, sdy_st
     g.nb = nb;
     g.row0 = a->row0;
     g.n_rows = n_rows;
-    g.xq = (const uint8_t *)a->xq;
+    if (EXP) g.e = *e;
+    else g.xq = (const uint8_t *)a->xq;
     g.n_tok = a->n_tok;
     g.out = a->out;
     g.out_stride = a->out_stride;
     g.bias = a->bias;
     g.resid = a->resid;
     g.swiglu = a->epilogue == SDY_EPI_SWIGLU;
-    hipStream_t st = (hipStream_t)s;
-    // two row tiles to a wave, sharing the activations' loads, when one each gives every CU more than two workgroups
-    // (22016 x 2048 Q4_K, 8 tokens: 11.2 us against 13.2; 2048 x 4096: 10.0 against 8.4). Not for Q6_K, whose registers
-    // then leave two waves to a SIMD (151936 x 2048: 104 us against 84)
-    if (m->type == SDY_Q6_K) return launch_sb<SDY_Q6_K, 1>(g, st);
-    return (n_rows + 15) / 16 * ((g.n_tok + 15) / 16) > 512 ? launch_sb<SDY_Q4_K, 2>(g, st) : launch_sb<SDY_Q4_K, 1>(g, st);
+    // Two row tiles to a wave, sharing the activations' loads: Q4_K when one each gives every CU more than two
+    // workgroups (22016 x 2048, 8 tokens: 11.2 us against 13.2; 2048 x 4096: 10.0 against 8.4), Q6_K, whose registers then
+    // leave two waves to a SIMD, only with several token tiles (2048 x 11008, 64 tokens: 31.6 against 37.0; 151936 x
+    // 2048, 8 tokens: 104 against 84)
+    const long tiles = (n_rows + 15) / 16 * ((g.n_tok + 15) / 16);
+    if (m->type == SDY_Q6_K)
+        return g.n_tok > 16 && tiles >= 512 ? launch_sb<SDY_Q6_K, 2, EXP>(g, st) : launch_sb<SDY_Q6_K, 1, EXP>(g, st);
+    return tiles > 512 ? launch_sb<SDY_Q4_K, 2, EXP>(g, st) : launch_sb<SDY_Q4_K, 1, EXP>(g, st);
+}
+
+}  // namespace
+
+// The tokens of a->xq through rows [a->row0, a->row1) of m (Q4_K, Q6_K), with the bits of sdy_matvec. Returns 1,
+// launching nothing, when the kernel's 32-bit offsets do not reach every byte of the matrix or the activations.
+extern "C" int sdy_mm_superblocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s) {
+    return run_sb<false>(m, a, nullptr, (hipStream_t)s);
+}
+
+// The same from the GEMM's expansion of the activations.
+int sdy_mm_superblocks_exp(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, sdy_stream s) {
+    return run_sb<true>(m, a, e, (hipStream_t)s);
 }

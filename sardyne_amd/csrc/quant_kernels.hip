@@ -279,7 +279,7 @@ __global__ void k_dequant_float(const uint8_t *__restrict__ w, int n_in, const i
 // ------------------------------------------------------------------------ activation quantisers
 
 // Q8_K (csrc/quant.c:118-144): one wave per 256-element block (four blocks of a row per 256-thread
-// workgroup), lane l holds elements 4l..4l+3. With e.y16 set, also the GEMM's expansion of the block.
+// workgroup), lane l holds elements 4l..4l+3. With e.y8 set, also the GEMM's expansion of the block.
 __global__ __launch_bounds__(256) void k_quant_q8k(const float *__restrict__ x, uint8_t *__restrict__ out, int n_in,
                                                    SdyGemmExp e) {
     const int nb = n_in / 256, s = blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y, l = threadIdx.x & 63;
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) void k_quant_q8k(const float *__restrict__ x, 
     *reinterpret_cast<uint32_t *>(ob + 4 + 4 * l) = r.packed;
     if ((l & 3) == 0) *reinterpret_cast<int16_t *>(ob + 260 + 2 * (l >> 2)) = (int16_t)r.gsum;
     if (l == 0) *reinterpret_cast<float *>(ob) = r.d;
-    if (e.y16) e.put(r, l, (size_t)t * nb + s);
+    if (e.y8) e.put(r, l, (size_t)t * nb + s);
 }
 
 // Q8_0 (csrc/quant.c:98-108): one wave per two 32-element blocks, one element per lane.
@@ -2041,8 +2041,7 @@ static int mat_alloc(sdy_mat *m, int type, int n_in, long n_rows, bool host) {
         if (pb[i]) off += align256(pb[i] * (size_t)n_rows);
     }
     // zero rows pass the GEMM check, so a matrix filled in several uploads is checked piecewise. A
-    // matrix in host memory is not checked (the check's reads would cross the host link) and takes
-    // the GEMM's wide variant, exact for every block
+    // matrix in host memory is not checked (the check's reads would cross the host link)
     m->gemm_ok = type == SDY_Q4_K || type == SDY_Q6_K ? (host ? 2 : 1) : 0;
     // (zeroed by the GPU for host memory too: its pages are mapped to the device at allocation, and the
     // CPU's first touch of each would fault. Completed before returning: the uploads run on other,

@@ -55,7 +55,7 @@ struct engine_ctx {
     const float *xq_src[2];
     int xq_n_tok[2], xq_n_in[2];
     unsigned xq_epoch;          /* bumped at every write of xq[] */
-    int gemm_ready;             /* gemm_ws holds the f16 expansion of gemm_xq made in epoch gemm_epoch */
+    int gemm_ready;             /* gemm_ws holds the expansion of gemm_xq made in epoch gemm_epoch */
     unsigned gemm_epoch;
     const void *gemm_xq;
     int gemm_n_tok, gemm_n_in;

@@ -64,8 +64,8 @@ typedef struct {
     long n_rows;    /* rows (experts stacked: n_expert * n_out) */
     int n_units;    /* 64-element units per row (quantized types) */
     size_t plane_off[5];
-    int gemm_ok;    /* Q4_K / Q6_K: 1 when the GEMM's one-fragment scheme is exact for every block,
-                       2 when some block needs the wide variant (Q6_K: twice the MFMA work); 0 other types */
+    int gemm_ok;    /* Q4_K / Q6_K: 1, or 2 when some block's |sc * q| exceed what real files hold (2^24 / 127 in a
+                       super-block; Q6_K 2048 in an element); the GEMM is exact for either. 0 other types */
     void *gbase;    /* the many-token kernels' copy of the planes (sdy_mat_gemm_layout) or NULL: rows in tiles of 32,
                        each tile's records unit-major ([tile][unit][32 rows][16 bytes], the per-super-block
                        records [tile][super-block][32 rows]) */
@@ -148,7 +148,7 @@ typedef struct {
                             row of x itself, RMS-normalised first when nw is set (x / rms(x) * nw, eps), with
                             the bytes sdy_quantize / sdy_norm_quant would write; see sdy_matvec_fused_ok */
     float eps;
-    int ws_ready;        /* sdy_gemm: ws already holds this xq's f16 expansion (same n_tok and n_in), written by
+    int ws_ready;        /* sdy_gemm: ws already holds this xq's expansion (same n_tok and n_in), written by
                             the previous sdy_gemm on ws with nothing written to xq or ws since: it is not
                             expanded again */
 } sdy_mv_args;
@@ -200,7 +200,7 @@ int sdy_gemm(const sdy_mat *m, const sdy_mv_args *a, void *ws, sdy_stream s);
 int sdy_gemm2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat *m2, const sdy_mv_args *a2, void *ws,
               sdy_stream s);
 /* Q8_K activations for the GEMM in one launch: the bytes of sdy_quantize (of sdy_norm_quant, with xb
- * as there) into xq, and their f16 expansion into ws, so that sdy_gemm on the same rows and ws runs
+ * as there) into xq, and their expansion (the values, scales and sums in planes) into ws, so that sdy_gemm on the same rows and ws runs
  * with ws_ready = 1. */
 int sdy_quantize_gemm(const float *x, void *xq, int n_in, int n_tok, void *ws, sdy_stream s);
 int sdy_norm_quant_gemm(const float *x, const float *w, float eps, int n, int n_rows, float *xb, void *xq, void *ws,
@@ -216,8 +216,7 @@ int sdy_gemm_grouped_tile(void);
 int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, const int *grp_tok, const int *grp_tile,
                      const int *out_row, const int *act_row, int n_act, const sdy_mv_args *a, void *ws,
                      sdy_stream s);
-/* Variant check of rows [r0, r0 + n) of m for the GEMM: *bad_host = 1 when some row has a block
- * that only the wide variant multiplies exactly. */
+/* The gemm_ok check of rows [r0, r0 + n) of m: *bad_host = 1 when some row has a block of gemm_ok 2. */
 int sdy_gemm_check_rows(const sdy_mat *m, long r0, long n, int *bad_host, sdy_stream s);
 /* The same, queued on s: sets *bad_dev (device int, zero beforehand) to nonzero for such a row */
 int sdy_gemm_check_rows_async(const sdy_mat *m, long r0, long n, int *bad_dev, sdy_stream s);

@@ -1502,6 +1502,33 @@ def test_superblock_mfma_few_tokens(kind, n_in, n_out, n_tok):
     assert np.array_equal(bits(run(tiled, 0, even, capi.EPI_SWIGLU)), bits(gate))
 
 
+@pytest.mark.parametrize("kind,n_in,n_out,n_tok,kernel", [
+    ("Q4_K", 256, 5120, 32, "k_mm_superblocks"), ("Q4_K", 2304, 5121, 32, "k_gemm"), ("Q4_K", 512, 8161, 33, "k_gemm"),
+    ("Q4_K", 256, 16417, 97, "k_gemm"), ("Q6_K", 2304, 2048, 63, "k_mm_superblocks"),
+    ("Q6_K", 256, 16384, 16, "k_mm_superblocks"), ("Q6_K", 768, 16385, 16, "k_gemm"), ("Q6_K", 1280, 700, 250, "k_gemm"),
+    ("Q6_K", 512, 65505, 18, "k_gemm")])
+def test_gemm_forms_bit_exact(kind, n_in, n_out, n_tok, kernel):
+    """Both sides of the lines between the GEMM's forms (super-blocks split over 8, 4, 2 or 1 waves) with partial tiles,
+    scales and quants over their whole range, a token of one sign and one whose scale products are subnormal: the
+    oracle's bits, from the tiled copy and the planes."""
+    t = TYPES[kind]
+    w = _full_range_blocks(kind, n_out, n_in, n_in + n_tok)
+    x = np.random.default_rng(n_tok).standard_normal((n_tok, n_in)).astype(np.float32)
+    x[0] = np.abs(x[0])
+    x[1] *= np.float32(1e-36)
+    xq = O.quantize(x, O.Q8_K)
+    exp = O.matmul_q(w, t, xq, n_in, simd=1)
+    assert np.array_equal(bits(_gemm_run(t, w, xq, n_in, n_out, n_tok)), bits(exp))
+    assert lib().sdy_last_kernel().decode().split("<")[0].endswith(kernel)
+    L = lib()
+    m = capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=False)
+    dq, out = capi.DeviceBuffer.from_array(xq), capi.DeviceBuffer(n_tok * n_out * 4)
+    ws = capi.DeviceBuffer(L.sdy_gemm_ws_bytes(n_tok, n_in))
+    a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out, row0=0, row1=n_out)
+    capi.check(L.sdy_gemm(ctypes.byref(m.m), ctypes.byref(a), ws.ptr, None))
+    assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out))), bits(exp))
+
+
 @pytest.mark.parametrize("variant", ["11", "12", "13", "14", "15", "16", "17", "18", "19", "20"])
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 def test_gemm_tile_variants_bit_exact(kind, variant, monkeypatch):
