@@ -1071,6 +1071,35 @@ def test_prefill_attention_flash(n_head, n_kv_head, hd, n_tok, n_kv0, kv):
     np.testing.assert_allclose(outs[0], exp, rtol=0, atol=1e-5 * float(np.abs(exp).max()))
 
 
+@pytest.mark.parametrize("hd,n_tok,n_kv0", [(128, 33, 1), (64, 70, 40)])
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+def test_prefill_attention_flash_extremes(hd, n_tok, n_kv0, kv):
+    """An infinite K element under a negative query component (a score of -inf, no weight), V at the type's largest
+    value, and queries of very different sizes: the reference's arithmetic to 1e-5 of each output column's scale, the
+    bound of the ordinary values."""
+    L = lib()
+    n_head, n_kv_head, max_seq = 4, 2, n_kv0 + n_tok + 3
+    rng = np.random.default_rng(hd + n_tok)
+    q = rng.standard_normal((n_tok, n_head * hd)).astype(np.float32)
+    q *= (2.0 ** rng.integers(-20, 2, (n_tok, 1))).astype(np.float32)
+    ct = np.float16 if kv == "f16" else np.float32
+    kc, vc = (rng.standard_normal((n_kv_head, max_seq, hd)).astype(ct) for _ in range(2))
+    kc[0, n_kv0 // 2 + 2, 3] = np.inf
+    q[:, 3] = q[:, hd + 3] = -1.0
+    vc[1, 0, 1] = np.finfo(ct).max
+    kv_type = capi.KV_F16 if kv == "f16" else capi.KV_F32
+    dq, dk, dv = (capi.DeviceBuffer.from_array(a) for a in (q, kc, vc))
+    dpart = capi.DeviceBuffer(L.sdy_attn_scores_floats(n_tok, n_head, max_seq) * 4)
+    outs = [capi.DeviceBuffer(q.nbytes) for _ in range(2)]
+    capi.check(L.sdy_attention(dq.ptr, dk.ptr, dv.ptr, kv_type, n_tok, n_head, n_kv_head, hd, n_kv0, max_seq * hd,
+                               n_head * hd, dpart.ptr, outs[0].ptr, n_head * hd, None))
+    capi.check(L.sdy_attention_flash(dq.ptr, dk.ptr, dv.ptr, kv_type, n_tok, n_head, n_kv_head, hd, n_kv0, max_seq * hd,
+                                     n_head * hd, outs[1].ptr, n_head * hd, None))
+    exp, got = (o.to_array(np.float32, q.shape) for o in outs)
+    assert np.all(np.isfinite(exp))
+    assert np.all(np.abs(got - exp) <= 1e-5 * np.abs(exp).max(axis=0))
+
+
 def test_prefill_attention_flash_rejects_layouts():
     """head_dim other than 64 / 128, GQA groups that do not divide, unaligned q rows: an error, no launch."""
     L = lib()
