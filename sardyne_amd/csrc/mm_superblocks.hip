@@ -6,8 +6,8 @@
 // the offset 32 of the quants (Q6_K) come from one f16 matrix instruction against the activations' 16-element
 // sums (exact integers below 2^24), and the f32 combine is the matvec's, super-blocks in order.
 //
-// Each wave takes one super-block of 16 MT rows and requests all it needs of it at once; the eight waves of a
-// workgroup take eight super-blocks side by side and hand their terms through LDS to the threads that add them in
+// Each wave takes one super-block of 16 MT rows and requests all it needs of it at once; the eight (or four) waves of a
+// workgroup take as many super-blocks side by side and hand their terms through LDS to the threads that add them in
 // order. What bounds it: the weights' stream and its latency; the VALU work of a super-block is about 115
 // instructions per 16 rows whatever the tokens, up to 16, where the 8-token matvec spends 245 per token and 64 units.
 // 22016 x 2048 Q4_K (25 MB), 8 tokens, with the quantiser's launch: 33.5 -> 11.2 us; 2048 x 2048 13.0 -> 7.6; Q6_K 2048 x
@@ -53,9 +53,8 @@ SDY_DEV long as_long(u32x2 v) { return __builtin_bit_cast(long, v); }
 // sub-blocks at once, in three instructions).
 SDY_DEV void opaque(i32x4 &v) { __asm__ volatile("" : "+v"(v)); }
 
-constexpr int KS = 8;  // waves, super-blocks of a round
-
-template <int WT, int MT, bool EXP>
+// KS: waves, super-blocks of a round
+template <int WT, int MT, int KS, bool EXP>
 __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     constexpr bool Q4 = WT == SDY_Q4_K;
     constexpr int OUT = MT * 256, NTH = 64 * KS;  // outputs of the workgroup, threads
@@ -203,11 +202,11 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     for (int j = 0; j < NO; j++) acc[j] = 0.0f;
     Regs R[2];
     const int nr = (nb + KS - 1) / KS;
-    auto sb_of = [&](int rd) { return rd * KS + wave < nb ? rd * KS + wave : nb - 1; };  // (past the end: not added)
-    load(sb_of(0), R[0]);
+    auto has = [&](int rd) { return rd * KS + wave < nb; };  // (waves past the last super-block only add)
+    if (has(0)) load(wave, R[0]);
     auto round = [&](int rd, const Regs &cur, Regs &nxt, int z) {
-        if (rd + 1 < nr) load(sb_of(rd + 1), nxt);
-        compute(cur, &terms[z][wave][0]);
+        if (has(rd + 1)) load((rd + 1) * KS + wave, nxt);
+        if (has(rd)) compute(cur, &terms[z][wave][0]);
         __syncthreads();  // (a buffer is written again two rounds on, past the next round's barrier)
         const int left = nb - rd * KS;
 #pragma unroll
@@ -247,12 +246,19 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
     }
 }
 
-template <int WT, int MT, bool EXP>
-int launch_sb(const SbArgs &g, hipStream_t st) {
-    SDY_NOTE_KERNEL((k_mm_superblocks<WT, MT, EXP>));
-    hipLaunchKernelGGL((k_mm_superblocks<WT, MT, EXP>),
+template <int WT, int MT, int KS, bool EXP>
+int launch_ks(const SbArgs &g, hipStream_t st) {
+    SDY_NOTE_KERNEL((k_mm_superblocks<WT, MT, KS, EXP>));
+    hipLaunchKernelGGL((k_mm_superblocks<WT, MT, KS, EXP>),
                        dim3((unsigned)((g.n_tok + 15) / 16), (unsigned)((g.n_rows + 16 * MT - 1) / (16 * MT))), dim3(64 * KS), 0, st, g);
     return sdy_check_launch("matvec (super-block MFMA)");
+}
+
+// Four waves to a workgroup where rows have no more super-blocks: with eight, half of them held their places for nothing
+// (1024 x 33786 Q4_K, 3 tokens: 12.9 us, where the 8-token matvec took 12.6; now 10.9)
+template <int WT, int MT, bool EXP>
+int launch_sb(const SbArgs &g, hipStream_t st) {
+    return g.nb <= 4 ? launch_ks<WT, MT, 4, EXP>(g, st) : launch_ks<WT, MT, 8, EXP>(g, st);
 }
 
 template <bool EXP>
