@@ -1939,6 +1939,178 @@ __global__ __launch_bounds__(256) void k_matvec_float_tile(const uint8_t *__rest
         }
 }
 
+// The same for larger grids on the matrix cores: v_mfma_f32_16x16x1_4b_f32 adds one f32 product, fused, to each of 4 x
+// 16 x 16 sums, so two waves carry the eight chains of 16 rows x 16 tokens (an instruction per 8-element step and
+// four chains), a workgroup's eight waves 32 x 32, with the bits of k_matvec_float_block. The chains' ends are added as
+// hsum adds the lanes: v + (v + 4), then the four sums, in the registers of the first chains' wave. The rows and
+// tokens are staged in LDS as f32, FM_K elements at a time in two buffers, two chunks requested ahead into registers;
+// at a pitch of FM_K + 4 floats 16-byte writes are aligned and a read's 64 lanes fall on 64 banks.
+// What bounds it: the f32 matrix instructions' 32 cycles per step and wave, and the LDS and VALU work, which hardly runs
+// beside them (1 024 cycles of 2 200 per chunk). F16 2048 x 2048: 128 tokens 31.66 -> 15.42 us (1.07 GFLOP: 6.8 us at the f32
+// matrix rate), 512 tokens 114 -> 60; 11008 x 2048, 203 tokens 262 -> 150. 32x32x1_2b tiles (half the LDS reads, with
+// conflicts): 20.2 us for the first; the staging not spread between the matrix instructions: 23.
+typedef float fm_f32x16 __attribute__((ext_vector_type(16)));
+constexpr int FM_ROWS = 32, FM_TOKS = 32, FM_K = 128, FM_P = FM_K + 4, FM_H = FM_K / 16, FM_TH = 512;
+constexpr size_t FM_LDS = 2 * (FM_ROWS + FM_TOKS) * FM_P * sizeof(float);
+
+template <int WT>
+__global__ __launch_bounds__(FM_TH, 4) void k_matvec_float_mfma(const uint8_t *__restrict__ w, int n_in,
+                                                             const float *__restrict__ x, int n_tok, float *out,
+                                                             long out_stride, const float *bias, const float *resid,
+                                                             long row0, long row1) {
+    constexpr int NV = FM_ROWS * FM_K / FM_TH / 4;  // 4-element loads per thread of a chunk's rows, and of its tokens
+    extern __shared__ __align__(16) float fm_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ch = wave & 1, wr = 16 * (wave >> 2), wt = 16 * (wave >> 1 & 1);
+    const long n_pr = (row1 - row0) & ~1L;
+    const int n_gt = n_tok & ~3, n8 = n_in & ~7;
+    const long r_tile = (long)blockIdx.y * FM_ROWS;
+    const int t_tile = blockIdx.x * FM_TOKS;
+    // the thread's loads: elements 4 (tid % 32) .. of rows (tokens) tid / 32 + 16 u, clamped to the last
+    const int e = 4 * (tid & 31), r0 = tid >> 5;
+    size_t wo[NV], xo[NV];
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+        const long r = r_tile + r0 + 16 * u;
+        const int t = t_tile + r0 + 16 * u;
+        wo[u] = (size_t)(row0 + (r < n_pr ? r : n_pr - 1)) * n_in;
+        xo[u] = (size_t)(t < n_gt ? t : n_gt - 1) * n_in;
+    }
+    struct Chunk {
+        ft_f32x4 x[NV], wf[WT == SDY_F32 ? NV : 1];
+        uint2 wh[WT == SDY_F32 ? 1 : NV];
+    };
+    const int nc = (n8 + FM_K - 1) / FM_K;
+    // (past the last chunk it is repeated, and past n8 its first elements: not used)
+    auto chunk_el = [&](int c) {
+        const int k0 = (c < nc ? c : nc - 1) * FM_K;
+        return k0 + (e < n8 - k0 ? e : 0);
+    };
+    auto fetch_u = [&](int el, Chunk &k, int u) {
+        if constexpr (WT == SDY_F32) k.wf[u] = *reinterpret_cast<const ft_f32x4 *>(reinterpret_cast<const float *>(w) + wo[u] + el);
+        else k.wh[u] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint16_t *>(w) + wo[u] + el);
+        k.x[u] = *reinterpret_cast<const ft_f32x4 *>(x + xo[u] + el);
+    };
+    auto fetch = [&](int c, Chunk &k) {
+#pragma unroll
+        for (int u = 0; u < NV; u++) fetch_u(chunk_el(c), k, u);
+    };
+    auto stage_u = [&](const Chunk &k, float *buf, int u) {
+        float *d = buf + (r0 + 16 * u) * FM_P + e;
+        ft_f32x4 v;
+        if constexpr (WT == SDY_F32) {
+            v = k.wf[u];
+        } else {
+            const uint32_t q[2] = {k.wh[u].x, k.wh[u].y};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const uint16_t hv = (uint16_t)(q[c >> 1] >> (16 * (c & 1)));
+                v[c] = WT == SDY_F16 ? sdy_h2f(hv) : __uint_as_float((uint32_t)hv << 16);
+            }
+        }
+        *reinterpret_cast<ft_f32x4 *>(d) = v;
+        *reinterpret_cast<ft_f32x4 *>(d + FM_ROWS * FM_P) = k.x[u];
+    };
+    auto stage = [&](const Chunk &k, float *buf) {
+#pragma unroll
+        for (int u = 0; u < NV; u++) stage_u(k, buf, u);
+    };
+    // the lane's operands of FM_H steps (half a chunk): elements 8 s + 4 ch + g (chain 4 ch + g) of its row and token
+    struct Ops {
+        float w[FM_H], x[FM_H];
+    };
+    const int wat = (wr + l16) * FM_P + 4 * ch + g, xat = (FM_ROWS + wt + l16) * FM_P + 4 * ch + g;
+    auto read_s = [&](const float *buf, Ops &o, int s) {
+        o.w[s] = buf[wat + 8 * s];
+        o.x[s] = buf[xat + 8 * s];
+    };
+    auto read = [&](const float *buf, Ops &o) {
+#pragma unroll
+        for (int s = 0; s < FM_H; s++) read_s(buf, o, s);
+    };
+    fm_f32x16 acc = {};  // chain 4 ch + b: registers 4 b .. 4 b + 3
+    auto mul_s = [&](const Ops &o, int s) { acc = __builtin_amdgcn_mfma_f32_16x16x1f32(o.x[s], o.w[s], acc, 0, 0, 0); };
+    auto mul = [&](const Ops &o, int ns) {
+#pragma unroll
+        for (int s = 0; s < FM_H; s++)
+            if (s < ns) mul_s(o, s);
+    };
+    // orders LDS only: the chunks in flight stay in flight
+    auto barrier = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    float *b0 = fm_lds, *b1 = fm_lds + (FM_ROWS + FM_TOKS) * FM_P;
+    if (nc > 0) {
+        Chunk k0, k1;
+        Ops o0, o1;
+        // Chunk c, its first half in o0: the second is read and chunk c + 1 staged (into the buffer of c - 1, which
+        // every wave has read before the last barrier) while the first is multiplied; c + 2 and c + 3 are in flight.
+        // A step's matrix instructions go out before each piece of the other work, which then runs beside them (a wave
+        // issues in order, and it is alone on its SIMD where the grid is small).
+        static_assert(FM_H >= 2 * NV, "a piece of staging or fetching per step");
+        auto step = [&](int c, const float *bc, float *bn, Chunk &k) {
+            const int el = chunk_el(c + 3);
+#pragma unroll
+            for (int s = 0; s < FM_H; s++) {
+                mul_s(o0, s);
+                __builtin_amdgcn_sched_barrier(0);
+                read_s(bc + FM_K / 2, o1, s);
+                if (s < NV) stage_u(k, bn, s);
+                else if (s < 2 * NV) fetch_u(el, k, s - NV);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            barrier();
+#pragma unroll
+            for (int s = 0; s < FM_H; s++) {
+                mul_s(o1, s);
+                __builtin_amdgcn_sched_barrier(0);
+                read_s(bn, o0, s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        const int nf = n8 / FM_K, left = (n8 - nf * FM_K) >> 3;  // whole chunks, the last one's steps
+        fetch(0, k0);
+        fetch(1, k1);
+        stage(k0, b0);
+        fetch(2, k0);
+        barrier();
+        read(b0, o0);
+        int c = 0;
+        for (; c + 2 <= nf; c += 2) {
+            step(c, b0, b1, k1);
+            step(c + 1, b1, b0, k0);
+        }
+        if (c < nf) step(c, b0, b1, k1);
+        read((nf & 1 ? b1 : b0) + FM_K / 2, o1);
+        mul(o0, left);
+        mul(o1, left - FM_H);
+    }
+    // register 4 b + i: chain 4 ch + b of token 4 g + i, row l16. The second four chains go through LDS to the first's wave
+    __syncthreads();
+    float *xch = fm_lds + (wave >> 1) * (16 * 64) + lane;
+    if (ch) {
+#pragma unroll
+        for (int f = 0; f < 16; f++) xch[f * 64] = acc[f];
+    }
+    __syncthreads();
+    if (ch) return;
+    const long r = r_tile + wr + l16;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int t = t_tile + wt + 4 * g + i;
+        float v[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) v[b] = acc[4 * b + i] + xch[(4 * b + i) * 64];
+        if (r < n_pr && t < n_gt) {
+            const uint8_t *wrow = w + (size_t)(row0 + r) * n_in * (WT == SDY_F32 ? 4 : 2);
+            float_store<WT>(float_tail<WT>(wrow, x + (size_t)t * n_in, n_in, (v[0] + v[2]) + (v[1] + v[3])), row0 + r, t,
+                            out, out_stride, bias, resid);
+        }
+    }
+}
+
 }  // namespace
 
 // =============================================================================== host launchers
@@ -2999,6 +3171,16 @@ extern "C" int sdy_matvec_float_norm(int wtype, const void *w, int n_in, const s
     return sdy_check_launch("matvec_float_norm");
 }
 
+template <int WT>
+static int launch_float_mfma(const uint8_t *w, int n_in, const sdy_mv_args *a, long n_pr, int n_gt, hipStream_t st) {
+    static size_t granted = 0;
+    if (int rc = sdy_lds_limit((const void *)k_matvec_float_mfma<WT>, FM_LDS, &granted)) return rc;
+    const dim3 grid((unsigned)((n_gt + FM_TOKS - 1) / FM_TOKS), (unsigned)((n_pr + FM_ROWS - 1) / FM_ROWS));
+    hipLaunchKernelGGL(k_matvec_float_mfma<WT>, grid, dim3(FM_TH), FM_LDS, st, w, n_in, a->x, a->n_tok, a->out,
+                       a->out_stride, a->bias, a->resid, a->row0, a->row1);
+    return sdy_check_launch("matvec_float (tile)");
+}
+
 extern "C" int sdy_matvec_float(int wtype, const void *w, int n_in, const sdy_mv_args *a, sdy_stream s) {
     hipStream_t st = (hipStream_t)s;
     const long n_rows = a->row1 - a->row0;
@@ -3022,8 +3204,16 @@ extern "C" int sdy_matvec_float(int wtype, const void *w, int n_in, const sdy_mv
             hipLaunchKernelGGL(KERNEL<SDY_BF16>, grid, dim3(THREADS), 0, st, wp, n_in, a->x, n_tok, a->out,           \
                                a->out_stride, a->bias, a->resid, a->row0, a->row1);                                  \
     }
-    if (n_pr >= FT_ROWS && n_gt >= FT_TOKS && n_in % 4 == 0 && ((uintptr_t)wp & 15) == 0 &&
-        ((uintptr_t)a->x & 15) == 0) {
+    const bool aligned = n_in % 4 == 0 && ((uintptr_t)wp & 15) == 0 && ((uintptr_t)a->x & 15) == 0;
+    if (aligned && n_pr >= 16 && n_gt >= 16 &&
+        ((n_pr + FM_ROWS - 1) / FM_ROWS) * ((n_gt + FM_TOKS - 1) / FM_TOKS) >= 64) {
+        // the matrix cores, from 64 tiles of 32 x 32 (2048 x 2048 F16, 16 tokens: 15.9 us against 16.2 on the 16 x 16
+        // tiles below; 64 tokens 16.8 against 21.8; the F32 router of 128 rows, 301 tokens, 40 tiles: 18.4 against 17.5)
+        const int rc = wtype == SDY_F32 ? launch_float_mfma<SDY_F32>(wp, n_in, a, n_pr, n_gt, st)
+                       : wtype == SDY_F16 ? launch_float_mfma<SDY_F16>(wp, n_in, a, n_pr, n_gt, st)
+                                          : launch_float_mfma<SDY_BF16>(wp, n_in, a, n_pr, n_gt, st);
+        if (rc) return rc;
+    } else if (aligned && n_pr >= FT_ROWS && n_gt >= FT_TOKS) {
         // many rows and tokens: the block-order pairs from tiles staged in LDS (4-element loads)
         const dim3 grid((unsigned)((n_gt + FT_TOKS - 1) / FT_TOKS), (unsigned)((n_pr + FT_ROWS - 1) / FT_ROWS));
         const dim3 block(256);

@@ -938,6 +938,35 @@ def test_float_matmul_reference_order_bit_exact(wtype, n_in, n_out, n_tok, r0, r
     assert np.array_equal(bits(got[:, r0:r1]), bits(exp[:, r0:r1]))
 
 
+@pytest.mark.parametrize("wtype", [O.F32, O.F16, O.BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("n_in,n_out,n_tok", [(4, 2050, 17), (12, 301, 250), (136, 16, 2047), (132, 1001, 67), (1028, 2047, 35),
+                                              (268, 2014, 16), (132, 66, 31), (2048, 2048, 128)])
+def test_float_tile_wide_values_bit_exact(wtype, n_in, n_out, n_tok):
+    """The f32 matrix-core tiles (and the smaller grids' VALU tiles) around the edges of the row, token and element
+    tiles, with values from subnormal to large, zeros of both signs and sums that cancel, with bias and residual: the
+    oracle's bits."""
+    rng = np.random.default_rng(n_in + n_out)
+    scale = 2.0 ** rng.integers(-24, 8, (n_out, n_in))
+    w32 = (rng.standard_normal((n_out, n_in)) * scale).astype(np.float32)
+    w32[:, ::5] = np.where(rng.random((n_out, w32[:, ::5].shape[1])) < 0.5, 0.0, -0.0)
+    w32[1::2] = -w32[0::2][:w32[1::2].shape[0]]
+    if wtype == O.F32:
+        w32[:, 1::7] *= np.float32(2.0 ** -125)
+    w = w32.astype(np.float16) if wtype == O.F16 else (w32.view(np.uint32) >> 16).astype(np.uint16) if wtype == O.BF16 else w32
+    w = np.ascontiguousarray(w)
+    x = (rng.standard_normal((n_tok, n_in)) * 2.0 ** rng.integers(-12, 12, (n_tok, n_in))).astype(np.float32)
+    x[0] *= np.float32(2.0 ** -120)
+    bias, resid = rng.standard_normal(n_out).astype(np.float32), rng.standard_normal((n_tok, n_out)).astype(np.float32)
+    dw, dx, db, dr = (capi.DeviceBuffer.from_array(a) for a in (w, x, bias, resid))
+    exp = np.empty((n_tok, n_out), np.float32)
+    O.lib().orc_matmul_rows(ptr(exp), ptr(x), ptr(w), wtype, n_tok, n_in, n_out, 0, n_out, 1)
+    for kw, want in (({}, exp), ({"bias": db.ptr, "resid": dr.ptr}, resid + (exp + bias))):
+        out = capi.DeviceBuffer(n_tok * n_out * 4)
+        a = capi.SdyMvArgs(x=dx.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out, row0=0, row1=n_out, **kw)
+        capi.check(lib().sdy_matvec_float(wtype, dw.ptr, n_in, ctypes.byref(a), None))
+        assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out))), bits(want))
+
+
 @pytest.mark.parametrize("n_expert,k", [(128, 8), (60, 4), (256, 16), (512, 64), (8, 3)])
 def test_moe_route_and_combine(n_expert, k):
     """Router softmax + top-k (ties to the lowest expert) and the weighted sum of the chosen experts'
