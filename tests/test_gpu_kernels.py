@@ -1823,6 +1823,13 @@ def test_decode_attention_chunked(n_head, n_kv_head, hd, qk_norm, interleaved, m
             assert dxq.to_array(np.uint8, n_head * hd // 256 * 292).tobytes() == O.quantize(got, O.Q8_K).tobytes()
 
 
+@pytest.mark.parametrize("n_span", [16, 17, 32, 33, 64, 65, 96, 128])
+def test_decode_attention_chunked_span_counts(n_span):
+    """The merge at the edges of its rounds of 16 spans, of a lane's second span and of the most spans there are, with
+    the tolerance of the other lengths."""
+    test_decode_attention_chunked(8, 2, 64, True, 0, 8192, 64 * n_span - 1, "f16")
+
+
 @pytest.mark.parametrize("n_head,n_kv_head,hd,qk_norm,interleaved",
                          [(16, 2, 128, False, 0), (32, 4, 128, True, 0), (6, 2, 64, False, 1), (4, 4, 64, True, 0),
                           (32, 2, 128, False, 0)],
