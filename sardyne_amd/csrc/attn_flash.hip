@@ -20,7 +20,7 @@
 // form's or less (512 tokens over 1024 cached positions, 32 heads of 128: 3.9e-7 against 4.7e-7): there are fewer
 // sums to round. The queries' fragments sit in LDS; K's and V's are made in registers, 3.5 VALU instructions per
 // element. What bounds it: latency at two waves per SIMD (254 registers), the splits (450 of the tile's 730 VALU
-// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 128 -> 86 us (10.7 GFLOP), f16 138 -> 83;
+// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 128 -> 82 us (10.7 GFLOP), f16 138 -> 83;
 // 301 tokens, 32 heads: 34 -> 24; 77 tokens over 3000 positions, 16 heads, f16: 126 -> 66. The XCD order is 6 us of the
 // first. Two blocks of queries per wave, sharing the splits and the stream: f32 spills (100 us), f16 76, and half the
 // workgroups for the shorter prompts (22 -> 32 us).
