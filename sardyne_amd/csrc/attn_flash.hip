@@ -67,13 +67,13 @@ struct FlashLds {
     static constexpr size_t bytes = 4 * (q_floats > merge_floats ? q_floats : merge_floats);
 };
 
-// Four consecutive elements of a buffer resource at byte offset o + so
+// Four consecutive elements of a buffer resource at byte offset o (zeros past its end)
 template <class KT>
-SDY_DEV sdy_f32x4 ld4_buf(__amdgpu_buffer_rsrc_t r, uint32_t o, int so) {
+SDY_DEV sdy_f32x4 ld4_buf(__amdgpu_buffer_rsrc_t r, uint32_t o) {
     if constexpr (std::is_same<KT, float>::value) {
-        return __builtin_bit_cast(sdy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o, so, 0));
+        return __builtin_bit_cast(sdy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0));
     } else {
-        const auto u = __builtin_amdgcn_raw_buffer_load_b64(r, o, so, 0);
+        const auto u = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0);
         return sdy_f32x4{sdy_h2f((uint16_t)(u[0] & 0xFFFFu)), sdy_h2f((uint16_t)((uint32_t)u[0] >> 16)),
                          sdy_h2f((uint16_t)(u[1] & 0xFFFFu)), sdy_h2f((uint16_t)((uint32_t)u[1] >> 16))};
     }
@@ -85,18 +85,18 @@ struct VLoad;
 template <class KT>
 struct VLoad<4, KT> {
     using T = sdy_f32x4;
-    SDY_DEV static T ld(__amdgpu_buffer_rsrc_t r, uint32_t o, int so) { return ld4_buf<KT>(r, o, so); }
+    SDY_DEV static T ld(__amdgpu_buffer_rsrc_t r, uint32_t o) { return ld4_buf<KT>(r, o); }
     SDY_DEV static float at(const T &v, int j) { return v[j]; }
 };
 template <class KT>
 struct VLoad<2, KT> {
     using T = float2;
-    SDY_DEV static T ld(__amdgpu_buffer_rsrc_t r, uint32_t o, int so) {
+    SDY_DEV static T ld(__amdgpu_buffer_rsrc_t r, uint32_t o) {
         if constexpr (std::is_same<KT, float>::value) {
-            const auto u = __builtin_amdgcn_raw_buffer_load_b64(r, o, so, 0);
+            const auto u = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0);
             return make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]));
         } else {
-            const uint32_t u = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, o, so, 0);
+            const uint32_t u = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0);
             return make_float2(sdy_h2f((uint16_t)(u & 0xFFFFu)), sdy_h2f((uint16_t)(u >> 16)));
         }
     }
@@ -204,17 +204,21 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
         const int k0 = kt * KB;
         // K: lane (key ql of the tile, dims hh * HH ...); V of the PV step r: key
         // 8 (r / 4) + 4 hh + r % 4 of the tile (the key of the lane's score register r), dims
-        // ND * ql ... Positions past the block's last one read as zeros (the resource ends there) and are masked below
-        const uint32_t left = (uint32_t)(n_kv_max - k0 < KB ? n_kv_max - k0 : KB) * RB;
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void *)(kb + (size_t)k0 * HD), (short)0, (int)left, 0x00020000),
-                                     rv = __builtin_amdgcn_make_buffer_rsrc((void *)(vb + (size_t)k0 * HD), (short)0, (int)left, 0x00020000);
+        // ND * ql ... Positions past the block's last one read as zeros (the resource ends there) and are masked below.
+        // A scalar offset is left out of the resource's bound, so each 8 V rows have a resource of their own.
+        const int rows = n_kv_max - k0 < KB ? n_kv_max - k0 : KB;
+        auto rows_from = [&](const KT *base, int r) {
+            return __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)(k0 + r) * HD), (short)0,
+                                                     (rows > r ? rows - r : 0) * (int)RB, 0x00020000);
+        };
+        const __amdgpu_buffer_rsrc_t rk = rows_from(kb, 0), rv[4] = {rows_from(vb, 0), rows_from(vb, 8), rows_from(vb, 16), rows_from(vb, 24)};
         sdy_f32x4 kv[HH / 4];
 #pragma unroll
-        for (int i = 0; i < HH / 4; i++) kv[i] = ld4_buf<KT>(rk, vk + 4 * i * (uint32_t)sizeof(KT), 0);
+        for (int i = 0; i < HH / 4; i++) kv[i] = ld4_buf<KT>(rk, vk + 4 * i * (uint32_t)sizeof(KT));
         typename VL::T vv[16];
         auto load_v = [&]() {
 #pragma unroll
-            for (int r = 0; r < 16; r++) vv[r] = VL::ld(rv, vo + (r & 3) * RB, 8 * (r >> 2) * (int)RB);
+            for (int r = 0; r < 16; r++) vv[r] = VL::ld(rv[r >> 2], vo + (r & 3) * RB);
         };
         if constexpr (SPLIT) load_v();
         // S^T[key][query] = sum over dims of K[key][d] Q[query][d]: step (i, j) pairs dim 4i + j

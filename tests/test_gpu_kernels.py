@@ -1129,6 +1129,32 @@ def test_prefill_attention_flash_extremes(hd, n_tok, n_kv0, kv):
     assert np.all(np.abs(got - exp) <= 1e-5 * np.abs(exp).max(axis=0))
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("tail", [1, 7, 8, 9, 17, 25, 32])
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+def test_prefill_attention_flash_reads_no_row_past_the_last(hd, tail, kv):
+    """`tail` positions in the last tile of 32 keys, the cache's later rows (and the second head's, up to the end of
+    the allocation) NaN: the bits of the same call with zeros there, in an early block of queries and in the last."""
+    L = lib()
+    n_head, n_kv_head, n_tok = 4, 2, 40
+    n_pos = 64 + tail  # positions the last query sees
+    n_kv0, max_seq = n_pos - n_tok + 1, 64 + 32 + 7
+    rng = np.random.default_rng(hd + tail)
+    q = rng.standard_normal((n_tok, n_head * hd)).astype(np.float32)
+    ct = np.float16 if kv == "f16" else np.float32
+    kc, vc = (rng.standard_normal((n_kv_head, max_seq, hd)).astype(ct) for _ in range(2))
+    kv_type = capi.KV_F16 if kv == "f16" else capi.KV_F32
+    dq, got = capi.DeviceBuffer.from_array(q), []
+    for fill in (0.0, np.nan):
+        kc[:, n_pos:] = vc[:, n_pos:] = fill
+        dk, dv, dout = capi.DeviceBuffer.from_array(kc), capi.DeviceBuffer.from_array(vc), capi.DeviceBuffer(q.nbytes)
+        capi.check(L.sdy_attention_flash(dq.ptr, dk.ptr, dv.ptr, kv_type, n_tok, n_head, n_kv_head, hd, n_kv0, max_seq * hd,
+                                         n_head * hd, dout.ptr, n_head * hd, None))
+        got.append(dout.to_array(np.float32, q.shape))
+    assert np.all(np.isfinite(got[0]))
+    assert np.array_equal(bits(got[1]), bits(got[0]))
+
+
 def test_prefill_attention_flash_rejects_layouts():
     """head_dim other than 64 / 128, GQA groups that do not divide, unaligned q rows: an error, no launch."""
     L = lib()
