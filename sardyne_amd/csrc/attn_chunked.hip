@@ -361,22 +361,26 @@ __global__ __launch_bounds__(256) void k_attn_merge(ChunkArgs a) {
     const int h_raw = blockIdx.x * HPS + slot, h = h_raw < a.n_head ? h_raw : a.n_head - 1;
     const int pos = a.step[1];  // (waited for after the loads below)
     const float *pb = a.part + (size_t)h * a.n_span_max * (HD + 4);
-    // The head is uniform over a wave (HD >= 64): lane u holds the m and l of spans u and u + 64, a thread its own
-    // dimension of each span's o, MERGE_ROUND of them requested while the last ones are folded. The first ones are
-    // requested before the position is known: any span's partial is there to be read, and only those below n_span
-    // are used. (Both launches, 16 heads of 128, f16: 72 spans 18.5 -> 17.0 us, 126 spans 22.2 -> 19.3, against rounds of 16
-    // spans each waiting for the last and rescaling)
+    // The head is uniform over a wave (HD >= 64): lane u holds the m and l of spans u and u + 64 (a cache that short has
+    // none), a thread its own dimension of each span's o, MERGE_ROUND of them requested while the last ones are folded.
+    // The first ones are requested before the position is known: any span's partial is there to be read, and only those
+    // below n_span are used. Both launches, 16 heads of 128, f16, against rounds of 16 spans that waited for the position
+    // and for each other: 1 span 9.23 -> 9.21 us, 5 spans (300 positions) 8.70 -> 8.30, 32 spans 10.15 -> 9.22, 71 spans 17.6
+    // -> 15.4. (A second round requested and 128 spans' m and l read whatever the position: 9.74 us for 1 span, 16.1 for 71.)
     const int lane = tid & 63, last = a.n_span_max - 1;
-    float m_s[2], l_s[2], ov[2][MERGE_ROUND];
+    const bool far = last >= 64;
+    float m_s[2] = {}, l_s[2] = {}, ov[2][MERGE_ROUND];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
+        if (k && !far) break;
         const float *pl = pb + (size_t)min(lane + 64 * k, last) * (HD + 4);
         m_s[k] = pl[0];
         l_s[k] = pl[1];
     }
     auto load = [&](int s0, float v[MERGE_ROUND]) {
 #pragma unroll
-        for (int u = 0; u < MERGE_ROUND; u++) v[u] = pb[(size_t)min(s0 + u, last) * (HD + 4) + 4 + d];
+        for (int u = 0; u < MERGE_ROUND; u++)
+            v[u] = pb[(size_t)min(s0 + u, last) * (HD + 4) + 4 + d];
     };
     load(0, ov[0]);
     __builtin_amdgcn_sched_barrier(0);
@@ -397,11 +401,15 @@ __global__ __launch_bounds__(256) void k_attn_merge(ChunkArgs a) {
             if (s0 + u < n_span) o = fmaf(v[u], lane_f(s0 < 64 ? w_s[0] : w_s[1], (s0 + u) & 63), o);
     };
     static_assert(64 % (2 * MERGE_ROUND) == 0 && MAX_SPANS <= 128, "two spans' m and l per lane");
-    for (int s0 = 0; s0 < n_span; s0 += 2 * MERGE_ROUND) {
-        load(s0 + MERGE_ROUND, ov[1]);
-        fold(s0, ov[0]);
-        if (s0 + 2 * MERGE_ROUND < n_span) load(s0 + 2 * MERGE_ROUND, ov[0]);
-        fold(s0 + MERGE_ROUND, ov[1]);
+    if (n_span <= MERGE_ROUND) {
+        fold(0, ov[0]);
+    } else {
+        for (int s0 = 0; s0 < n_span; s0 += 2 * MERGE_ROUND) {
+            load(s0 + MERGE_ROUND, ov[1]);
+            fold(s0, ov[0]);
+            if (s0 + 2 * MERGE_ROUND < n_span) load(s0 + 2 * MERGE_ROUND, ov[0]);
+            fold(s0 + MERGE_ROUND, ov[1]);
+        }
     }
     const float r = o * (1.0f / L);
     if (h_raw < a.n_head) a.out[(size_t)h * HD + d] = r;

@@ -1856,6 +1856,33 @@ def test_decode_attention_chunked_span_counts(n_span):
     test_decode_attention_chunked(8, 2, 64, True, 0, 8192, 64 * n_span - 1, "f16")
 
 
+@pytest.mark.parametrize("max_seq,pos", [(64, 5), (100, 70), (1024, 1023), (1025, 1024), (4096, 20), (4096, 1023), (4096, 1024),
+                                         (4160, 4159), (8192, 63), (8192, 2100)])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_decode_attention_chunked_reads_its_own_partials(max_seq, pos, hd):
+    """The merge requests partials before it knows how many spans there are: whatever the scratch holds behind the
+    position's span (NaN here) the bits are those of a zeroed one, in caches of 1 to 128 spans and on both sides of the
+    first round of 16."""
+    L = lib()
+    n_head, n_kv_head = 4, 2
+    rng = np.random.default_rng(pos + hd)
+    cs, sn = np.empty(max_seq * hd // 2, np.float32), np.empty(max_seq * hd // 2, np.float32)
+    L.op_rope_table(ptr(cs), ptr(sn), max_seq, hd, 1e6)
+    host = dict(q=rng.standard_normal(n_head * hd), k=rng.standard_normal(n_kv_head * hd), v=rng.standard_normal(n_kv_head * hd),
+                kc=rng.standard_normal((n_kv_head, max_seq, hd)), vc=rng.standard_normal((n_kv_head, max_seq, hd)))
+    dev = {n: capi.DeviceBuffer.from_array(a.astype(np.float32)) for n, a in host.items()}
+    dcs, dsn, step = (capi.DeviceBuffer.from_array(a) for a in (cs, sn, np.array([0, pos], np.int32)))
+    n_part, got = L.sdy_attn_chunked_floats(n_head, hd, max_seq), []
+    for fill in (0.0, np.nan):
+        part, out = capi.DeviceBuffer.from_array(np.full(n_part, fill, np.float32)), capi.DeviceBuffer(n_head * hd * 4)
+        capi.check(L.sdy_attn_decode_chunked(dev["q"].ptr, dev["k"].ptr, dev["v"].ptr, None, None, 1e-6, dcs.ptr, dsn.ptr,
+                                             step.ptr, n_head, n_kv_head, hd, 0, dev["kc"].ptr, dev["vc"].ptr, capi.KV_F32,
+                                             max_seq * hd, max_seq, part.ptr, out.ptr, None, None))
+        got.append(out.to_array(np.float32, n_head * hd))
+    assert np.all(np.isfinite(got[0]))
+    assert np.array_equal(bits(got[1]), bits(got[0]))
+
+
 @pytest.mark.parametrize("n_head,n_kv_head,hd,qk_norm,interleaved",
                          [(16, 2, 128, False, 0), (32, 4, 128, True, 0), (6, 2, 64, False, 1), (4, 4, 64, True, 0),
                           (32, 2, 128, False, 0)],
