@@ -2777,27 +2777,40 @@ static int launch_mv(const sdy_mat *m, const sdy_mv_args *a, int n_tok, const ui
     return launch_mv_k<WT, MT, false>(A, lds, st);
 }
 
+// The fewest tokens that mm_superblocks.hip multiplies faster than the matvecs below, which give the same bits. Its time
+// hardly depends on the tokens, but a workgroup's waves take a row's super-blocks eight at a time, each after the last
+// one's loads: few rows of many super-blocks leave that chain alone on the chip. From the tiled copy, without the
+// quantiser's launch: Q4_K is faster from two tokens on (22016 x 2048: 13.7 -> 6.9 us; 2048 x 2048: 5.6 -> 4.2); so is Q6_K up
+// to 4096 rows (4096 x 8192, two tokens: 15.6 -> 10.7) but for some on few rows (1024 x 8192: two tokens 8.8 against 10.5,
+// three 10.7 against 11.0; 512 x 11008: two 11.3 against 13.3, three 14.5 against 13.9). On more rows Q6_K's arithmetic counts:
+// 151936 x 2048 takes 84 us whatever the tokens, the matvecs 57, 74, 85 and 100 for 2, 3, 4 and 5.
+// From the planes a load instruction meets as many cache lines as rows: Q6_K 1024 x 4096, two tokens 6.2 against 9.2, four 9.1
+// against 9.5, five 11.4 against 9.6; 1024 x 8192, six 16.0 against 18.6, eight 19.3 against 19.3; 2048 x 11008, three 18.8
+// against 18.6; Q4_K 1024 x 8192, three 10.4 against 11.7, five 13.8 against 12.1.
+// In host memory the link is what counts, and the matvecs, up to their eight tokens, take whole lines (Q4_K 2048 x 11008, 8
+// tokens: 245 against 302 us).
+static int superblocks_min_tok(const sdy_mat *m, long rows) {
+    const int nb = m->n_in / 256, few = rows <= 1024;
+    if (m->hbase) return 9;
+    if (m->type == SDY_Q4_K) return m->gbase || !few ? 2 : 2 + nb / 16;
+    if (rows > 4096) return 5;
+    if (m->gbase) return few ? 2 + nb / 24 : 2;
+    return 2 + (int)(nb * 144 / (few ? 1024 : rows));
+}
+
 template <int WT>
 static int mv_type(const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
     // Five and more tokens of the 32-element types: the matrix cores (mm_blocks.hip). With 3 or 4 tokens the 4-token
     // matvec below is still the faster one on small matrices (2048 x 2048: 11.1 us against 12.1; the 8-token one takes
-    // 15.2 against 12.3).
+    // 15.2 against 12.3). Several tokens of the K-quants: mm_superblocks.hip.
     if constexpr (!is_k(WT)) {
         if (a->n_tok >= 5) {
             const int rc = sdy_mm_blocks(m, a, (sdy_stream)st);
             if (rc <= 0) return rc;
         }
-    }
-    // Several tokens of the K-quants: the matrix cores too (mm_superblocks.hip), with the same bits. Q4_K from two
-    // tokens (22016 x 2048: 10.7 us against 17.0 with the quantiser's launch; 2048 x 2048: 7.3 against 7.7); Q6_K,
-    // whose super-blocks take the kernel longer, from two on matrices of up to 4096 rows (2048 x 11008: 17.6 against
-    // 18.4) and from five on larger ones (151936 x 2048: 84 us whatever the tokens, against 57, 74, 85 and 100
-    // for 2, 3, 4 and 5).
-    if constexpr (is_k(WT)) {
-        if (a->n_tok >= (WT == SDY_Q4_K || a->row1 - a->row0 <= 4096 ? 2 : 5)) {
-            const int rc = sdy_mm_superblocks(m, a, (sdy_stream)st);
-            if (rc <= 0) return rc;
-        }
+    } else if (a->n_tok >= superblocks_min_tok(m, a->row1 - a->row0)) {
+        const int rc = sdy_mm_superblocks(m, a, (sdy_stream)st);
+        if (rc <= 0) return rc;
     }
     size_t xrow = sdy_raw_row_bytes(is_k(WT) ? SDY_Q8_K : SDY_Q8_0, m->n_in);
     const int T = m->n_units, nb = n_blocks(WT, m->n_in);

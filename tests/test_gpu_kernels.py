@@ -1540,6 +1540,36 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
 
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("n_in,n_out,n_tok,planes,mfma", [
+    (2048, 1024, 2, "Q-", "KK"), (6144, 1024, 2, "--", "K-"), (6144, 1024, 3, "Q-", "KK"), (4096, 300, 2, "--", "KK"),
+    (4096, 1024, 3, "Q-", "KK"), (4096, 300, 4, "QQ", "KK"), (4096, 1025, 3, "Q-", "KK"), (4096, 2049, 2, "Q-", "KK"),
+    (8192, 40, 8, "QQ", "KK"), (1024, 4097, 4, "Q-", "K-"), (1024, 4097, 5, "QQ", "KK"), (256, 40, 8, "QQ", "KK")])
+def test_superblocks_few_tokens_dispatch(kind, n_in, n_out, n_tok, planes, mfma):
+    """Both sides of the lines between the matvecs and the matrix cores (first letter Q4_K, second Q6_K; "-" the matvecs),
+    from the planes, from the tiled copy, and from pinned host memory, which takes the matvecs up to eight tokens: the
+    oracle's bits."""
+    i, t = 0 if kind == "Q4_K" else 1, TYPES[kind]
+    w = _full_range_blocks(kind, n_out, n_in, n_in + n_tok)
+    xq = O.quantize(np.random.default_rng(n_tok).standard_normal((n_tok, n_in)).astype(np.float32), O.Q8_K)
+    exp = O.matmul_q(w, t, xq, n_in, simd=1)
+    L = lib()
+    host = capi.SdyMat()
+    capi.check(L.sdy_mat_alloc_host(ctypes.byref(host), t, n_in, n_out))
+    capi.check(L.sdy_mat_upload_rows(ctypes.byref(host), 0, 1, n_out, w.ctypes.data, None))
+    tiled, plain = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=False)
+    dq = capi.DeviceBuffer.from_array(xq)
+    try:
+        for m, want in ((plain.m, planes[i] != "-"), (tiled.m, mfma[i] != "-"), (host, False)):
+            out = capi.DeviceBuffer(n_tok * n_out * 4)
+            a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out, row0=0, row1=n_out)
+            capi.check(L.sdy_matvec(ctypes.byref(m), ctypes.byref(a), None))
+            assert (b"k_mm_superblocks" in L.sdy_last_kernel()) == want
+            assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out))), bits(exp))
+    finally:
+        L.sdy_mat_free(ctypes.byref(host))
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("n_in,n_out,n_tok", [(256, 3, 2), (2304, 33, 5), (2048, 16, 15), (4096, 130, 16), (11008, 31, 7),
                                               (2048, 8300, 3), (1024, 4200, 6), (768, 70, 33)])
 def test_superblock_mfma_few_tokens(kind, n_in, n_out, n_tok):
