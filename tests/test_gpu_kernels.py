@@ -1480,10 +1480,10 @@ def test_matrix_in_host_memory_same_bits(kind):
 
 
 @pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
-@pytest.mark.parametrize("n_in,n_out,n_tok", [(32, 33, 5), (96, 31, 31), (544, 130, 64), (2048, 129, 33), (2080, 66, 32),
+@pytest.mark.parametrize("n_in,n_out,n_tok", [(32, 33, 8), (96, 31, 31), (544, 130, 64), (2048, 129, 33), (2080, 66, 32),
                                               (4064, 96, 65), (11008, 70, 255), (11008, 200, 256), (2048, 2600, 517)])
 def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
-    """Five and more tokens of the 32-element types (int8 MFMA), around the edges of its row, token and
+    """Eight and more tokens of the 32-element types (int8 MFMA), around the edges of its row, token and
     block tiles and of its wave splits, against float64: the integer dots and the scale products are exact, each
     output is a sum over the row's nb blocks whose longest chain is 8 + nb / 16 + 4 additions, each rounding by
     at most 2^-24 of a partial sum (itself at most the sum of the terms' magnitudes). The tiled copy, the
@@ -1537,6 +1537,42 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
     gate, up = np.ascontiguousarray(got[:, 0:even:2]), np.ascontiguousarray(got[:, 1:even:2])
     L.op_silu_mul(ptr(gate), ptr(up), gate.size)
     assert np.array_equal(bits(run(tiled, dq.ptr, 0, even, capi.EPI_SWIGLU)), bits(gate))
+
+
+@pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
+@pytest.mark.parametrize("n_in,n_out,n_tok,mfma", [
+    (32, 33, 5, False), (2048, 2048, 5, False), (4096, 3072, 5, False), (4096, 3073, 5, True), (2048, 4096, 6, False),
+    (2048, 4097, 6, True), (2048, 2048, 7, False), (2048, 2049, 7, True), (2048, 64, 8, True), (1536, 70, 5, True),
+    (1536, 70, 4, False), (4160, 40, 7, False)])
+def test_block_types_few_tokens(kind, n_in, n_out, n_tok, mfma):
+    """Where the block types change from the matvecs to the matrix cores: the kernel that runs; on the matvecs' side the
+    bits of one token at a time; and either way the same bits from the planes, the tiled copy, pinned host memory and over
+    a row range."""
+    t, w, xq = _matvec_case(kind, n_in, n_out, n_tok, seed=n_in + n_tok)
+    L = lib()
+    host = capi.SdyMat()
+    capi.check(L.sdy_mat_alloc_host(ctypes.byref(host), t, n_in, n_out))
+    capi.check(L.sdy_mat_upload_rows(ctypes.byref(host), 0, 1, n_out, w.ctypes.data, None))
+    tiled, planes = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=False)
+    dq = capi.DeviceBuffer.from_array(xq)
+
+    def run(m, first=0, n=n_tok, r0=0, r1=n_out):
+        out = capi.DeviceBuffer.from_array(np.full((n, n_out), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=dq.ptr + first * (n_in // 32) * 34, n_tok=n, out=out.ptr, out_stride=n_out, row0=r0, row1=r1)
+        capi.check(L.sdy_matvec(ctypes.byref(m), ctypes.byref(a), None))
+        return out.to_array(np.float32, (n, n_out))
+
+    try:
+        got = run(tiled.m)
+        assert (b"k_mm_blocks" in L.sdy_last_kernel()) == mfma
+        for m in (planes.m, host):
+            assert np.array_equal(bits(run(m)), bits(got))
+        assert np.array_equal(bits(run(planes.m, r0=2, r1=n_out - 3)[:, 2:n_out - 3]), bits(got[:, 2:n_out - 3]))
+        if not mfma:
+            for i in range(n_tok):
+                assert np.array_equal(bits(run(tiled.m, i, 1)[0]), bits(got[i]))
+    finally:
+        L.sdy_mat_free(ctypes.byref(host))
 
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
