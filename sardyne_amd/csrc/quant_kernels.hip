@@ -2800,15 +2800,16 @@ static int superblocks_min_tok(const sdy_mat *m, long rows) {
 
 // Whether mm_blocks.hip takes the tokens of a Q8_0 / Q4_0 / Q5_0 matrix. It adds a row's blocks in another order than the
 // matvecs below, so it is chosen by the matrix' size and the tokens alone: not by the row range of a call or by where the
-// matrix is kept. From eight tokens on always. With five to seven, on larger matrices (rows x inputs, without the
-// quantiser's launch, five tokens, Q8_0 / Q5_0: 22016 x 2048 20.2 -> 12.8 / 20.8 -> 14.7 us, 2048 x 8192 29.1 -> 20.3 / 28.2 ->
-// 24.1, but 2048 x 2048 7.9 against 8.8 / 8.1 against 10.8 and 2048 x 4096 11.1 against 12.3 / 11.4 against 14.4; 2048 x 4096,
-// six tokens 12.5 against 12.2 / 12.8 against 14.3, seven 14.3 against 12.3 / 14.7 against 14.3), and where the matvecs leave
-// lanes idle: rows of fewer than 64 units (of 64 elements) that do not divide a wave's lanes (2048 x 3072, five tokens:
-// 12.5 -> 10.3 / 12.6 -> 11.8).
+// matrix is kept. From nine tokens on always. With five to eight, on larger matrices (rows x inputs, without the quantiser's
+// launch, five tokens, Q8_0 / Q5_0: 22016 x 2048 20.2 -> 12.8 / 20.8 -> 14.7 us, 2048 x 8192 29.1 -> 20.3 / 28.2 -> 24.1, but
+// 2048 x 2048 7.9 against 8.8 / 8.1 against 10.8 and 2048 x 4096 11.1 against 12.3 / 11.4 against 14.4; 2048 x 4096, six tokens
+// 12.5 against 12.2 / 12.8 against 14.3, seven 14.3 against 12.3 / 14.7 against 14.3), and where a wave of the matvecs has lanes
+// idle: rows of 33 to 63 units of 64 elements (2048 x 3072, five tokens: 12.5 -> 10.3 / 12.6 -> 11.8). Not with very short rows, whose tiles end before they have begun (131072 x 256, five tokens 1.7 / 2.0 times the
+// matvec's time, eight 1.5 / 1.7; 131072 x 800, five 1.12 / 1.07).
 static bool blocks_take(const sdy_mat *m, int n_tok) {
-    if (n_tok < 5 || n_tok >= 8) return n_tok >= 8;
-    return (m->n_units < 64 && 64 % m->n_units) || (size_t)m->n_rows * m->n_in > (size_t)(8 - n_tok) << 22;
+    if (n_tok < 5 || n_tok > 8) return n_tok > 8;
+    if (m->n_units <= 4 || m->n_rows > 128L * m->n_in) return false;
+    return (m->n_units > 32 && m->n_units < 64) || (size_t)m->n_rows * m->n_in > (size_t)(8 - n_tok) << 22;
 }
 
 template <int WT>

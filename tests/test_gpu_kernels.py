@@ -1480,10 +1480,10 @@ def test_matrix_in_host_memory_same_bits(kind):
 
 
 @pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
-@pytest.mark.parametrize("n_in,n_out,n_tok", [(32, 33, 8), (96, 31, 31), (544, 130, 64), (2048, 129, 33), (2080, 66, 32),
+@pytest.mark.parametrize("n_in,n_out,n_tok", [(32, 33, 9), (96, 31, 31), (544, 130, 64), (2048, 129, 33), (2080, 66, 32),
                                               (4064, 96, 65), (11008, 70, 255), (11008, 200, 256), (2048, 2600, 517)])
 def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
-    """Eight and more tokens of the 32-element types (int8 MFMA), around the edges of its row, token and
+    """Nine and more tokens of the 32-element types (int8 MFMA), around the edges of its row, token and
     block tiles and of its wave splits, against float64: the integer dots and the scale products are exact, each
     output is a sum over the row's nb blocks whose longest chain is 8 + nb / 16 + 4 additions, each rounding by
     at most 2^-24 of a partial sum (itself at most the sum of the terms' magnitudes). The tiled copy, the
@@ -1541,9 +1541,9 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
 
 @pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
 @pytest.mark.parametrize("n_in,n_out,n_tok,mfma", [
-    (32, 33, 5, False), (2048, 2048, 5, False), (4096, 3072, 5, False), (4096, 3073, 5, True), (2048, 4096, 6, False),
-    (2048, 4097, 6, True), (2048, 2048, 7, False), (2048, 2049, 7, True), (2048, 64, 8, True), (1536, 70, 5, True),
-    (1536, 70, 4, False), (4160, 40, 7, False)])
+    (32, 33, 5, False), (256, 9000, 8, False), (320, 40961, 8, False), (320, 40960, 8, True), (2048, 2048, 5, False), (4096, 3072, 5, False), (4096, 3073, 5, True), (2048, 4096, 6, False),
+    (2048, 4097, 6, True), (2048, 2048, 7, False), (2048, 2049, 7, True), (2048, 64, 8, True), (3072, 70, 5, True),
+    (3072, 70, 4, False), (1536, 70, 7, False), (4160, 40, 7, False)])
 def test_block_types_few_tokens(kind, n_in, n_out, n_tok, mfma):
     """Where the block types change from the matvecs to the matrix cores: the kernel that runs; on the matvecs' side the
     bits of one token at a time; and either way the same bits from the planes, the tiled copy, pinned host memory and over
