@@ -66,20 +66,21 @@ SDY_DEV u32x2 bload8(__amdgpu_buffer_rsrc_t r, uint32_t v, int s) {
     return u32x2{(uint32_t)x[0], (uint32_t)x[1]};
 }
 
-template <int RW, int KS>
-constexpr size_t gemm_lds_bytes() { return 2 * (size_t)(32 * 292 * KS) + (KS > 1 ? RW * KS * 16 * 64 * 4 : 0); }
+template <int RW, int KS, int NT>
+constexpr size_t gemm_lds_bytes() { return 2 * (size_t)(32 * NT * 292 * KS) + (KS > 1 ? RW * KS * 16 * 64 * 4 : 0); }
 
-// A workgroup of RW * KS waves computes 32 RW rows x 32 tokens; a wave owns a row tile and, with KS > 1, every KS-th
+// A workgroup of RW * KS waves computes 32 RW rows x 32 NT tokens; a wave owns a row tile and, with KS > 1, every KS-th
 // super-block: its f32 terms go through LDS to the tile's waves, each adding up a part of the outputs over the KS
 // super-blocks in order. The activations are shared through LDS in stages of KS super-blocks, requested a stage ahead
 // into registers, 16-byte chunk c of a token's 256 at slot c ^ (token % 16) (16 tokens' reads of one chunk then hit all
 // 64 banks once). The weights go straight to registers, each lane (row lr, k-half h) loading its own records, and
 // are reloaded for the next stage as they are used: from the tiled copy a load instruction reads runs of 512
 // bytes. The workgroup's place in the grid is (bx, by) of (gx, gy): a pair launch gives each matrix a part of one grid.
-template <int WT, int RW, int KS>
+template <int WT, int RW, int KS, int NT>
 SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_t *lds) {
     constexpr bool Q4 = WT == SDY_Q4_K;
-    constexpr int BM = 32 * RW, BN = 32, NTH = 64 * RW * KS;
+    static_assert(NT == 1 || KS == 1, "token tiles share a wave's weights only where it has the row tile to itself");
+    constexpr int BM = 32 * RW, BN = 32 * NT, NTH = 64 * RW * KS;
     constexpr int NA = BN * 16 * KS / NTH;             // 16-byte chunks of activations per thread and stage
     constexpr int NS = (BN * 2 * KS + NTH - 1) / NTH;  // of their 16-element sums
     constexpr int NY = (BN * KS + NTH - 1) / NTH;      // and scales
@@ -192,32 +193,38 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
     };
 
     constexpr int NF = 16 / KS;  // the outputs a wave adds up: registers NF ks .. of the tile's 16
-    float acc[NF];
+    float acc[NT][NF];
 #pragma unroll
-    for (int i = 0; i < NF; i++) acc[i] = 0.0f;
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int i = 0; i < NF; i++) acc[nt][i] = 0.0f;
     float *xch = reinterpret_cast<float *>(lds + 2 * STAGE);
-    // isum += scale(j) * products j = 0 .. n - 1, each issued a step ahead of its use
-    auto sums = [&](auto issue, auto scale, auto n, i32x16 &isum) {
+    // isum[nt] += scale(j) * products (j, nt), j = 0 .. n - 1, each issued a step ahead of its use
+    auto sums = [&](auto issue, auto scale, auto n, i32x16 isum[NT]) {
         i32x16 p[2];
-        issue(0, p[0]);
+        issue(0, 0, p[0]);
 #pragma unroll
-        for (int j = 0; j < n(); j++) {
-            if (j + 1 < n()) issue(j + 1, p[(j + 1) & 1]);
-            const int f = scale(j);
+        for (int k = 0; k < n() * NT; k++) {
+            if (k + 1 < n() * NT) issue((k + 1) / NT, (k + 1) % NT, p[(k + 1) & 1]);
+            const int f = scale(k / NT), nt = k % NT;
 #pragma unroll
-            for (int i = 0; i < 16; i++) isum[i] += __mul24(f, p[j & 1][i]);  // |p| <= 32 * 15 * 128 or 16 * 63 * 128
+            for (int i = 0; i < 16; i++) isum[nt][i] += __mul24(f, p[k & 1][i]);  // |p| <= 32 * 15 * 128 or 16 * 63 * 128
             // hide where the sums come from: the compiler then keeps one multiply-add per product (it would add
             // the products of two sub-blocks at once, in three instructions and with both products' registers)
-            __asm__ volatile("" : "+v"(isum));
+            __asm__ volatile("" : "+v"(isum[nt]));
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     // the wave's super-block of stage s, and its weights' reload for the next stage
     auto compute = [&](int s, const uint8_t *buf) {
         const uint8_t *ab = buf + (ks * BN + lr) * 256;
-        i32x16 isum = {};
-        f16x8 gw;  // the mins (Q4_K) or scales (Q6_K) of the lane's 16-element groups 8 h .. 8 h + 7
+        i32x16 isum[NT] = {};
+        f16x8 gw;  // the mins (Q4_K) or -32 times the scales (Q6_K) of the lane's 16-element groups 8 h .. 8 h + 7
         float dl;  // d, and for Q4_K dmin in lane half 1
+        auto group_sums = [&](int nt, const f16x8 &w) {
+            const f16x8 bs = *reinterpret_cast<const f16x8 *>(buf + OFF_B + (ks * BN + 32 * nt + lr) * 32 + 16 * h);
+            return __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, w, f32x16{}, 0, 0, 0);
+        };
         if constexpr (Q4) {
             // 6-bit scales and mins of the 8 sub-blocks as bytes (csrc/quant.h:72-80)
             const uint32_t A = sc.y, B = sc.z, C = sc.w;
@@ -227,11 +234,14 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
 #pragma unroll
             for (int e = 0; e < 8; e++) gw[e] = (_Float16)(float)((mw >> (8 * (e >> 1))) & 255u);
             load_s(s + 1);
-            auto issue = [&](int j, i32x16 &p) {  // sub-block j: the low or high nibbles of unit j / 2, 16 to a lane half
-                const u32x4 w = w4[j >> 1];
-                const i32x4 wf = __builtin_bit_cast(i32x4, ((j & 1) ? w >> 4u : w) & 0x0F0F0F0Fu);
-                if (j & 1) load_u(s + 1, j >> 1);
-                const i32x4 a = *reinterpret_cast<const i32x4 *>(ab + 16 * ((2 * j + h) ^ (lr & 15)));
+            i32x4 wf;
+            auto issue = [&](int j, int nt, i32x16 &p) {  // sub-block j: the low or high nibbles of unit j / 2, 16 to a lane half
+                if (nt == 0) {
+                    const u32x4 w = w4[j >> 1];
+                    wf = __builtin_bit_cast(i32x4, ((j & 1) ? w >> 4u : w) & 0x0F0F0F0Fu);
+                    if (j & 1) load_u(s + 1, j >> 1);
+                }
+                const i32x4 a = *reinterpret_cast<const i32x4 *>(ab + 32 * 256 * nt + 16 * ((2 * j + h) ^ (lr & 15)));
                 p = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, wf, i32x16{}, 0, 0, 0);
             };
             sums(issue, [&](int j) { return (int)((sw[j >> 2] >> (8 * (j & 3))) & 255u); }, std::integral_constant<int, 8>{}, isum);
@@ -240,37 +250,51 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
             dl = sdy_h2f((uint16_t)d6);
             const uint32_t g0 = h ? scv.z : scv.x, g1 = h ? scv.w : scv.y;
 #pragma unroll
-            for (int e = 0; e < 8; e++) gw[e] = (_Float16)(float)(int8_t)(((e < 4 ? g0 : g1) >> (8 * (e & 3))) & 255u);
+            for (int e = 0; e < 8; e++) gw[e] = (_Float16)(-32.0f * (float)(int8_t)(((e < 4 ? g0 : g1) >> (8 * (e & 3))) & 255u));
             load_s(s + 1);
-            auto issue = [&](int j, i32x16 &p) {  // sub-block j = 4 u + k: elements 16 k .. of unit u, stored 32 too high
+            // the sums begin with what the 32 in every quant adds to them: exact, multiples of 32 below 2^27
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const f32x16 off = group_sums(nt, gw);
+#pragma unroll
+                for (int i = 0; i < 16; i++) isum[nt][i] = (int)off[i];
+            }
+            long wf;
+            auto issue = [&](int j, int nt, i32x16 &p) {  // sub-block j = 4 u + k: elements 16 k .. of unit u, stored 32 too high
                 const int u = j >> 2, k = j & 3;
-                const u32x2 nn = w6[u][k & 1], hb = w6[u][2];
-                const u32x2 lo = (k & 2) ? (nn >> 4u) & 0x0F0F0F0Fu : nn & 0x0F0F0F0Fu;
-                const u32x2 hi = k == 0 ? (hb & 0x03030303u) << 4u : k == 1 ? (hb & 0x0C0C0C0Cu) << 2u
-                                 : k == 2 ? hb & 0x30303030u : (hb >> 2u) & 0x30303030u;
-                if (k == 3) load_u(s + 1, u);
-                const long a = *reinterpret_cast<const long *>(ab + 16 * (j ^ (lr & 15)) + 8 * h);
-                p = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, as_long(lo | hi), i32x16{}, 0, 0, 0);
+                if (nt == 0) {
+                    const u32x2 nn = w6[u][k & 1], hb = w6[u][2];
+                    const u32x2 lo = (k & 2) ? (nn >> 4u) & 0x0F0F0F0Fu : nn & 0x0F0F0F0Fu;
+                    const u32x2 hi = k == 0 ? (hb & 0x03030303u) << 4u : k == 1 ? (hb & 0x0C0C0C0Cu) << 2u
+                                     : k == 2 ? hb & 0x30303030u : (hb >> 2u) & 0x30303030u;
+                    wf = as_long(lo | hi);
+                    if (k == 3) load_u(s + 1, u);
+                }
+                const long a = *reinterpret_cast<const long *>(ab + 32 * 256 * nt + 16 * (j ^ (lr & 15)) + 8 * h);
+                p = __builtin_amdgcn_mfma_i32_32x32x16_i8(a, wf, i32x16{}, 0, 0, 0);
             };
             sums(issue, [&](int j) { return (int)(int8_t)((scv[j >> 2] >> (8 * (j & 3))) & 255u); }, std::integral_constant<int, 16>{}, isum);
         }
-        const float yd = *reinterpret_cast<const float *>(buf + OFF_Y + (ks * BN + lr) * 4);
-        const f16x8 bs = *reinterpret_cast<const f16x8 *>(buf + OFF_B + (ks * BN + lr) * 32 + 16 * h);
-        const f32x16 off = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, gw, f32x16{}, 0, 0, 0);
-        // yd d in registers 0 .. 15 and (Q4_K) yd dmin in 16 .. 31: block b takes its factors from lane half b
-        const f32x32 sd = __builtin_amdgcn_mfma_f32_32x32x1f32(yd, dl, f32x32{}, 0, 0, 0);
         float *xw = xch + (size_t)wave * (16 * 64) + lane;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            float term;
-            if constexpr (Q4) {
-                const float t1 = sd[i] * (float)isum[i], t2 = sd[16 + i] * off[i];
-                term = t1 - t2;
-            } else {
-                term = sd[i] * (float)(isum[i] - 32 * (int)off[i]);
+        for (int nt = 0; nt < NT; nt++) {
+            const float yd = *reinterpret_cast<const float *>(buf + OFF_Y + (ks * BN + 32 * nt + lr) * 4);
+            f32x16 off;
+            if constexpr (Q4) off = group_sums(nt, gw);
+            // yd d in registers 0 .. 15 and (Q4_K) yd dmin in 16 .. 31: block b takes its factors from lane half b
+            const f32x32 sd = __builtin_amdgcn_mfma_f32_32x32x1f32(yd, dl, f32x32{}, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                float term;
+                if constexpr (Q4) {
+                    const float t1 = sd[i] * (float)isum[nt][i], t2 = sd[16 + i] * off[i];
+                    term = t1 - t2;
+                } else {
+                    term = sd[i] * (float)isum[nt][i];
+                }
+                if constexpr (KS == 1) acc[nt][i] = acc[nt][i] + term;
+                else xw[i * 64] = term;
             }
-            if constexpr (KS == 1) acc[i] = acc[i] + term;
-            else xw[i * 64] = term;
         }
     };
     // orders LDS only: the weights in flight stay in flight
@@ -301,7 +325,7 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
 #pragma unroll
             for (int k = 0; k < KS; k++)
 #pragma unroll
-                for (int i = 0; i < NF; i++) acc[i] = k < left ? acc[i] + v[k][i] : acc[i];
+                for (int i = 0; i < NF; i++) acc[0][i] = k < left ? acc[0][i] + v[k][i] : acc[0][i];
             barrier();  // the terms are read before the next stage's overwrite them
         }
     }
@@ -311,39 +335,42 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
     const bool on_row = ri < g.n_rows;
     const long row = g.grp_tile ? ri : g.row0 + ri;
     const float bias = g.bias && on_row ? g.bias[row] : 0.0f;
-    int orow[NF];
-    bool on[NF];
 #pragma unroll
-    for (int i = 0; i < NF; i++) {
-        const int f = NF * ks + i, t = t0 + 8 * (f >> 2) + 4 * h + (f & 3), tc = t < t_end ? t : t_end - 1;
-        on[i] = on_row && t < t_end;
-        orow[i] = g.out_row ? g.out_row[tc] : tc;
-    }
-    if (g.swiglu) {  // the pair's up row is in the next lane
+    for (int nt = 0; nt < NT; nt++) {
+        int orow[NF];
+        bool on[NF];
 #pragma unroll
         for (int i = 0; i < NF; i++) {
-            const float up = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc[i]), 0xB1, 0xF, 0xF, false));
-            const float v = sdy_silu_mul1_reg(acc[i], up, etab);
-            if (on[i] && !(lr & 1)) g.out[(size_t)orow[i] * g.out_stride + (ri >> 1)] = v;
+            const int f = NF * ks + i, t = t0 + 32 * nt + 8 * (f >> 2) + 4 * h + (f & 3), tc = t < t_end ? t : t_end - 1;
+            on[i] = on_row && t < t_end;
+            orow[i] = g.out_row ? g.out_row[tc] : tc;
         }
-        return;
-    }
-    float rv[NF];
+        if (g.swiglu) {  // the pair's up row is in the next lane
 #pragma unroll
-    for (int i = 0; i < NF; i++) rv[i] = g.resid && on[i] ? g.resid[(size_t)orow[i] * g.out_stride + row] : 0.0f;
+            for (int i = 0; i < NF; i++) {
+                const float up = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc[nt][i]), 0xB1, 0xF, 0xF, false));
+                const float v = sdy_silu_mul1_reg(acc[nt][i], up, etab);
+                if (on[i] && !(lr & 1)) g.out[(size_t)orow[i] * g.out_stride + (ri >> 1)] = v;
+            }
+            continue;
+        }
+        float rv[NF];
 #pragma unroll
-    for (int i = 0; i < NF; i++) {
-        float v = acc[i];
-        if (g.bias) v = v + bias;
-        if (g.resid) v = rv[i] + v;
-        if (on[i]) g.out[(size_t)orow[i] * g.out_stride + row] = v;
+        for (int i = 0; i < NF; i++) rv[i] = g.resid && on[i] ? g.resid[(size_t)orow[i] * g.out_stride + row] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < NF; i++) {
+            float v = acc[nt][i];
+            if (g.bias) v = v + bias;
+            if (g.resid) v = rv[i] + v;
+            if (on[i]) g.out[(size_t)orow[i] * g.out_stride + row] = v;
+        }
     }
 }
 
-template <int WT, int RW, int KS>
-__global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm(GemmArgs g) {
+template <int WT, int RW, int KS, int NT>
+__global__ __launch_bounds__(64 * RW * KS, NT == 1 ? 3 : 2) void k_gemm(GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds[];
-    gemm_body<WT, RW, KS>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
+    gemm_body<WT, RW, KS, NT>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
 }
 
 // Two GEMMs on the same activations in one launch (a layer's q|k and a v of another type): row tiles [0, gy1) of
@@ -351,8 +378,8 @@ __global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm(GemmArgs g) {
 template <int WT1, int WT2, int RW, int KS>
 __global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm_pair(GemmArgs g1, GemmArgs g2, int gy1) {
     extern __shared__ __align__(16) uint8_t lds[];
-    if ((int)blockIdx.y < gy1) gemm_body<WT1, RW, KS>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds);
-    else gemm_body<WT2, RW, KS>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x, (int)gridDim.y - gy1, lds);
+    if ((int)blockIdx.y < gy1) gemm_body<WT1, RW, KS, 1>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds);
+    else gemm_body<WT2, RW, KS, 1>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x, (int)gridDim.y - gy1, lds);
 }
 
 // Q8_K rows -> the GEMM's expansion: int8 values, f32 scales and f16 sums in planes of their own (exact: |bsum| <=
@@ -565,43 +592,68 @@ extern "C" int sdy_gemm_ok(const sdy_mat *m, int n_tok) {
 // rows of one take the matvec.)
 static bool gemm_far(const GemmArgs &g) { return (size_t)(g.p[1] - g.p[0]) + (size_t)g.T * 4096 > 0xFFFFFFFFu; }
 
-template <int WT, int RW, int KS>
+template <int WT, int RW, int KS, int NT = 1>
 static int launch_gemm(const GemmArgs &g, unsigned tok_tiles, hipStream_t st) {
-    constexpr size_t lds = gemm_lds_bytes<RW, KS>();
+    constexpr size_t lds = gemm_lds_bytes<RW, KS, NT>();
     static size_t granted = 0;
-    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS>, lds, &granted)) return rc;
-    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS>));
-    hipLaunchKernelGGL((k_gemm<WT, RW, KS>), dim3(tok_tiles, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))), dim3(64 * RW * KS),
-                       lds, st, g);
+    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS, NT>, lds, &granted)) return rc;
+    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS, NT>));
+    hipLaunchKernelGGL((k_gemm<WT, RW, KS, NT>), dim3((tok_tiles + NT - 1) / NT, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))),
+                       dim3(64 * RW * KS), lds, st, g);
     return sdy_check_launch("gemm");
 }
 
-// The forms of the GEMM, by the 32 x 32 tiles of its output: four waves to two tiles' super-blocks each (KS 4) while
-// the tiles alone are fewer than two to a CU, two up to eight (KS 2), one to a tile beyond (with the quantiser's
-// launch, forms KS 4, 2, 1: Q4_K 2048 x 2048, 130 tokens: 11.8, 13.6, 17.3 us; 512 tokens: 21.2, 18.5, 19.1;
-// 22016 x 2048, 64 tokens: 27.0, 20.8, 22.6; 128 tokens: 47.4, 33.4, 29.0).
-static int gemm_form(long n_rows, int n_tok) {
-    const long tiles = (n_rows + 31) / 32 * ((n_tok + 31) / 32);
-    return tiles < 512 ? 4 : tiles < 2048 ? 2 : 1;
+// The forms of the GEMM: the 16 x 16 tiles of mm_superblocks.hip (0); 32 x 32 tiles, a tile's super-blocks over four waves
+// (4), two (2) or one (1); and one wave to two token tiles (12), which unpacks the weights once for 64 tokens with two
+// waves to a SIMD instead of three. All give the same bits, so they are chosen by size and by whether the weights come
+// from the tiled copy. By the 32 x 32 tiles: four waves while these alone are fewer than two to a CU, two up to eight, one
+// beyond (Q4_K 2048 x 2048, 130 tokens: 11.8, 13.6, 17.3 us; 512 tokens: 21.2, 18.5, 19.1; 22016 x 2048, 64 tokens: 27.0,
+// 20.8, 22.6; 128 tokens: 47.4, 33.4, 29.0; with the quantiser's launch). Beside that (rows x inputs, without it):
+// - Small grids: the 16 x 16 tiles, up to 2.5 to a CU and up to 16 tokens on more rows (Q4_K 2560 x 2048, 64 tokens: 10.0
+//   against 11.4, 128 tokens 12.7 against 11.8; 22016 x 2048, 16 tokens 12.2 against 16.1).
+// - Rows too short to split (Q4_K to two super-blocks, Q6_K to three): the 16 x 16 tiles further, then two waves, then one
+//   (Q6_K 4096 x 768, 64 tokens: 6.3 us, with four waves 8.4; 8192 x 768, 96 tokens: one wave 10.4, two 10.9; 4096 x 256, 96 tokens:
+//   5.5, two waves 6.7; Q4_K 4096 x 512, 96 tokens: 5.5, two 6.0; Q6_K 8192 x 512, 160 tokens: two 9.7, one 11.2, 256: 12.7, 11.8).
+// - Q6_K on large grids: two token tiles, half the unpacking of 6 bits (32768 x 2048, 512 tokens: 183 -> 160 us; 256: 95 -> 85),
+//   from four workgroups to a CU, six on shorter rows (147456 x 1024, 128 tokens: 110 -> 106; 22016 x 768, 512 tokens 55.0
+//   against 59.9), where the last pair of tiles is whole or one of several (65536 x 2048, 96 tokens: 72 against 84). Q4_K's
+//   nibbles cost less than the third wave (22016 x 2048, 512 tokens: 70.4 against 83.9).
+// - From the planes, where a wave's load of 32 rows' units meets as many cache lines: two token tiles as soon as they
+//   fill the chip (22016 x 2048, 512 tokens: Q6_K 176 -> 131 us, Q4_K 107 -> 89), two waves before (Q4_K 22016 x 8192, 96
+//   tokens: 111 -> 82).
+static int gemm_form(const sdy_mat *m, long n_rows, int n_tok) {
+    const int nb = m->n_in / 256;
+    const bool q4 = m->type == SDY_Q4_K, tiled = m->gbase != nullptr, few = nb <= (q4 ? 2 : tiled ? 3 : 4);
+    const long t16 = (n_rows + 15) / 16 * ((n_tok + 15) / 16), t32 = (n_rows + 31) / 32 * ((n_tok + 31) / 32);
+    const long wide = (n_rows + 127) / 128 * ((n_tok + 63) / 64);
+    const long line = few ? (nb == 1 ? (q4 ? 3072 : 2560) : q4 ? 1408 : 1024) : tiled ? 640 : 512;
+    // (host memory: a row's token tiles read it together only where they run on one XCD, not as 16 x 16 tiles)
+    if (m->hbase ? n_tok <= 16 : t16 <= line || (n_tok <= 16 && t16 <= (q4 && (tiled || few) ? 4096 : 1024))) return 0;
+    if (few && (tiled || q4 || t32 < 2048)) {
+        const long two = nb == 2 && (tiled || q4) ? (tiled ? 1536 : 2048) : q4 ? 1024 : 513;
+        return t32 < two ? 2 : 1;
+    }
+    if (!tiled) return t32 < 512 ? 4 : t32 < (q4 ? 4096 : 2048) ? 2 : 12;
+    const int tt = (n_tok + 31) / 32;
+    if (!q4 && (wide >= 1536 ? nb >= 4 : wide >= 1024 && nb >= 6) && (tt % 2 == 0 || tt > 8)) return 12;
+    return t32 < 512 ? 4 : t32 < 2048 ? 2 : 1;
 }
 
 template <int WT>
 static int gemm_type(const GemmArgs &g, const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
-    // SARDYNE_GEMM_VARIANT picks one form (tests and tuning); default: by shape
+    // SARDYNE_GEMM_VARIANT picks one form (tests and tuning): 11, 12, 13: one, two, four waves; 14: 16 x 16 tiles; 15: two
+    // token tiles. Default: by shape
     const char *ev = getenv("SARDYNE_GEMM_VARIANT");
     const int variant = ev ? atoi(ev) : 0;
+    static const int forms[] = {1, 2, 4, 0, 12};
+    int form = variant >= 11 && variant <= 15 ? forms[variant - 11] : gemm_form(m, g.n_rows, g.n_tok);
     const unsigned tt = (unsigned)((g.n_tok + 31) / 32);
-    // Small grids: the 16 x 16 tiles of mm_superblocks.hip, up to 2.5 to a CU, and up to 16 tokens on more rows (with the
-    // quantiser's launch: Q4_K 2560 x 2048, 64 tokens: 10.0 us against 11.4, 128 tokens 12.7 against 11.8; 22016 x 2048,
-    // 16 tokens: 12.2 against 16.1, 24 tokens 18.1 against 16.3; Q6_K 2048 x 11008, 64 tokens 31.6 against 42.3, 128
-    // tokens 63.7 against 44.3; 151936 x 2048, 16 tokens: 88.4 against 72.5).
-    const long t16 = (g.n_rows + 15) / 16 * ((g.n_tok + 15) / 16);
-    const bool small = variant == 14 || (!variant && (t16 <= 640 || (g.n_tok <= 16 && t16 <= (WT == SDY_Q4_K ? 4096 : 1024))));
-    if (small) {
+    if (form == 0) {
         const int rc = sdy_mm_superblocks_exp(m, a, &g.e, (sdy_stream)st);
         if (rc <= 0) return rc;
+        form = 4;
     }
-    const int form = variant == 11 ? 1 : variant == 12 ? 2 : variant == 13 ? 4 : gemm_form(g.n_rows, g.n_tok);
+    if (form == 12) return launch_gemm<WT, 4, 1, 2>(g, tt, st);
     if (form == 4) return launch_gemm<WT, 2, 4>(g, tt, st);
     return form == 2 ? launch_gemm<WT, 2, 2>(g, tt, st) : launch_gemm<WT, 4, 1>(g, tt, st);
 }
@@ -657,7 +709,7 @@ extern "C" int sdy_gemm(const sdy_mat *m, const sdy_mv_args *a, void *ws, sdy_st
 
 template <int RW, int KS>
 static int launch_gemm_pair(const GemmArgs &g1, const GemmArgs &g2, hipStream_t st) {
-    constexpr size_t lds = gemm_lds_bytes<RW, KS>();
+    constexpr size_t lds = gemm_lds_bytes<RW, KS, 1>();
     static size_t granted = 0;
     if (int rc = sdy_lds_limit((const void *)k_gemm_pair<SDY_Q4_K, SDY_Q6_K, RW, KS>, lds, &granted)) return rc;
     const int gy1 = (int)((g1.n_rows + 32 * RW - 1) / (32 * RW)), gy2 = (int)((g2.n_rows + 32 * RW - 1) / (32 * RW));
@@ -667,17 +719,17 @@ static int launch_gemm_pair(const GemmArgs &g1, const GemmArgs &g2, hipStream_t 
     return sdy_check_launch("gemm2");
 }
 
-// Two GEMMs over the same activations (a layer's q|k and its v): one launch when the first matrix is Q4_K and the
-// second Q6_K and neither would fill the GPU by itself (the KS forms); otherwise, or with SARDYNE_GEMM_VARIANT set, two
-// sdy_gemm calls. The same bits either way.
+// Two GEMMs over the same activations (a layer's q|k and its v): one launch, on the forms of four waves or two (rows of one
+// or two super-blocks: the 16 x 16 tiles), when the first matrix is Q4_K and the second Q6_K and neither would fill the GPU
+// by itself; otherwise, or with SARDYNE_GEMM_VARIANT set, two sdy_gemm calls. The same bits either way.
 extern "C" int sdy_gemm2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat *m2, const sdy_mv_args *a2, void *ws,
                          sdy_stream s) {
     hipStream_t st = (hipStream_t)s;
     if (a2->xq != a1->xq || a2->n_tok != a1->n_tok || m2->n_in != m1->n_in)
         return sdy_fail(-1, "gemm2: the two GEMMs must read the same activation rows");
-    const long rows = (a1->row1 - a1->row0) + (a2->row1 - a2->row0);
+    const long rows = (a1->row1 - a1->row0) + (a2->row1 - a2->row0), tiles = (rows + 31) / 32 * ((a1->n_tok + 31) / 32);
     const bool pair = m1->type == SDY_Q4_K && m2->type == SDY_Q6_K && !getenv("SARDYNE_GEMM_VARIANT") &&
-                      a1->row1 > a1->row0 && a2->row1 > a2->row0 && gemm_form(rows, a1->n_tok) > 1;
+                      a1->row1 > a1->row0 && a2->row1 > a2->row0 && tiles < 2048;
     sdy_mv_args b = *a2;
     b.ws_ready = 1;  // the expansion the first call makes (or finds)
     if (!pair) {
@@ -692,7 +744,12 @@ extern "C" int sdy_gemm2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat
         if (int rc = sdy_matvec(m1, a1, s)) return rc;
         return sdy_gemm(m2, &b, ws, s);
     }
-    return gemm_form(rows, g1.n_tok) == 4 ? launch_gemm_pair<2, 4>(g1, g2, st) : launch_gemm_pair<2, 2>(g1, g2, st);
+    // (384 + 128 rows x 256, 64 tokens: 3.5 us, four waves to a tile 7.4; 768 + 256 x 512: 3.8 against 6.6)
+    if (g1.nb <= 2 && (rows + 30) / 16 * ((a1->n_tok + 15) / 16) <= 1408) {
+        const int rc = sdy_mm_superblocks_exp2(m1, a1, m2, &b, &g1.e, s);
+        if (rc <= 0) return rc;
+    }
+    return tiles < 512 ? launch_gemm_pair<2, 4>(g1, g2, st) : launch_gemm_pair<2, 2>(g1, g2, st);
 }
 
 extern "C" int sdy_gemm_grouped_tile(void) { return 32; }

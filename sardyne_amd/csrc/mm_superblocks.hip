@@ -53,15 +53,14 @@ SDY_DEV long as_long(u32x2 v) { return __builtin_bit_cast(long, v); }
 // sub-blocks at once, in three instructions).
 SDY_DEV void opaque(i32x4 &v) { __asm__ volatile("" : "+v"(v)); }
 
-// KS: waves, super-blocks of a round
+// KS: waves, super-blocks of a round. by: the workgroup's row tile
 template <int WT, int MT, int KS, bool EXP>
-__global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
+SDY_DEV void sb_body(const SbArgs &g, int by, float (*terms)[KS][MT * 256]) {
     constexpr bool Q4 = WT == SDY_Q4_K;
     constexpr int OUT = MT * 256, NTH = 64 * KS;  // outputs of the workgroup, threads
-    __shared__ float terms[2][KS][OUT];
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const long rt = (long)blockIdx.y * (16 * MT);
+    const long rt = (long)by * (16 * MT);
     const int t0 = (int)blockIdx.x * 16, nb = g.nb;
 
     // The lane's rows n of each row tile: byte offsets of their records, and from one unit's (super-block's) to the
@@ -247,6 +246,21 @@ __global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
 }
 
 template <int WT, int MT, int KS, bool EXP>
+__global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks(SbArgs g) {
+    __shared__ float terms[2][KS][MT * 256];
+    sb_body<WT, MT, KS, EXP>(g, (int)blockIdx.y, terms);
+}
+
+// Two matrices, Q4_K and Q6_K, on the same activations in one launch: row tiles [0, gy1) of the grid multiply g1, the rest
+// g2.
+template <int KS>
+__global__ __launch_bounds__(64 * KS, 2) void k_mm_superblocks_pair(SbArgs g1, SbArgs g2, int gy1) {
+    __shared__ float terms[2][KS][256];
+    if ((int)blockIdx.y < gy1) sb_body<SDY_Q4_K, 1, KS, true>(g1, (int)blockIdx.y, terms);
+    else sb_body<SDY_Q6_K, 1, KS, true>(g2, (int)blockIdx.y - gy1, terms);
+}
+
+template <int WT, int MT, int KS, bool EXP>
 int launch_ks(const SbArgs &g, hipStream_t st) {
     SDY_NOTE_KERNEL((k_mm_superblocks<WT, MT, KS, EXP>));
     hipLaunchKernelGGL((k_mm_superblocks<WT, MT, KS, EXP>),
@@ -254,22 +268,24 @@ int launch_ks(const SbArgs &g, hipStream_t st) {
     return sdy_check_launch("matvec (super-block MFMA)");
 }
 
-// Four waves to a workgroup where rows have no more super-blocks: with eight, half of them held their places for nothing
-// (1024 x 33786 Q4_K, 3 tokens: 12.9 us, where the 8-token matvec took 12.6; now 10.9)
+// As many waves to a workgroup as rows have super-blocks, up to eight: the others would only hold their places (1024 x 33786
+// Q4_K, 3 tokens: 12.9 us with eight, 10.9 with four, where the 8-token matvec took 12.6).
 template <int WT, int MT, bool EXP>
 int launch_sb(const SbArgs &g, hipStream_t st) {
+    if (g.nb <= 2) return launch_ks<WT, MT, 2, EXP>(g, st);
     return g.nb <= 4 ? launch_ks<WT, MT, 4, EXP>(g, st) : launch_ks<WT, MT, 8, EXP>(g, st);
 }
 
+// The kernel's arguments of one call; 1 when its 32-bit offsets do not reach every byte of the matrix or the activations.
 template <bool EXP>
-int run_sb(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, hipStream_t st) {
+int sb_args(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, SbArgs &g) {
     const int nb = m->n_in / 256;
     const size_t lim = 0xFFFFFFFFu;
     const long n_rows = a->row1 - a->row0;
     if (m->bytes >= lim || m->gbytes >= lim || (size_t)nb * 292 * a->n_tok >= lim || (!EXP && ((uintptr_t)a->xq & 3)) ||
         (n_rows + 15) / 16 > 65535)
         return 1;
-    SbArgs g = {};
+    g = SbArgs{};
     for (int i = 0; i < 5; i++) g.p[i] = (const uint8_t *)m->base + m->plane_off[i];
     if (m->gbase) {
         size_t off[5];
@@ -290,11 +306,18 @@ int run_sb(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, hipStrea
     g.bias = a->bias;
     g.resid = a->resid;
     g.swiglu = a->epilogue == SDY_EPI_SWIGLU;
+    return 0;
+}
+
+template <bool EXP>
+int run_sb(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, hipStream_t st) {
+    SbArgs g;
+    if (int rc = sb_args<EXP>(m, a, e, g)) return rc;
     // Two row tiles to a wave, sharing the activations' loads: Q4_K when one each gives every CU more than two
     // workgroups (22016 x 2048, 8 tokens: 11.2 us against 13.2; 2048 x 4096: 10.0 against 8.4), Q6_K, whose registers then
     // leave two waves to a SIMD, only with several token tiles (2048 x 11008, 64 tokens: 31.6 against 37.0; 151936 x
     // 2048, 8 tokens: 104 against 84)
-    const long tiles = (n_rows + 15) / 16 * ((g.n_tok + 15) / 16);
+    const long tiles = (g.n_rows + 15) / 16 * ((g.n_tok + 15) / 16);
     if (m->type == SDY_Q6_K)
         return g.n_tok > 16 && tiles >= 512 ? launch_sb<SDY_Q6_K, 2, EXP>(g, st) : launch_sb<SDY_Q6_K, 1, EXP>(g, st);
     return tiles > 512 ? launch_sb<SDY_Q4_K, 2, EXP>(g, st) : launch_sb<SDY_Q4_K, 1, EXP>(g, st);
@@ -311,4 +334,18 @@ extern "C" int sdy_mm_superblocks(const sdy_mat *m, const sdy_mv_args *a, sdy_st
 // The same from the GEMM's expansion of the activations.
 int sdy_mm_superblocks_exp(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, sdy_stream s) {
     return run_sb<true>(m, a, e, (hipStream_t)s);
+}
+
+// A Q4_K and a Q6_K matrix of one or two super-blocks to a row in one launch, from one expansion.
+int sdy_mm_superblocks_exp2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat *m2, const sdy_mv_args *a2,
+                            const SdyGemmExp *e, sdy_stream s) {
+    SbArgs g1, g2;
+    if (m1->type != SDY_Q4_K || m2->type != SDY_Q6_K || m1->n_in > 512 || sb_args<true>(m1, a1, e, g1) || sb_args<true>(m2, a2, e, g2))
+        return 1;
+    const long gy1 = (g1.n_rows + 15) / 16, gy2 = (g2.n_rows + 15) / 16;
+    if (gy1 + gy2 > 65535) return 1;
+    SDY_NOTE_KERNEL(k_mm_superblocks_pair<2>);
+    hipLaunchKernelGGL(k_mm_superblocks_pair<2>, dim3((unsigned)((g1.n_tok + 15) / 16), (unsigned)(gy1 + gy2)), dim3(128), 0,
+                       (hipStream_t)s, g1, g2, (int)gy1);
+    return sdy_check_launch("gemm2 (super-block MFMA)");
 }

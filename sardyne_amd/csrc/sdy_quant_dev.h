@@ -123,6 +123,9 @@ inline SdyGemmExp sdy_gemm_exp(void *ws, int n_tok, int n_in) {
 // Several tokens of a Q4_K / Q6_K matrix from that form (mm_superblocks.hip): 0, 1 when it does not take the call, or
 // an error.
 int sdy_mm_superblocks_exp(const sdy_mat *m, const sdy_mv_args *a, const SdyGemmExp *e, sdy_stream s);
+// A Q4_K and a Q6_K matrix of short rows in one launch, likewise.
+int sdy_mm_superblocks_exp2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat *m2, const sdy_mv_args *a2,
+                            const SdyGemmExp *e, sdy_stream s);
 
 // The block in the reference layout (292 bytes at ob: f32 d, int8 qs[256], int16 bsums[16]).
 SDY_DEV void sdy_q8k_block(const float xs[4], int lane, uint8_t *ob) {

@@ -1679,17 +1679,68 @@ def test_gemm_forms_bit_exact(kind, n_in, n_out, n_tok, kernel):
     assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out))), bits(exp))
 
 
-@pytest.mark.parametrize("variant", ["11", "12", "13", "14", "15", "16", "17", "18", "19", "20"])
+@pytest.mark.parametrize("kind,n_in,n_out,n_tok,tiled,planes", [
+    ("Q4_K", 256, 12288, 64, "k_mm_superblocks<12, 2, 2", "k_mm_superblocks<12, 2, 2"), ("Q4_K", 256, 12289, 64, "k_gemm<12, 2, 2, 1", "k_gemm<12, 2, 2, 1"),
+    ("Q4_K", 512, 5633, 64, "k_gemm<12, 2, 2, 1", "k_gemm<12, 2, 2, 1"), ("Q4_K", 512, 24577, 40, "k_gemm<12, 4, 1, 1", "k_gemm<12, 2, 2, 1"),
+    ("Q6_K", 256, 10240, 64, "k_mm_superblocks<14, 2, 2", "k_mm_superblocks<14, 2, 2"), ("Q6_K", 512, 4096, 64, "k_mm_superblocks<14, 2, 2", "k_mm_superblocks<14, 2, 2"),
+    ("Q6_K", 512, 16385, 40, "k_gemm<14, 2, 2, 1", "k_gemm<14, 4, 1, 1"), ("Q6_K", 768, 4097, 64, "k_gemm<14, 2, 2, 1", "k_gemm<14, 2, 2, 1"),
+    ("Q6_K", 768, 8224, 64, "k_gemm<14, 4, 1, 1", "k_gemm<14, 4, 1, 1"), ("Q6_K", 1280, 65505, 17, "k_gemm<14, 4, 1, 1", "k_gemm<14, 4, 1, 2"),
+    ("Q4_K", 768, 65505, 33, "k_gemm<12, 4, 1, 1", "k_gemm<12, 4, 1, 2"), ("Q6_K", 1536, 130945, 33, "k_gemm<14, 4, 1, 2", "k_gemm<14, 4, 1, 2")])
+def test_gemm_form_lines(kind, n_in, n_out, n_tok, tiled, planes):
+    """The forms chosen for short rows, for large grids and for weights read from the planes, near the lines between them
+    and with partial tiles: the kernel, and the oracle's bits."""
+    t = TYPES[kind]
+    w = _full_range_blocks(kind, n_out, n_in, n_in + n_tok)
+    xq = O.quantize(np.random.default_rng(n_tok).standard_normal((n_tok, n_in)).astype(np.float32), O.Q8_K)
+    exp = O.matmul_q(w, t, xq, n_in, simd=1)
+    L = lib()
+    dq, out = capi.DeviceBuffer.from_array(xq), capi.DeviceBuffer(n_tok * n_out * 4)
+    ws = capi.DeviceBuffer(L.sdy_gemm_ws_bytes(n_tok, n_in))
+    for layout, kernel in ((True, tiled), (False, planes)):
+        m = capi.DeviceMatrix(t, n_in, n_out, w, gemm_layout=layout)
+        a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out, row0=0, row1=n_out)
+        capi.check(L.sdy_gemm(ctypes.byref(m.m), ctypes.byref(a), ws.ptr, None))
+        assert kernel in L.sdy_last_kernel().decode()
+        assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_out))), bits(exp))
+        m.close()
+
+
+@pytest.mark.parametrize("n_in", [256, 512])
+@pytest.mark.parametrize("rows1,rows2,n_tok,pair", [(33, 7, 2, True), (384, 128, 64, True), (600, 77, 450, True), (1281, 300, 450, False)])
+def test_gemm2_short_rows_bit_exact(n_in, rows1, rows2, n_tok, pair):
+    """sdy_gemm2 over rows of one and two super-blocks: small grids as 16 x 16 tiles in one launch, larger ones on the form
+    of two waves; the oracle's bits, with bias and residual, from the tiled copies and the planes."""
+    L = lib()
+    rng = np.random.default_rng(rows1 + n_tok)
+    xq = O.quantize(rng.standard_normal((n_tok, n_in)).astype(np.float32), O.Q8_K)
+    dq, ws = capi.DeviceBuffer.from_array(xq), capi.DeviceBuffer(L.sdy_gemm_ws_bytes(n_tok, n_in))
+    w = [_full_range_blocks(k, r, n_in, r) for k, r in (("Q4_K", rows1), ("Q6_K", rows2))]
+    bias, resid = rng.standard_normal(rows1).astype(np.float32), rng.standard_normal((n_tok, rows2)).astype(np.float32)
+    db, dr = capi.DeviceBuffer.from_array(bias), capi.DeviceBuffer.from_array(resid)
+    exp = [O.matmul_q(w[0], O.Q4_K, xq, n_in, simd=1) + bias, resid + O.matmul_q(w[1], O.Q6_K, xq, n_in, simd=1)]
+    for layout in (True, False):
+        m = [capi.DeviceMatrix(t, n_in, r, x, gemm_layout=layout) for t, r, x in ((O.Q4_K, rows1, w[0]), (O.Q6_K, rows2, w[1]))]
+        d = [capi.DeviceBuffer.from_array(np.full((n_tok, r), np.nan, np.float32)) for r in (rows1, rows2)]
+        a1 = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=d[0].ptr, out_stride=rows1, row0=0, row1=rows1, bias=db.ptr)
+        a2 = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=d[1].ptr, out_stride=rows2, row0=0, row1=rows2, resid=dr.ptr)
+        capi.check(L.sdy_gemm2(ctypes.byref(m[0].m), ctypes.byref(a1), ctypes.byref(m[1].m), ctypes.byref(a2), ws.ptr, None))
+        assert ("k_mm_superblocks_pair" if pair else "k_gemm_pair<12, 14, 2, 2>") in L.sdy_last_kernel().decode()
+        for i, r in enumerate((rows1, rows2)):
+            assert np.array_equal(bits(d[i].to_array(np.float32, (n_tok, r))), bits(exp[i]))
+
+
+@pytest.mark.parametrize("variant,kernel", [("11", "k_gemm<%d, 4, 1, 1>"), ("12", "k_gemm<%d, 2, 2, 1>"), ("13", "k_gemm<%d, 2, 4, 1>"),
+                                            ("14", "k_mm_superblocks<%d, "), ("15", "k_gemm<%d, 4, 1, 2>")])
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
-def test_gemm_tile_variants_bit_exact(kind, variant, monkeypatch):
-    """Every workgroup tile shape of the GEMM (forced through SARDYNE_GEMM_VARIANT; 17, 18 and 20 split
-    each super-block's units between two waves, 19 and 20 keep two super-blocks in flight) gives the
-    reference's bits, with partial row and token tiles (1 to 43 super-blocks: every remainder of the
-    rounds of three), in its one-fragment and wide forms, and with the SwiGLU and residual epilogues."""
+def test_gemm_tile_variants_bit_exact(kind, variant, kernel, monkeypatch):
+    """Every form of the GEMM (forced through SARDYNE_GEMM_VARIANT: one, two or four waves to a tile's super-blocks, the 16 x 16
+    tiles, two token tiles to a wave) runs the kernel it names and gives the reference's bits, with partial row and token
+    tiles, 1 to 43 super-blocks, scales over their whole range, and with the SwiGLU and residual epilogues."""
     monkeypatch.setenv("SARDYNE_GEMM_VARIANT", variant)
     for n_in, n_out, n_tok in [(256, 64, 40), (512, 96, 33), (2048, 300, 200), (768, 40, 17), (11008, 70, 130)]:
         t, w, xq = _gemm_case(kind, n_in, n_out, n_tok, seed=n_in + n_out + n_tok + 1)
         got = _gemm_run(t, w, xq, n_in, n_out, n_tok)
+        assert kernel % t in lib().sdy_last_kernel().decode()
         exp = O.matmul_q(w, t, xq, n_in, simd=1)
         assert np.array_equal(bits(got), bits(exp)), (n_in, n_out, n_tok)
     sw = _gemm_run(t, w, xq, n_in, n_out, n_tok, epilogue=capi.EPI_SWIGLU)
