@@ -76,7 +76,8 @@ constexpr size_t gemm_lds_bytes() { return 2 * (size_t)(32 * NT * 292 * KS) + (K
 // 64 banks once). The weights go straight to registers, each lane (row lr, k-half h) loading its own records, and
 // are reloaded for the next stage as they are used: from the tiled copy a load instruction reads runs of 512
 // bytes. The workgroup's place in the grid is (bx, by) of (gx, gy): a pair launch gives each matrix a part of one grid.
-template <int WT, int RW, int KS, int NT>
+// FAR: Q4_K planes too far apart for a lane to reach both by a 32-bit offset: 64-bit addresses.
+template <int WT, int RW, int KS, int NT, bool FAR>
 SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_t *lds) {
     constexpr bool Q4 = WT == SDY_Q4_K;
     static_assert(NT == 1 || KS == 1, "token tiles share a wave's weights only where it has the row tile to itself");
@@ -133,13 +134,16 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
                                  r2 = rsrc(g.p[2] + (Q4 ? sb0 : ub) * 16), r3 = rsrc(g.p[3] + sb0 * 16), r4 = rsrc(g.p[4] + sb0 * 2);
     // (Q4_K: lane half h reads plane h; Q6_K: bytes 8 h .. of each plane's record)
     const uint32_t vq = vu + (Q4 ? (h ? (uint32_t)(g.p[1] - g.p[0]) : 0u) : 8u * (uint32_t)h);
+    const uint8_t *const vfar = (h ? g.p[1] : g.p[0]) + ub * 16 + vu;
     u32x4 w4[Q4 ? 4 : 1], sc;
     u32x2 w6[Q4 ? 1 : 4][3];
     uint32_t d6 = 0;
     auto sb_of = [&](int s) { return s * KS + ks < nb ? s * KS + ks : nb - 1; };  // (past the end: not added)
     auto load_u = [&](int s, int u) {
         const int so = (4 * sb_of(s) + u) * us;
-        if constexpr (Q4) {
+        if constexpr (Q4 && FAR) {
+            w4[u] = *reinterpret_cast<const u32x4 *>(vfar + so);
+        } else if constexpr (Q4) {
             w4[u] = __builtin_amdgcn_raw_buffer_load_b128(r0, vq, so, 0);
         } else {
             w6[u][0] = bload8(r0, vq, so);
@@ -367,10 +371,10 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
     }
 }
 
-template <int WT, int RW, int KS, int NT>
+template <int WT, int RW, int KS, int NT, bool FAR>
 __global__ __launch_bounds__(64 * RW * KS, NT == 1 ? 3 : 2) void k_gemm(GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds[];
-    gemm_body<WT, RW, KS, NT>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
+    gemm_body<WT, RW, KS, NT, FAR>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
 }
 
 // Two GEMMs on the same activations in one launch (a layer's q|k and a v of another type): row tiles [0, gy1) of
@@ -378,8 +382,8 @@ __global__ __launch_bounds__(64 * RW * KS, NT == 1 ? 3 : 2) void k_gemm(GemmArgs
 template <int WT1, int WT2, int RW, int KS>
 __global__ __launch_bounds__(64 * RW * KS, 3) void k_gemm_pair(GemmArgs g1, GemmArgs g2, int gy1) {
     extern __shared__ __align__(16) uint8_t lds[];
-    if ((int)blockIdx.y < gy1) gemm_body<WT1, RW, KS, 1>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds);
-    else gemm_body<WT2, RW, KS, 1>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x, (int)gridDim.y - gy1, lds);
+    if ((int)blockIdx.y < gy1) gemm_body<WT1, RW, KS, 1, false>(g1, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, gy1, lds);
+    else gemm_body<WT2, RW, KS, 1, false>(g2, (int)blockIdx.x, (int)blockIdx.y - gy1, (int)gridDim.x, (int)gridDim.y - gy1, lds);
 }
 
 // Q8_K rows -> the GEMM's expansion: int8 values, f32 scales and f16 sums in planes of their own (exact: |bsum| <=
@@ -588,17 +592,17 @@ extern "C" int sdy_gemm_ok(const sdy_mat *m, int n_tok) {
            (size_t)m->n_rows * m->n_units * 16 < 0xFFFFFFFFu;
 }
 
-// A Q4_K lane reaches both quant planes by one 32-bit offset from its row tile in the first. (A plane of 4 GiB: the
-// rows of one take the matvec.)
+// A Q4_K lane reaches both quant planes by one 32-bit offset from its row tile in the first, but where a plane ends just
+// short of 4 GiB (the most sdy_gemm_ok takes): the FAR form.
 static bool gemm_far(const GemmArgs &g) { return (size_t)(g.p[1] - g.p[0]) + (size_t)g.T * 4096 > 0xFFFFFFFFu; }
 
-template <int WT, int RW, int KS, int NT = 1>
+template <int WT, int RW, int KS, int NT = 1, bool FAR = false>
 static int launch_gemm(const GemmArgs &g, unsigned tok_tiles, hipStream_t st) {
     constexpr size_t lds = gemm_lds_bytes<RW, KS, NT>();
     static size_t granted = 0;
-    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS, NT>, lds, &granted)) return rc;
-    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS, NT>));
-    hipLaunchKernelGGL((k_gemm<WT, RW, KS, NT>), dim3((tok_tiles + NT - 1) / NT, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))),
+    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS, NT, FAR>, lds, &granted)) return rc;
+    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS, NT, FAR>));
+    hipLaunchKernelGGL((k_gemm<WT, RW, KS, NT, FAR>), dim3((tok_tiles + NT - 1) / NT, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))),
                        dim3(64 * RW * KS), lds, st, g);
     return sdy_check_launch("gemm");
 }
@@ -703,7 +707,7 @@ extern "C" int sdy_gemm(const sdy_mat *m, const sdy_mv_args *a, void *ws, sdy_st
     bool empty;
     if (int rc = gemm_setup(m, a, ws, st, g, &empty)) return rc;
     if (empty) return 0;
-    if (gemm_far(g)) return sdy_matvec(m, a, s);
+    if (m->type == SDY_Q4_K && gemm_far(g)) return launch_gemm<SDY_Q4_K, 4, 1, 1, true>(g, (unsigned)((g.n_tok + 31) / 32), st);
     return m->type == SDY_Q4_K ? gemm_type<SDY_Q4_K>(g, m, a, st) : gemm_type<SDY_Q6_K>(g, m, a, st);
 }
 
@@ -741,7 +745,9 @@ extern "C" int sdy_gemm2(const sdy_mat *m1, const sdy_mv_args *a1, const sdy_mat
     if (int rc = gemm_setup(m1, a1, ws, st, g1, &e1)) return rc;  // (both ranges non-empty here)
     if (int rc = gemm_setup(m2, &b, ws, st, g2, &e2)) return rc;
     if (gemm_far(g1)) {
-        if (int rc = sdy_matvec(m1, a1, s)) return rc;
+        sdy_mv_args a = *a1;
+        a.ws_ready = 1;
+        if (int rc = sdy_gemm(m1, &a, ws, s)) return rc;
         return sdy_gemm(m2, &b, ws, s);
     }
     // (384 + 128 rows x 256, 64 tokens: 3.5 us, four waves to a tile 7.4; 768 + 256 x 512: 3.8 against 6.6)
@@ -772,7 +778,6 @@ extern "C" int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, cons
                             "caller made (ws_ready)");
     GemmArgs g = gemm_args(m, true);
     if (int rc = gemm_expand(a, act_row ? n_act : n_tok, g.n_in, ws, g.e, st)) return rc;
-    if (gemm_far(g)) return sdy_fail(-1, "gemm_grouped: quant planes of 4 GiB");
     g.row0 = 0;
     g.n_rows = grp_rows;
     g.n_tok = n_tok;
@@ -789,6 +794,7 @@ extern "C" int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, cons
     g.n_grp = n_grp;
     // token tiles: at most one partial tile per group beyond the full ones (the grid's extra workgroups return at once)
     const unsigned tok_tiles = (unsigned)((n_tok + 31) / 32 + n_grp - 1);
+    if (m->type == SDY_Q4_K && gemm_far(g)) return launch_gemm<SDY_Q4_K, 4, 1, 1, true>(g, tok_tiles, st);
     const char *ev = getenv("SARDYNE_GEMM_VARIANT");
     const int v = ev ? atoi(ev) : 0;
     if (v == 12) return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 2, 2>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 2, 2>(g, tok_tiles, st);

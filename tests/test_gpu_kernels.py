@@ -1729,8 +1729,121 @@ def test_gemm2_short_rows_bit_exact(n_in, rows1, rows2, n_tok, pair):
             assert np.array_equal(bits(d[i].to_array(np.float32, (n_tok, r))), bits(exp[i]))
 
 
-@pytest.mark.parametrize("variant,kernel", [("11", "k_gemm<%d, 4, 1, 1>"), ("12", "k_gemm<%d, 2, 2, 1>"), ("13", "k_gemm<%d, 2, 4, 1>"),
-                                            ("14", "k_mm_superblocks<%d, "), ("15", "k_gemm<%d, 4, 1, 2>")])
+@pytest.mark.parametrize("layout", [False, True], ids=["planes", "tiled"])
+def test_q4k_planes_of_4_gib(layout):
+    """The largest Q4_K matrix the GEMM takes (its quant planes end where the second begins 4 GiB after the first), zero but
+    for a few rows at both ends: the GEMM over a row range at the end, the grouped GEMM over its first and last groups,
+    the pair with a small Q6_K matrix, and the matvecs of 2 to 9 tokens with their epilogues (the matrix-core kernel of a few
+    tokens does not reach such a matrix): the oracle's bits."""
+    L = lib()
+    n_in, n_rows = 256, (1 << 26) - 1
+    n_tok, grp_rows, n_grp, n_set = 40, 8128, 8256, 150
+    m = capi.SdyMat()
+    capi.check(L.sdy_mat_alloc(ctypes.byref(m), O.Q4_K, n_in, n_rows))
+    assert m.plane_off[1] - m.plane_off[0] == 1 << 32
+    try:
+        starts = (0, grp_rows * n_grp - n_set, n_rows - n_set)  # (the last group ends before the matrix does)
+        w = [_full_range_blocks("Q4_K", n_set, n_in, i) for i in range(3)]
+        for r0, x in zip(starts, w):
+            capi.check(L.sdy_mat_upload_rows(ctypes.byref(m), r0, 1, n_set, x.ctypes.data, None))
+        if layout:
+            capi.check(L.sdy_mat_gemm_layout(ctypes.byref(m), None))
+        assert L.sdy_gemm_ok(ctypes.byref(m), n_tok) and bool(m.gbase) == layout
+        xq = O.quantize(np.random.default_rng(1).standard_normal((n_tok, n_in)).astype(np.float32), O.Q8_K)
+        exp = [O.matmul_q(x, O.Q4_K, xq, n_in, simd=1) for x in w]
+        dq, ws = capi.DeviceBuffer.from_array(xq), capi.DeviceBuffer(L.sdy_gemm_ws_bytes(n_tok, n_in))
+        view = L.sdy_mat_rows(ctypes.byref(m), n_rows - n_set - 5, n_set + 5)  # (the whole matrix' copy and planes)
+
+        # the end of the matrix, by row range
+        last = n_rows - n_set
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, n_set), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr - 4 * last, out_stride=n_set, row0=last, row1=n_rows)
+        capi.check(L.sdy_gemm(ctypes.byref(m), ctypes.byref(a), ws.ptr, None))
+        assert b"true>" in L.sdy_last_kernel()
+        assert np.array_equal(bits(out.to_array(np.float32, (n_tok, n_set))), bits(exp[2]))
+
+        # two groups of 10 and 30 tokens
+        cnt = np.zeros(n_grp, np.int64)
+        cnt[0], cnt[-1] = 10, 30
+        tok = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+        tile = np.concatenate([[0], np.cumsum((cnt + 31) // 32)]).astype(np.int32)
+        dtok, dtile = capi.DeviceBuffer.from_array(tok), capi.DeviceBuffer.from_array(tile)
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, grp_rows), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=grp_rows, row0=0, row1=grp_rows)
+        capi.check(L.sdy_gemm_grouped(ctypes.byref(m), grp_rows, n_grp, dtok.ptr, dtile.ptr, None, None, 0, ctypes.byref(a), ws.ptr, None))
+        got = out.to_array(np.float32, (n_tok, grp_rows))
+        assert np.array_equal(bits(got[:10, :n_set]), bits(exp[0][:10]))
+        assert np.array_equal(bits(got[10:, grp_rows - n_set:]), bits(exp[1][10:]))
+        assert not got[:10, n_set:].any() and not got[10:, :grp_rows - n_set].any()
+
+        # with a Q6_K matrix on the same activations
+        w6 = _full_range_blocks("Q6_K", 70, n_in, 9)
+        m6 = capi.DeviceMatrix(O.Q6_K, n_in, 70, w6)
+        o1, o2 = capi.DeviceBuffer(n_tok * n_set * 4), capi.DeviceBuffer(n_tok * 70 * 4)
+        a1 = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=o1.ptr - 4 * last, out_stride=n_set, row0=last, row1=n_rows)
+        a2 = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=o2.ptr, out_stride=70, row0=0, row1=70)
+        capi.check(L.sdy_gemm2(ctypes.byref(m), ctypes.byref(a1), ctypes.byref(m6.m), ctypes.byref(a2), ws.ptr, None))
+        assert np.array_equal(bits(o1.to_array(np.float32, (n_tok, n_set))), bits(exp[2]))
+        assert np.array_equal(bits(o2.to_array(np.float32, (n_tok, 70))), bits(O.matmul_q(w6, O.Q6_K, xq, n_in, simd=1)))
+
+        # a few tokens: the matvecs, over the view's last rows
+        resid = np.random.default_rng(2).standard_normal((n_tok, n_set + 5)).astype(np.float32)
+        dr = capi.DeviceBuffer.from_array(resid)
+        for n in (2, 3, 5, 8, 9):
+            out = capi.DeviceBuffer.from_array(np.full((n, n_set + 5), np.nan, np.float32))
+            a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n, out=out.ptr, out_stride=n_set + 5, row0=5, row1=n_set + 5, resid=dr.ptr)
+            capi.check(L.sdy_matvec(ctypes.byref(view), ctypes.byref(a), None))
+            assert b"k_mm_superblocks" not in L.sdy_last_kernel()
+            got = out.to_array(np.float32, (n, n_set + 5))
+            assert np.array_equal(bits(got[:, 5:]), bits(resid[:n, 5:] + exp[2][:n])) and np.all(np.isnan(got[:, :5]))
+            a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n, out=out.ptr, out_stride=n_set // 2, row0=last + 1, row1=n_rows, epilogue=capi.EPI_SWIGLU)
+            a.row0 = last + (last & 1)  # (an even row)
+            a.row1 = n_rows - (n_rows & 1)
+            capi.check(L.sdy_matvec(ctypes.byref(m), ctypes.byref(a), None))
+            k = a.row0 - last
+            g, u = exp[2][:n, k:n_set - 1 + k:2].copy(), exp[2][:n, k + 1:n_set:2].copy()
+            g = g[:, :u.shape[1]].copy()
+            L.op_silu_mul(ptr(g), ptr(u), g.size)
+            pairs = (a.row1 - a.row0) // 2
+            got = out.to_array(np.float32, n * (n_set + 5))[:n * (n_set // 2)].reshape(n, n_set // 2)
+            assert np.array_equal(bits(got[:, :pairs]), bits(g[:, :pairs]))
+    finally:
+        L.sdy_mat_free(ctypes.byref(m))
+
+
+@pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
+def test_block_matrix_beyond_4_gib(kind):
+    """A matrix of more than 4 GiB, which the matrix-core kernel's 32-bit offsets do not reach, zero but for its last rows:
+    nine tokens take the matvecs, with the bits of one token at a time."""
+    L = lib()
+    t, n_in, n_set, n_tok = TYPES[kind], 64, 70, 9
+    n_rows = (1 << 32) // (L.sdy_mat_bytes(t, n_in, 1 << 20) >> 20) + 1000
+    m = capi.SdyMat()
+    capi.check(L.sdy_mat_alloc(ctypes.byref(m), t, n_in, n_rows))
+    try:
+        assert m.bytes >= (1 << 32) - 1
+        _, w, xq = _matvec_case(kind, n_in, n_set, n_tok, seed=5)
+        last = n_rows - n_set
+        capi.check(L.sdy_mat_upload_rows(ctypes.byref(m), last, 1, n_set, w.ctypes.data, None))
+        dq, got = capi.DeviceBuffer.from_array(xq), []
+        small = capi.DeviceMatrix(t, n_in, n_set, w)
+        for n, first in [(n_tok, 0)] + [(1, i) for i in range(n_tok)]:
+            out = capi.DeviceBuffer(n * n_set * 4)
+            a = capi.SdyMvArgs(xq=dq.ptr + first * 68, n_tok=n, out=out.ptr - 4 * last, out_stride=n_set, row0=last, row1=n_rows)
+            capi.check(L.sdy_matvec(ctypes.byref(m), ctypes.byref(a), None))
+            assert b"k_mm_blocks" not in L.sdy_last_kernel()
+            got.append(out.to_array(np.float32, (n, n_set)))
+            if n == 1:
+                a = capi.SdyMvArgs(xq=dq.ptr + first * 68, n_tok=1, out=out.ptr, out_stride=n_set, row0=0, row1=n_set)
+                capi.check(L.sdy_matvec(ctypes.byref(small.m), ctypes.byref(a), None))
+                assert np.array_equal(bits(got[-1]), bits(out.to_array(np.float32, (1, n_set))))
+                assert np.array_equal(bits(got[-1][0]), bits(got[0][first]))
+    finally:
+        L.sdy_mat_free(ctypes.byref(m))
+
+
+@pytest.mark.parametrize("variant,kernel", [("11", "k_gemm<%d, 4, 1, 1,"), ("12", "k_gemm<%d, 2, 2, 1,"), ("13", "k_gemm<%d, 2, 4, 1,"),
+                                            ("14", "k_mm_superblocks<%d, "), ("15", "k_gemm<%d, 4, 1, 2,")])
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 def test_gemm_tile_variants_bit_exact(kind, variant, kernel, monkeypatch):
     """Every form of the GEMM (forced through SARDYNE_GEMM_VARIANT: one, two or four waves to a tile's super-blocks, the 16 x 16
