@@ -145,7 +145,9 @@ SDY_DEV f32x16 mfma_split(const Frag<NA> &a, const Frag<3> &b, f32x16 c) {
 }
 
 // One block. SPLIT: the products on the bf16 matrix cores, from fragments; else on the f32 ones. Returns, the same for
-// all threads, whether (SPLIT) some sum is NaN; nothing is written then.
+// all threads, whether (SPLIT) the fragments may not have held the values; nothing is written then: some sum is infinite or
+// NaN, or is so small (below 2^-90, but not 0) that a whole column of values may be below 2^-110, whose last fragments bf16
+// does not hold. (A column of nothing but values below 2^-134, half of bf16's least, counts as zeros.)
 template <int HD, class KT, int MS, bool SPLIT>
 SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
     using LY = FlashLds<HD, MS>;
@@ -303,12 +305,17 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
     }
 
     if constexpr (SPLIT) {
-        int nan = l_run != l_run;
+        float z = 0.0f * l_run;  // NaN from an infinity or a NaN on
+        uint32_t least = ~0u;    // the least |o| but 0, its bits shifted and less one
 #pragma unroll
         for (int dt = 0; dt < ND; dt++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) nan |= o[dt][e] != o[dt][e];
-        if (__syncthreads_or(nan)) return true;
+            for (int e = 0; e < 16; e++) {
+                z = __builtin_fmaf(0.0f, o[dt][e], z);
+                const uint32_t u = (__float_as_uint(o[dt][e]) << 1) - 1;
+                least = u < least ? u : least;
+            }
+        if (__syncthreads_or(z != z || least < (127u - 90u) << 24)) return true;
     }
     // merge of the waves' partials in wave order (the Q^T area is reused), in MS parts of the dims:
     // part x holds the O columns dt in [x NDH, (x + 1) NDH), dims ND * row + dt, at NDH * row + dt - x NDH
@@ -353,7 +360,8 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
 template <int HD, class KT, int MS>
 __global__ __launch_bounds__(64 * FW) void k_attn_flash(FlashArgs a) {
     extern __shared__ __align__(16) float lds[];
-    // (an infinity's fragments are NaN, so a block that met one, or a value beyond bf16's largest, is computed again)
+    // (an infinity's fragments are NaN, so a block that met one, or a value beyond bf16's largest, is computed again; so is
+    // one with a column of values too small for theirs)
     if (flash_block<HD, KT, MS, true>(a, lds)) flash_block<HD, KT, MS, false>(a, lds);
 }
 

@@ -1155,6 +1155,30 @@ def test_prefill_attention_flash_reads_no_row_past_the_last(hd, tail, kv):
     assert np.array_equal(bits(got[1]), bits(got[0]))
 
 
+@pytest.mark.parametrize("hd,n_tok,n_kv0", [(128, 33, 1), (64, 70, 40), (128, 40, 300)])
+@pytest.mark.parametrize("exp2", [-100, -112, -120, -126, -131])
+def test_prefill_attention_flash_tiny_values(hd, n_tok, n_kv0, exp2):
+    """V columns of very small magnitude beside ordinary ones, where the third (and second) bf16 of a value is below
+    the type's range: the reference's arithmetic to 1e-5 of each column's scale, the bound of the ordinary values, and a
+    unit of the smallest f32 per position."""
+    L = lib()
+    n_head, n_kv_head, max_seq = 4, 2, n_kv0 + n_tok + 3
+    rng = np.random.default_rng(hd + n_tok)
+    q = rng.standard_normal((n_tok, n_head * hd)).astype(np.float32)
+    kc, vc = (rng.standard_normal((n_kv_head, max_seq, hd)).astype(np.float32) for _ in range(2))
+    vc[:, :, ::5] = (vc[:, :, ::5].astype(np.float64) * 2.0 ** exp2).astype(np.float32)
+    vc[1, :, 7] = 0.0
+    dq, dk, dv = (capi.DeviceBuffer.from_array(a) for a in (q, kc, vc))
+    dpart = capi.DeviceBuffer(L.sdy_attn_scores_floats(n_tok, n_head, max_seq) * 4)
+    outs = [capi.DeviceBuffer(q.nbytes) for _ in range(2)]
+    capi.check(L.sdy_attention(dq.ptr, dk.ptr, dv.ptr, capi.KV_F32, n_tok, n_head, n_kv_head, hd, n_kv0, max_seq * hd,
+                               n_head * hd, dpart.ptr, outs[0].ptr, n_head * hd, None))
+    capi.check(L.sdy_attention_flash(dq.ptr, dk.ptr, dv.ptr, capi.KV_F32, n_tok, n_head, n_kv_head, hd, n_kv0, max_seq * hd,
+                                     n_head * hd, outs[1].ptr, n_head * hd, None))
+    exp, got = (o.to_array(np.float32, q.shape).astype(np.float64) for o in outs)
+    assert np.all(np.abs(got - exp) <= 1e-5 * np.abs(exp).max(axis=0) + max_seq * 2.0 ** -149)
+
+
 def test_prefill_attention_flash_rejects_layouts():
     """head_dim other than 64 / 128, GQA groups that do not divide, unaligned q rows: an error, no launch."""
     L = lib()
