@@ -380,11 +380,12 @@ static int mm_type(const MmArgs &g, hipStream_t st) {
 }
 
 // The tokens of a->xq through rows [a->row0, a->row1) of m (Q8_0, Q4_0, Q5_0), as sdy_matvec. Returns 1, launching
-// nothing, when the kernel's 32-bit offsets do not reach every byte of the matrix or the activations, or the rows are
-// not 2-byte aligned.
+// nothing, when the kernel's 32-bit offsets do not reach every byte of the matrix or the activations, a grid's 65535
+// row tiles every row of the matrix, or the rows are not 2-byte aligned.
 extern "C" int sdy_mm_blocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream s) {
     const size_t row_bytes = (size_t)(m->n_in / 32) * 34, lim = 0xFFFFFFFFu;
-    if (m->bytes >= lim || m->gbytes >= lim || row_bytes * a->n_tok >= lim || ((uintptr_t)a->xq & 1)) return 1;
+    if (m->bytes >= lim || m->gbytes >= lim || row_bytes * a->n_tok >= lim || ((uintptr_t)a->xq & 1) || m->n_rows > 65535L * 32)
+        return 1;
     MmArgs g = {};
     for (int i = 0; i < 5; i++) g.p[i] = (const uint8_t *)m->base + m->plane_off[i];
     if (m->gbase) {

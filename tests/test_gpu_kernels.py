@@ -1835,6 +1835,34 @@ def test_q4k_planes_of_4_gib(layout):
         L.sdy_mat_free(ctypes.byref(m))
 
 
+@pytest.mark.parametrize("more", [0, 1])
+def test_block_matrix_of_most_rows(more):
+    """The most rows a grid of the matrix-core kernel has row tiles for, and one more, which takes the matvecs: the last
+    rows against float64 (the bound of the many-token test), over the whole matrix and over their row range the same bits."""
+    L = lib()
+    t, n_in, n_rows, n_tok, n_set = O.Q4_0, 32, 65535 * 32 + more, 9, 40
+    m = capi.SdyMat()
+    capi.check(L.sdy_mat_alloc(ctypes.byref(m), t, n_in, n_rows))
+    try:
+        _, w, xq = _matvec_case("Q4_0", n_in, n_set, n_tok, seed=6)
+        last = n_rows - n_set
+        capi.check(L.sdy_mat_upload_rows(ctypes.byref(m), last, 1, n_set, w.ctypes.data, None))
+        dq, got = capi.DeviceBuffer.from_array(xq), []
+        for r0, n in ((0, n_rows), (last, n_set)):
+            out = capi.DeviceBuffer(n_tok * n * 4)
+            a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr - 4 * r0, out_stride=n, row0=r0, row1=n_rows)
+            capi.check(L.sdy_matvec(ctypes.byref(m), ctypes.byref(a), None))
+            assert (b"k_mm_blocks" in L.sdy_last_kernel()) == (more == 0)
+            got.append(out.to_array(np.float32, (n_tok, n))[:, n - n_set:])
+        xb = xq.reshape(n_tok, 34)
+        x = xb[:, 2:].copy().view(np.int8).astype(np.float64) * xb[:, :2].copy().view(np.float16).astype(np.float64)
+        exp = x @ O.dequant(w, t, n_in * n_set).astype(np.float64).reshape(n_set, n_in).T
+        assert np.all(np.abs(got[0] - exp) <= 13 * 2.0 ** -24 * np.abs(exp) + 1e-45)
+        assert np.array_equal(bits(got[1]), bits(got[0]))
+    finally:
+        L.sdy_mat_free(ctypes.byref(m))
+
+
 @pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
 def test_block_matrix_beyond_4_gib(kind):
     """A matrix of more than 4 GiB, which the matrix-core kernel's 32-bit offsets do not reach, zero but for its last rows:
