@@ -802,6 +802,10 @@ engine_ctx *engine_ctx_new(const engine_model *m, int32_t max_seq, int32_t n_bat
     c->moe_device = c->decode_fused && !env_on("SARDYNE_NO_DEVICE_MOE") && sdy_engine_moe_device_ok(c);
     c->use_graph = c->decode_fused && (!m->info.n_expert || c->moe_device) && !env_on("SARDYNE_NO_GRAPH");
     c->fuse_act = c->decode_fused && !env_on("SARDYNE_NO_FUSED_ACT");
+    /* SARDYNE_BLOCK_MATVEC: several tokens of Q8_0 / Q4_0 / Q5_0 weights four at a time through the matvec, which
+       adds a row's blocks as the one-token steps do; default: larger matrices and more tokens on the matrix cores,
+       in another order (within tolerance) */
+    c->block_matvec = env_on("SARDYNE_BLOCK_MATVEC");
     const engine_model_info *in = &m->info;
     /* the split forms take the fused one-token step and their head layouts; otherwise the exact chain */
     if (!c->decode_fused || (c->attn_mode == SDY_ATTN_CHUNKED && !sdy_attn_chunked_ok(in->n_head, in->n_kv_head,

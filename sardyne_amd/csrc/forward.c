@@ -194,6 +194,17 @@ static int mm_epi(engine_ctx *c, float *out, const float *x, const dmat *w, int 
             gemm_record(c, a.xq, n_tok, w->n_in);
             return 0;
         }
+        if (c->block_matvec && vt == SDY_Q8_0) { /* four tokens at a time: the bits of one */
+            for (int t = 0; t < n_tok; t += 4) {
+                sdy_mv_args b = a;
+                b.n_tok = n_tok - t < 4 ? n_tok - t : 4;
+                b.xq = (const uint8_t *)a.xq + (size_t)t * (w->n_in / 32) * 34;
+                b.out = a.out + t * a.out_stride;
+                b.resid = a.resid ? a.resid + t * a.out_stride : NULL;
+                TRY(sdy_matvec(&w->m, &b, c->st));
+            }
+            return 0;
+        }
     }
     return sdy_matvec(&w->m, &a, c->st);
 }

@@ -74,6 +74,7 @@ struct engine_ctx {
     int attn_mode;              /* one-token attention: SDY_ATTN_EXACT (the reference's bits), or split
                                    over positions within tolerance: SDY_ATTN_CHUNKED (two launches),
                                    SDY_ATTN_SPLIT (one launch) */
+    int block_matvec;           /* several tokens of Q8_0 / Q4_0 / Q5_0 weights with the bits of one at a time */
     int prefill_flash;          /* many-token attention in flash form (sdy_attention_flash), within tolerance */
     float *attn_part;           /* chunked / split attention: per-span partials */
     unsigned *attn_count;       /* split attention: arrivals per kv head (zero between launches) */

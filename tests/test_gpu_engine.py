@@ -241,6 +241,23 @@ def test_decode_paths_bit_identical(model_path):
     assert_close(fused_graph, np.stack(exp))
 
 
+@pytest.mark.parametrize("n", [5, 9, 33])
+def test_block_matvec_prompt_has_the_one_token_bits(tmp_path, n):
+    """SARDYNE_BLOCK_MATVEC=1 with the exact attention: a prompt of a Q8_0 / Q4_0 / Q5_0 model leaves the logits that feeding
+    its tokens one at a time leaves, bit for bit; without it they agree within the tolerance of the models' tests."""
+    path = tmp_path / "m.gguf"
+    write_model(path, SPECS["qwen2-q0"], seed=9)
+    model = LoadedModel(path)
+    toks = np.random.default_rng(n).integers(0, 300, n).tolist()
+    with engine_env(SARDYNE_ATTENTION="exact", SARDYNE_BLOCK_MATVEC="1"):
+        whole, single = model.session(max_seq=64, n_batch=64), model.session(max_seq=64, n_batch=64)
+    with engine_env(SARDYNE_ATTENTION="exact"):
+        default = model.session(max_seq=64, n_batch=64)
+    got, exp = whole.feed(toks), [single.feed([t]) for t in toks][-1]
+    assert np.array_equal(got.view(np.uint32), exp.view(np.uint32))
+    assert_close(default.feed(toks), got)
+
+
 KQUANT_SPECS = ["qwen2-kquant", "llama-kquant", "qwen2-gqa8-hd128", "moe-128x8", "moe-16x4-ffn768", "moe-192x6",
                 "qwen2-kquant-v4k", "qwen2-kquant-vmix"]
 
