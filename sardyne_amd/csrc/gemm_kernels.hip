@@ -76,8 +76,10 @@ constexpr size_t gemm_lds_bytes() { return 2 * (size_t)(32 * NT * 292 * KS) + (K
 // 64 banks once). The weights go straight to registers, each lane (row lr, k-half h) loading its own records, and
 // are reloaded for the next stage as they are used: from the tiled copy a load instruction reads runs of 512
 // bytes. The workgroup's place in the grid is (bx, by) of (gx, gy): a pair launch gives each matrix a part of one grid.
-// FAR: Q4_K planes too far apart for a lane to reach both by a 32-bit offset: 64-bit addresses.
-template <int WT, int RW, int KS, int NT, bool FAR>
+// ALT, another way to the weights. Q4_K: planes too far apart for a lane to reach both by a 32-bit offset, by 64-bit
+// addresses. Q6_K: the planes, where a lane's 8 bytes of a unit are half of a 16-byte record in a cache line per row: it
+// loads a whole record of every second unit, and the two lanes of a row swap halves.
+template <int WT, int RW, int KS, int NT, bool ALT>
 SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_t *lds) {
     constexpr bool Q4 = WT == SDY_Q4_K;
     static_assert(NT == 1 || KS == 1, "token tiles share a wave's weights only where it has the row tile to itself");
@@ -132,23 +134,33 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
     const int us = g.blk ? 512 : 16, ss = g.blk ? 32 : 1;
     const __amdgpu_buffer_rsrc_t r0 = rsrc(g.p[0] + ub * 16), r1 = rsrc(g.p[1] + ub * 16),
                                  r2 = rsrc(g.p[2] + (Q4 ? sb0 : ub) * 16), r3 = rsrc(g.p[3] + sb0 * 16), r4 = rsrc(g.p[4] + sb0 * 2);
-    // (Q4_K: lane half h reads plane h; Q6_K: bytes 8 h .. of each plane's record)
-    const uint32_t vq = vu + (Q4 ? (h ? (uint32_t)(g.p[1] - g.p[0]) : 0u) : 8u * (uint32_t)h);
+    // (Q4_K: lane half h reads plane h; Q6_K: bytes 8 h .. of each plane's record, ALT: the record of unit 2 p + h)
+    const uint32_t vq = vu + (Q4 ? (h ? (uint32_t)(g.p[1] - g.p[0]) : 0u) : (ALT ? (uint32_t)us : 8u) * (uint32_t)h);
     const uint8_t *const vfar = (h ? g.p[1] : g.p[0]) + ub * 16 + vu;
     u32x4 w4[Q4 ? 4 : 1], sc;
-    u32x2 w6[Q4 ? 1 : 4][3];
+    u32x4 w6[Q4 ? 1 : 2][3];  // of units 2 p and 2 p + 1, eight bytes of each (ALT: as loaded, before the swap)
     uint32_t d6 = 0;
     auto sb_of = [&](int s) { return s * KS + ks < nb ? s * KS + ks : nb - 1; };  // (past the end: not added)
     auto load_u = [&](int s, int u) {
         const int so = (4 * sb_of(s) + u) * us;
-        if constexpr (Q4 && FAR) {
+        if constexpr (Q4 && ALT) {
             w4[u] = *reinterpret_cast<const u32x4 *>(vfar + so);
         } else if constexpr (Q4) {
             w4[u] = __builtin_amdgcn_raw_buffer_load_b128(r0, vq, so, 0);
+        } else if constexpr (ALT) {
+            if (u & 1) {
+                const int sp = so - us;
+                w6[u >> 1][0] = __builtin_amdgcn_raw_buffer_load_b128(r0, vq, sp, 0);
+                w6[u >> 1][1] = __builtin_amdgcn_raw_buffer_load_b128(r1, vq, sp, 0);
+                w6[u >> 1][2] = __builtin_amdgcn_raw_buffer_load_b128(r2, vq, sp, 0);
+            }
         } else {
-            w6[u][0] = bload8(r0, vq, so);
-            w6[u][1] = bload8(r1, vq, so);
-            w6[u][2] = bload8(r2, vq, so);
+            const u32x2 x[3] = {bload8(r0, vq, so), bload8(r1, vq, so), bload8(r2, vq, so)};
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                w6[u >> 1][i][2 * (u & 1)] = x[i][0];
+                w6[u >> 1][i][2 * (u & 1) + 1] = x[i][1];
+            }
         }
     };
     auto load_s = [&](int s) {
@@ -267,7 +279,20 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
             auto issue = [&](int j, int nt, i32x16 &p) {  // sub-block j = 4 u + k: elements 16 k .. of unit u, stored 32 too high
                 const int u = j >> 2, k = j & 3;
                 if (nt == 0) {
-                    const u32x2 nn = w6[u][k & 1], hb = w6[u][2];
+                    if constexpr (ALT) {
+                        if (k == 0 && !(u & 1)) {  // dwords 2, 3 of the first lane's unit for 0, 1 of the second's
+#pragma unroll
+                            for (int i = 0; i < 3; i++)
+#pragma unroll
+                                for (int e = 0; e < 2; e++) {
+                                    const auto x = __builtin_amdgcn_permlane32_swap(w6[u >> 1][i][e], w6[u >> 1][i][e + 2], false, false);
+                                    w6[u >> 1][i][e] = x[0];
+                                    w6[u >> 1][i][e + 2] = x[1];
+                                }
+                        }
+                    }
+                    auto unit = [&](int i) { return u & 1 ? u32x2{w6[u >> 1][i][2], w6[u >> 1][i][3]} : u32x2{w6[u >> 1][i][0], w6[u >> 1][i][1]}; };
+                    const u32x2 nn = unit(k & 1), hb = unit(2);
                     const u32x2 lo = (k & 2) ? (nn >> 4u) & 0x0F0F0F0Fu : nn & 0x0F0F0F0Fu;
                     const u32x2 hi = k == 0 ? (hb & 0x03030303u) << 4u : k == 1 ? (hb & 0x0C0C0C0Cu) << 2u
                                      : k == 2 ? hb & 0x30303030u : (hb >> 2u) & 0x30303030u;
@@ -371,10 +396,10 @@ SDY_DEV void gemm_body(const GemmArgs &g, int bx, int by, int gx, int gy, uint8_
     }
 }
 
-template <int WT, int RW, int KS, int NT, bool FAR>
+template <int WT, int RW, int KS, int NT, bool ALT>
 __global__ __launch_bounds__(64 * RW * KS, NT == 1 ? 3 : 2) void k_gemm(GemmArgs g) {
     extern __shared__ __align__(16) uint8_t lds[];
-    gemm_body<WT, RW, KS, NT, FAR>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
+    gemm_body<WT, RW, KS, NT, ALT>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.x, (int)gridDim.y, lds);
 }
 
 // Two GEMMs on the same activations in one launch (a layer's q|k and a v of another type): row tiles [0, gy1) of
@@ -596,13 +621,13 @@ extern "C" int sdy_gemm_ok(const sdy_mat *m, int n_tok) {
 // short of 4 GiB (the most sdy_gemm_ok takes): the FAR form.
 static bool gemm_far(const GemmArgs &g) { return (size_t)(g.p[1] - g.p[0]) + (size_t)g.T * 4096 > 0xFFFFFFFFu; }
 
-template <int WT, int RW, int KS, int NT = 1, bool FAR = false>
+template <int WT, int RW, int KS, int NT = 1, bool ALT = false>
 static int launch_gemm(const GemmArgs &g, unsigned tok_tiles, hipStream_t st) {
     constexpr size_t lds = gemm_lds_bytes<RW, KS, NT>();
     static size_t granted = 0;
-    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS, NT, FAR>, lds, &granted)) return rc;
-    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS, NT, FAR>));
-    hipLaunchKernelGGL((k_gemm<WT, RW, KS, NT, FAR>), dim3((tok_tiles + NT - 1) / NT, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))),
+    if (int rc = sdy_lds_limit((const void *)k_gemm<WT, RW, KS, NT, ALT>, lds, &granted)) return rc;
+    SDY_NOTE_KERNEL((k_gemm<WT, RW, KS, NT, ALT>));
+    hipLaunchKernelGGL((k_gemm<WT, RW, KS, NT, ALT>), dim3((tok_tiles + NT - 1) / NT, (unsigned)((g.n_rows + 32 * RW - 1) / (32 * RW))),
                        dim3(64 * RW * KS), lds, st, g);
     return sdy_check_launch("gemm");
 }
@@ -623,8 +648,8 @@ static int launch_gemm(const GemmArgs &g, unsigned tok_tiles, hipStream_t st) {
 //   against 59.9), where the last pair of tiles is whole or one of several (65536 x 2048, 96 tokens: 72 against 84). Q4_K's
 //   nibbles cost less than the third wave (22016 x 2048, 512 tokens: 70.4 against 83.9).
 // - From the planes, where a wave's load of 32 rows' units meets as many cache lines: two token tiles as soon as they
-//   fill the chip (22016 x 2048, 512 tokens: Q6_K 176 -> 131 us, Q4_K 107 -> 89), two waves before (Q4_K 22016 x 8192, 96
-//   tokens: 111 -> 82).
+//   fill the chip (22016 x 2048, 512 tokens: Q6_K 176 -> 131 us, with whole records loaded 120; Q4_K 107 -> 89), two waves
+//   before (Q4_K 22016 x 8192, 96 tokens: 111 -> 82).
 static int gemm_form(const sdy_mat *m, long n_rows, int n_tok) {
     const int nb = m->n_in / 256;
     const bool q4 = m->type == SDY_Q4_K, tiled = m->gbase != nullptr, few = nb <= (q4 ? 2 : tiled ? 3 : 4);
@@ -643,6 +668,13 @@ static int gemm_form(const sdy_mat *m, long n_rows, int n_tok) {
     return t32 < 512 ? 4 : t32 < 2048 ? 2 : 1;
 }
 
+template <int WT, bool ALT>
+static int launch_form(const GemmArgs &g, int form, unsigned tok_tiles, hipStream_t st) {
+    if (form == 12) return launch_gemm<WT, 4, 1, 2, ALT>(g, tok_tiles, st);
+    if (form == 4) return launch_gemm<WT, 2, 4, 1, ALT>(g, tok_tiles, st);
+    return form == 2 ? launch_gemm<WT, 2, 2, 1, ALT>(g, tok_tiles, st) : launch_gemm<WT, 4, 1, 1, ALT>(g, tok_tiles, st);
+}
+
 template <int WT>
 static int gemm_type(const GemmArgs &g, const sdy_mat *m, const sdy_mv_args *a, hipStream_t st) {
     // SARDYNE_GEMM_VARIANT picks one form (tests and tuning): 11, 12, 13: one, two, four waves; 14: 16 x 16 tiles; 15: two
@@ -657,9 +689,8 @@ static int gemm_type(const GemmArgs &g, const sdy_mat *m, const sdy_mv_args *a, 
         if (rc <= 0) return rc;
         form = 4;
     }
-    if (form == 12) return launch_gemm<WT, 4, 1, 2>(g, tt, st);
-    if (form == 4) return launch_gemm<WT, 2, 4>(g, tt, st);
-    return form == 2 ? launch_gemm<WT, 2, 2>(g, tt, st) : launch_gemm<WT, 4, 1>(g, tt, st);
+    if (WT == SDY_Q6_K && !g.blk) return launch_form<WT, WT == SDY_Q6_K>(g, form, tt, st);
+    return launch_form<WT, false>(g, form, tt, st);
 }
 
 // The activations' expansion of one call in ws: made unless ws_ready.
@@ -797,7 +828,9 @@ extern "C" int sdy_gemm_grouped(const sdy_mat *m, long grp_rows, int n_grp, cons
     if (m->type == SDY_Q4_K && gemm_far(g)) return launch_gemm<SDY_Q4_K, 4, 1, 1, true>(g, tok_tiles, st);
     const char *ev = getenv("SARDYNE_GEMM_VARIANT");
     const int v = ev ? atoi(ev) : 0;
-    if (v == 12) return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 2, 2>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 2, 2>(g, tok_tiles, st);
-    if (v == 13) return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 2, 4>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 2, 4>(g, tok_tiles, st);
-    return m->type == SDY_Q4_K ? launch_gemm<SDY_Q4_K, 4, 1>(g, tok_tiles, st) : launch_gemm<SDY_Q6_K, 4, 1>(g, tok_tiles, st);
+    // One wave to a row tile; from the planes, whose loads take longer, two where rows have eight super-blocks for them (128
+    // groups of 1536 rows x 2048, 512 tokens: Q4_K 71 -> 62 us, Q6_K 107 -> 99; 32 tokens 28 -> 19 and 37 -> 24)
+    const int form = v ? (v == 12 ? 2 : v == 13 ? 4 : 1) : !g.blk && !m->hbase && g.nb >= 8 ? 2 : 1;
+    if (m->type == SDY_Q4_K) return launch_form<SDY_Q4_K, false>(g, form, tok_tiles, st);
+    return g.blk ? launch_form<SDY_Q6_K, false>(g, form, tok_tiles, st) : launch_form<SDY_Q6_K, true>(g, form, tok_tiles, st);
 }

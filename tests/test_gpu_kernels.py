@@ -1729,6 +1729,37 @@ def test_gemm_form_lines(kind, n_in, n_out, n_tok, tiled, planes):
         m.close()
 
 
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("n_in,rows", [(256, 130), (1792, 64), (2048, 66), (2304, 97)])
+def test_gemm_grouped_planes_and_copy(kind, n_in, rows):
+    """The grouped GEMM from the planes (from eight super-blocks to a row on two waves each) and from the tiled copy, groups
+    of 0 to 70 tokens, rows that do not fill a tile: the oracle's bits per group, with and without the SwiGLU epilogue."""
+    L, t, cnt = lib(), TYPES[kind], np.array([0, 1, 70, 0, 33, 5])
+    n_tok, n_grp = int(cnt.sum()), len(cnt)
+    w = _full_range_blocks(kind, rows * n_grp, n_in, n_in + rows)
+    xq = O.quantize(np.random.default_rng(3).standard_normal((n_tok, n_in)).astype(np.float32), O.Q8_K)
+    exp, t0 = np.empty((n_tok, rows), np.float32), 0
+    for e, c in enumerate(cnt):
+        if c:
+            exp[t0:t0 + c] = O.matmul_q(np.ascontiguousarray(w.reshape(n_grp, rows, -1)[e]), t, xq.reshape(n_tok, -1)[t0:t0 + c], n_in, simd=1)
+        t0 += c
+    tok = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    tile = np.concatenate([[0], np.cumsum((cnt + 31) // 32)]).astype(np.int32)
+    dq, dtok, dtile = (capi.DeviceBuffer.from_array(a) for a in (xq, tok, tile))
+    ws = capi.DeviceBuffer(L.sdy_gemm_ws_bytes(n_tok, n_in))
+    gate, up = np.ascontiguousarray(exp[:, 0:rows & ~1:2]), np.ascontiguousarray(exp[:, 1::2])
+    L.op_silu_mul(ptr(gate), ptr(up), gate.size)
+    for layout in (True, False):
+        m = capi.DeviceMatrix(t, n_in, rows * n_grp, w, gemm_layout=layout)
+        for epilogue, want in ((capi.EPI_NONE, exp),) + (((capi.EPI_SWIGLU, gate),) if rows % 2 == 0 else ()):
+            cols = want.shape[1]
+            out = capi.DeviceBuffer.from_array(np.full((n_tok, cols), np.nan, np.float32))
+            a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=cols, row0=0, row1=rows, epilogue=epilogue)
+            capi.check(L.sdy_gemm_grouped(ctypes.byref(m.m), rows, n_grp, dtok.ptr, dtile.ptr, None, None, 0, ctypes.byref(a), ws.ptr, None))
+            assert ("k_gemm<%d, 2, 2, 1," if not layout and n_in >= 2048 else "k_gemm<%d, 4, 1, 1,") % t in L.sdy_last_kernel().decode()
+            assert np.array_equal(bits(out.to_array(np.float32, (n_tok, cols))), bits(want))
+
+
 @pytest.mark.parametrize("n_in", [256, 512])
 @pytest.mark.parametrize("rows1,rows2,n_tok,pair", [(33, 7, 2, True), (384, 128, 64, True), (600, 77, 450, True), (1281, 300, 450, False)])
 def test_gemm2_short_rows_bit_exact(n_in, rows1, rows2, n_tok, pair):
