@@ -9,9 +9,10 @@
 //
 // What bounds it: per 32 x 32 x 32 products the VALU's 32 instructions take 128 cycles, beside them the matrix
 // cores' two instructions 64. (The f32 outer product on v_mfma_f32_32x32x1 does not run beside VALU work.) At
-// 22016 x 2048 and 512 tokens, 46 GFLOP: 2213 us on the 8-token matvec before, 121 us now; the VALU's share is 47
-// us. Up to 32 tokens it is the weights' stream, a stage's latency per 128 inputs of a wave: 22016 x 2048
-// (46 MB) with 8 tokens 32.1 -> 16.2 us, 11008 x 2048 62 -> 29.5, 2048 x 2048 15.2 -> 12.3.
+// 22016 x 2048 and 512 tokens, 46 GFLOP: 2213 us on the 8-token matvec before, 121 us now, the VALU busy in 50 % of
+// the cycles; a wave waits 27 % of its time for data and barriers, 21 % for its turn to issue, at two waves per SIMD.
+// Up to 32 tokens it is the weights' stream, a stage's latency per 128 inputs of a wave: 22016 x 2048 (46 MB) with 8
+// tokens 32.1 -> 16.2 us, 11008 x 2048 62 -> 29.5, 2048 x 2048 15.2 -> 12.3.
 #include <hip/hip_runtime.h>
 
 #include "sdy_device.h"
@@ -66,7 +67,7 @@ SDY_DEV i32x4 quants(u32x4 raw, uint32_t qh, int h) {
 }
 
 // A workgroup of RW * KS waves computes 32 RW rows x 32 NT tokens; a wave owns 32 rows and all the
-// tokens and, with KS > 1, every KS-th group of 4 blocks (the KS partial sums are added in order through
+// tokens and, with KS > 1, every KS-th group of 4 blocks (the KS partial sums are added through
 // LDS at the end: for few tokens the waves of a matrix' rows would otherwise be too few to keep HBM
 // busy). The weights go straight to registers, each lane (row lr, k-half h) loading its own 16-byte
 // records: from the tiled copy a load instruction reads two runs of 512 bytes, from the row-major planes 64
@@ -222,9 +223,11 @@ __global__ __launch_bounds__(64 * RW * KS, 2) void k_mm_blocks(MmArgs g) {
         if (j == 1 && (b & 1)) load_wd(s + WS, z, b >> 1);
     };
     // The sums in two levels (the blocks of two stages, then those sums): the rounding error of a row of 64 blocks
-    // is half of one chain's. Against 64 bits (relative, with the KS split): 7.3e-8 at 2048 inputs, 7.9e-8 at 4096,
-    // 9e-8 at 11008; the one-token kernel, a tree up to 4096 inputs where 64 units divide among the lanes and a chain
-    // elsewhere: 7.2e-8, 7.7e-8 and 2.4e-7 (1.0e-7 at 1536, 1.5e-7 at 4000).
+    // is half of one chain's. Against 64 bits (relative, with the KS split): 7.29e-8 at 2048 inputs, 7.78e-8 at 4096,
+    // 9.3e-8 at 11008 (64 tokens; 1.08e-7 from 256, on two waves); the one-token kernel, a tree up to 4096 inputs where
+    // 64 units divide among the lanes and a chain elsewhere: 7.16e-8, 7.66e-8 and 2.41e-7 (1.0e-7 at 1536, 1.5e-7 at
+    // 4000). So against the tree it is 2 to 3 % more (at most 5 % by the partial sums' sizes), against the chain half
+    // or less.
     float part[NT][16];
     auto fold = [&](int j, const f32x16 &sc, bool first) {
         const int t = NT == 2 ? j : 0;
@@ -292,7 +295,7 @@ __global__ __launch_bounds__(64 * RW * KS, 2) void k_mm_blocks(MmArgs g) {
         stage(s, 0);
         stage(s + 1, 1);
     }
-    if constexpr (KS > 1) {  // the partial sums of the waves ks > 0, added in order
+    if constexpr (KS > 1) {  // the partial sums of the waves: 0 + 1, or (0 + 1) + (2 + 3)
         float *red = reinterpret_cast<float *>(lds);
         constexpr int TILE = NT * 16 * 64;
         float *mine = red + wave * TILE + lane;
@@ -304,12 +307,15 @@ __global__ __launch_bounds__(64 * RW * KS, 2) void k_mm_blocks(MmArgs g) {
         }
         __syncthreads();
         if (ks > 0) return;
+        static_assert(KS == 2 || KS == 4, "the order of the sums");
 #pragma unroll
-        for (int k = 1; k < KS; k++)
+        for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[nt][i] += mine[k * TILE + (nt * 16 + i) * 64];
+            for (int i = 0; i < 16; i++) {
+                const float *v = mine + (nt * 16 + i) * 64;
+                acc[nt][i] += v[TILE];
+                if constexpr (KS == 4) acc[nt][i] += v[2 * TILE] + v[3 * TILE];
+            }
     }
     // lane (lr, h) holds row ri and, in register i, token 8 (i / 4) + 4 h + i % 4 of each token tile
     const uint32_t etab = sdy_expf_tab_lane(lane);
@@ -367,9 +373,10 @@ template <int WT>
 static int mm_type(const MmArgs &g, hipStream_t st) {
     // The split of a row's blocks over KS waves sets the order of its sum, so it is chosen by the row length and the
     // tokens alone: a row's result does not depend on how many rows a call computes. Two waves for rows of up to
-    // 2048 inputs, four for longer ones (11008 x 2048, 32 tokens: 31.7 us against 41.6 with two), whose error
-    // against 64 bits is then not above that of the one-token kernel either (see fold); from 256 tokens the
-    // rows above 4096, where that kernel adds its units one by one, have waves enough with two (72 against 80 us).
+    // 2048 inputs, four for longer ones (11008 x 2048, 32 tokens: 31.7 us against 41.6 with two), whose error against
+    // 64 bits then is 2 to 3 % above the one-token kernel's at 4096 (see fold; the four sums added one by one: 1 %
+    // more); from 256 tokens the rows above 4096, where that kernel adds its units one by one, have waves enough with
+    // two (72 against 80 us).
     // Tiles of 128 rows x 64 tokens where that leaves work for most CUs (22016 x 2048, 512 tokens: 121 us against
     // 155 with 64 x 32), else 64 x 32 (2048 x 2048, 512 tokens: 20.5 against 25.3).
     if (g.nb <= 64 || (g.nb > 128 && g.n_tok >= 256)) {

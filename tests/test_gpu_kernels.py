@@ -1563,6 +1563,33 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
     assert np.array_equal(bits(run(tiled, dq.ptr, 0, even, capi.EPI_SWIGLU)), bits(gate))
 
 
+@pytest.mark.parametrize("n_in,most", [(2048, 1.052), (4096, 1.046), (11008, 0.6)])
+def test_block_mfma_error_beside_one_token(n_in, most):
+    """The rel-L2 error against float64 of the block types' many-token kernel, over that of the one-token kernels. A rounding's
+    variance goes with the blocks in its partial sum. Over the 64 blocks of 2048 inputs: per wave four chains of 8
+    (4 * 36) and their sum (16 + 24 + 32), two waves and their sum (64), in all 496, against the products (64), pairs
+    (32 * 2) and tree of 32 lanes (5 * 64) there: sqrt(496 / 448) = 1.052 at most. Over 4096: 4 * 216 + (0 + 1) + (2 + 3), 256,
+    against 256 + 6 * 128: sqrt(1120 / 1024) = 1.046. Over 11008 the one-token kernel is a chain: half of its error."""
+    n_out, n_tok = 2048, 64
+    t, w, xq = _matvec_case("Q8_0", n_in, n_out, n_tok, seed=n_in)
+    xb = xq.reshape(n_tok, n_in // 32, 34)
+    xd = xb[:, :, 2:].copy().view(np.int8).astype(np.float64) * xb[:, :, :2].copy().view(np.float16).astype(np.float64)
+    exp = xd.reshape(n_tok, n_in) @ O.dequant(w, t, n_in * n_out).astype(np.float64).reshape(n_out, n_in).T
+    L = lib()
+    m, dq = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceBuffer.from_array(xq)
+    err = []
+    for n in (4, n_tok):
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, n_out), np.nan, np.float32))
+        for t0 in range(0, n_tok, n):
+            a = capi.SdyMvArgs(xq=dq.ptr + t0 * (n_in // 32) * 34, n_tok=n, out=out.ptr + 4 * t0 * n_out, out_stride=n_out,
+                               row0=0, row1=n_out)
+            capi.check(L.sdy_matvec(ctypes.byref(m.m), ctypes.byref(a), None))
+        assert (b"k_mm_blocks" in L.sdy_last_kernel()) == (n > 4)
+        err.append(np.linalg.norm(out.to_array(np.float32, (n_tok, n_out)) - exp))
+    print("one-token", err[0] / np.linalg.norm(exp), "ratio", err[1] / err[0])
+    assert err[1] / err[0] < most
+
+
 @pytest.mark.parametrize("kind", ["Q8_0", "Q4_0", "Q5_0"])
 @pytest.mark.parametrize("n_in,n_out,n_tok,mfma", [
     (32, 33, 5, False), (256, 9000, 8, False), (320, 40961, 8, False), (320, 40960, 8, True), (2048, 2048, 5, False), (4096, 3072, 5, False), (4096, 3073, 5, True), (2048, 4096, 6, False),
