@@ -297,7 +297,7 @@ def test_logits_bit_identical_to_reference(spec, tmp_path):
 @pytest.mark.parametrize("spec", ["qwen2-kquant", "moe-128x8", "qwen2-kquant-v4k", "llama-kquant"])
 def test_file_scales_logits_bit_identical(spec, tmp_path):
     """K-quant scales as quantized model files hold them (Q6_K int8 scales down to -128, Q4_K
-    scales normalised to 63): the prefill GEMMs take the wide variant and the logits keep the
+    scales normalised to 63): gemm_ok 2 in the prefill GEMMs, and the logits keep the
     oracle's bits, prompt chunks and one-token steps alike."""
     path = tmp_path / "m.gguf"
     write_model(path, dataclasses.replace(SPECS[spec], context=160, scales="file"), seed=11)

@@ -1070,7 +1070,7 @@ def test_prefill_attention_tokens_bit_identical(n_head, n_kv_head, hd, n_tok, n_
 @pytest.mark.parametrize("n_tok,n_kv0", [(16, 1), (40, 70), (77, 3), (512, 1), (100, 900)])
 @pytest.mark.parametrize("kv", ["f32", "f16"])
 def test_prefill_attention_flash(n_head, n_kv_head, hd, n_tok, n_kv0, kv):
-    """The flash-form prompt attention (f32 matrix cores, eight waves per 32 queries over key tiles
+    """The flash-form prompt attention (bf16 fragments, eight waves per 32 queries over key tiles
     of 32, merged in wave order) is within 1e-5 of the output scale of the reference's arithmetic
     (sdy_attention, bit-exact with the oracle), for partial query blocks and key tiles, q rows at a
     stride wider than the heads (the engine's q|k|v rows) and both cache types; it is deterministic."""
@@ -1313,7 +1313,7 @@ def test_gemm_bit_exact_with_subnormal_scale_products(kind):
 
 @pytest.mark.parametrize("n_in,n_tok", [(2048, 512), (11008, 33), (256, 16)])
 def test_gemm_ws_ready_reuses_expansion(n_in, n_tok):
-    """ws_ready = 1 skips the f16 expansion of the activations: a Q6_K GEMM that reuses the workspace
+    """ws_ready = 1 skips the expansion of the activations: a Q6_K GEMM that reuses the workspace
     a Q4_K GEMM on the same Q8_K input just filled gives the bits of its own full call and of the
     oracle; after a different input has been expanded into the workspace, a full call is needed again."""
     L = lib()
@@ -1390,7 +1390,7 @@ def test_quantize_gemm_expansion(norm, n_in, n_tok):
 @pytest.mark.parametrize("n_in,rows1,rows2,n_tok", [(2048, 2304, 256, 512), (1024, 200, 77, 45)])
 def test_gemm2_pair_launch_bit_exact(n_in, rows1, rows2, n_tok, wide1, wide2):
     """sdy_gemm2 (a layer's Q4_K q|k and Q6_K v on the same activations, one launch) gives each matrix
-    the oracle's bits, bias included, in the one-fragment and wide forms of either matrix, and with
+    the oracle's bits, bias included, with ordinary and full-range scales of either matrix, and with
     row counts that do not fill the 64-row tiles."""
     L = lib()
     rng = np.random.default_rng(rows1 + rows2 + n_tok)
@@ -1454,8 +1454,8 @@ def test_gemm_layout_copy_and_planes_same_bits(kind):
 def test_matrix_in_host_memory_same_bits(kind):
     """A matrix in pinned host memory (sdy_mat_alloc_host, read in place by the kernels over the host
     link, as the engine keeps expert stacks the device has no room for): its dequantised rows, its
-    one-token and 40-token matvecs and, for the K-quants, the GEMM (the wide variant: a host matrix is
-    not checked, and keeps no tiled copy) have the bits of the same matrix in device memory."""
+    one-token and 40-token matvecs and, for the K-quants, the GEMM (a host matrix keeps no
+    tiled copy) have the bits of the same matrix in device memory."""
     L = lib()
     n_in, n_out, n_tok = 2048, 70, 40
     t, w, xq = _matvec_case(kind, n_in, n_out, n_tok, seed=31)
@@ -2017,11 +2017,10 @@ def _full_range_blocks(kind, n_out, n_in, seed):
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("n_in,n_out,n_tok", [(2048, 96, 40), (1024, 37, 129), (256, 64, 2)])
 def test_gemm_wide_variant_bit_exact(kind, n_in, n_out, n_tok):
-    """Matrices whose blocks the one-fragment scheme would round (Q6_K |sc * (q - 32)| above 2048,
-    partial sums of 2^24 and more) are flagged for the wide variant (gemm_ok 2), which keeps
-    the oracle's bits for every row and token: scales over the whole stored range, a token of one
-    sign (Q8_K values all -127) that drives the extreme rows' sums to their bounds. The same shapes
-    with the workload's scales take the one-fragment variant (gemm_ok 1)."""
+    """Matrices with scales beyond what real files hold (Q6_K |sc * (q - 32)| above 2048, partial sums
+    of 2^24 and more: gemm_ok 2) have the oracle's bits for every row and token: scales over the whole
+    stored range, a token of one sign (Q8_K values all -127) that drives the extreme rows' sums to
+    their bounds. The same shapes with the workload's scales have gemm_ok 1."""
     L = lib()
     t = TYPES[kind]
     w = _full_range_blocks(kind, n_out, n_in, n_in + n_out)
@@ -2043,8 +2042,7 @@ def test_gemm_wide_variant_bit_exact(kind, n_in, n_out, n_tok):
 
 
 def test_gemm_variant_check_flags_rows():
-    """One Q6_K block with scales -128 anywhere in the matrix selects the wide variant;
-    ordinary rows keep the one-fragment one."""
+    """One Q6_K block with scales -128 anywhere in the matrix gives it gemm_ok 2; ordinary rows alone 1."""
     L = lib()
     w = random_blocks("Q6_K", 8 * 4, np.random.default_rng(3)).reshape(8, -1)
     ok = capi.DeviceMatrix(O.Q6_K, 1024, 8, w)
@@ -2296,8 +2294,8 @@ def _mat_bytes(m):
 def test_pipelined_upload_equals_synchronous(kind, n_in, grp, n_grp, bad_scale):
     """The pipelined uploader (1 MiB pinned/device slots, so a tensor spans several slots; the rows of
     a per-group interleaved map, as the engine's per-expert gate|up, split at group boundaries) leaves
-    the same device bytes as the synchronous upload, and the deferred variant check the same
-    gemm_ok (a Q6_K block with scale -128 selects the wide variant)."""
+    the same device bytes as the synchronous upload, and the deferred scale check the same
+    gemm_ok (2 with a Q6_K block of scale -128)."""
     L = lib()
     t = TYPES[kind]
     rng = np.random.default_rng(grp + n_in)
