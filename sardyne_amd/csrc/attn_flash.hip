@@ -14,13 +14,15 @@
 //   The waves' (m, l, O) are then merged through LDS in wave order:
 //   out = sum_w O_w exp(m_w - M) / sum_w l_w exp(m_w - M), M = max_w m_w.
 //
-// Every f32 operand is the exact sum of three bf16 (an f16 cache's of two), and a product the sum of the six (five)
-// bf16 products above 2^-26 of it, added in f32 by v_mfma_f32_32x32x16_bf16: 192 matrix-core cycles per 32 x 32 x 16
-// where v_mfma_f32_32x32x2_f32 takes 512 and lets no VALU work run beside it. The error against 64 bits is the f32
-// form's or less (512 tokens over 1024 cached positions, 32 heads of 128: 3.9e-7 against 4.7e-7): there are fewer
+// Every f32 operand is the exact sum of three bf16 (an f16 cache's of two), each at most 2^-8 of the one before, and a
+// product the sum of the six (five) greatest of their bf16 products, added in f32 by v_mfma_f32_32x32x16_bf16: 192
+// matrix-core cycles per 32 x 32 x 16 where v_mfma_f32_32x32x2_f32 takes 512 and lets no VALU work run beside it. Left
+// out are two products of at most about 2^-25 of the whole each and less, together at most 2^-24 (found: 2^-24.01), as
+// much as one rounding of an f32 product. The error against 64 bits is the f32 form's or less (512 tokens over 1024 cached positions, 32 heads of 128: 3.9e-7 against 4.7e-7): there are fewer
 // sums to round. The queries' fragments sit in LDS; K's and V's are made in registers, 3.5 VALU instructions per
-// element. What bounds it: latency at two waves per SIMD (254 registers), the splits (450 of the tile's 730 VALU
-// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 128 -> 82 us (10.7 GFLOP), f16 138 -> 83;
+// element. What bounds it: latency at two waves per SIMD (254 registers; the VALU busy in 36 % of the cycles, a
+// wave ready but not issuing 44 % of its time, waiting for data 26 %), the splits (450 of the tile's 730 VALU
+// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 128 -> 84 us (10.7 GFLOP), f16 138 -> 83;
 // 301 tokens, 32 heads: 34 -> 24; 77 tokens over 3000 positions, 16 heads, f16: 126 -> 66. The XCD order is 6 us of the
 // first. Two blocks of queries per wave, sharing the splits and the stream: f32 spills (100 us), f16 76, and half the
 // workgroups for the shorter prompts (22 -> 32 us).
@@ -132,7 +134,7 @@ struct Frag {
     }
 };
 
-// c + A B in f32 from the fragments, least products first. Those left out are below 2^-26 of |a b|.
+// c + A B in f32 from the fragments, least products first. Those left out are together at most 2^-24 of |a b|.
 template <int NA>
 SDY_DEV f32x16 mfma_split(const Frag<NA> &a, const Frag<3> &b, f32x16 c) {
 #pragma unroll

@@ -656,7 +656,7 @@ static int load(engine_model *m, const char *path, char *err, size_t len) {
     if (sdy_uploader_free(ld.up) && !rc) rc = device_fail(&ld, "upload");
     if (!rc) rc = gemm_copies(&ld);
     if (!rc) {
-        /* views taken before the exactness checks ran: take them again (gemm_ok of the stack) */
+        /* views taken before the scale checks and the tiled copies: take them again (gemm_ok and gbase of the stack) */
         for (int l = 0; l < in->n_layer; l++) {
             dlayer *L = &m->layers[l];
             if (L->qkv_parts >= 2) {

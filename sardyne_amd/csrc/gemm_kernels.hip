@@ -10,14 +10,17 @@
 // rounding, the VALU multiply's; a zero product may be +0 where the multiply gives -0, which no sum keeps), and
 // the combine is the reference's expression, super-blocks in order.
 //
-// What bounds it: the VALU. Per super-block and 32 x 32 outputs Q4_K takes 315 VALU instructions (128 multiply-adds,
-// 96 of the combine) and the f32 outer product's 64 cycles, Q6_K about 500; the matrix cores' 290 and 540 cycles run
-// beside them. The weights dequantised to f16 (sc * q, one fragment, two for the scales of real Q6_K files) summed
-// whole super-blocks on the matrix cores with fewer VALU instructions, but its registers and LDS left two waves
-// to a SIMD that waited for each other; here three or more keep the VALU busy. With the quantiser's launch, f16
-// form -> this: 22016 x 2048 Q4_K, 512 tokens 90.6 -> 82.0 us (565 TFLOP/s; VALU busy 65 %), 128 tokens 40.4 -> 29.0;
-// 2048 x 11008 Q6_K, 203 tokens 69.4 -> 46.7, 64 tokens 66.3 -> 31.6 (on mm_superblocks.hip); 151936 x 2048 Q6_K, 32
-// tokens 110 -> 79, 64 tokens 127 -> 125.
+// What bounds it: VALU work and the waits between it. Per super-block and 32 x 32 outputs Q4_K takes 304 VALU
+// instructions (128 multiply-adds, 96 of the combine) and the f32 outer product's 64 cycles, Q6_K 524, or 424 where a
+// wave unpacks the weights once for two token tiles; the matrix cores' 290 and 540 cycles run beside them. With three
+// or more waves to a SIMD (22016 x 2048 Q4_K, 512 tokens) the VALU is busy in 73 % of the cycles; with two, a wave's
+// waits show (151936 x 2048 Q6_K, 64 tokens, two token tiles to a wave: 51 %; 2048 x 11008 Q6_K, 203 tokens, 448 tiles
+// split over four waves each: 40 %). The weights dequantised to f16 (sc * q, one fragment, two for the scales of real
+// Q6_K files) summed whole super-blocks on the matrix cores with fewer VALU instructions, but its registers and LDS left
+// two waves to a SIMD that waited for each other. With the quantiser's launch, f16 form -> this: 22016 x 2048 Q4_K, 512
+// tokens 90.7 -> 81.2 us (568 TFLOP/s), 128 tokens 40.4 -> 29.0; 2048 x 11008 Q6_K, 203 tokens 69.1 -> 42.1, 64 tokens
+// 66.3 -> 31.6 (on mm_superblocks.hip); 151936 x 2048 Q6_K, 32 tokens 110 -> 79, 64 tokens 121 -> 113. Q6_K on the
+// largest grids is slower than on the f16 form: 22016 x 2048, 512 tokens 109 -> 113, 22016 x 4096 196 -> 216.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -577,7 +580,7 @@ extern "C" int sdy_mat_gemm_layout(sdy_mat *m, sdy_stream s) {
 
 // Flags (bad = 1) rows [r0, r0 + n) of m with a block of gemm_ok 2. Synchronous.
 extern "C" int sdy_gemm_check_rows_async(const sdy_mat *m, long r0, long n, int *bad_dev, sdy_stream s) {
-    if ((m->type != SDY_Q4_K && m->type != SDY_Q6_K) || m->hbase) return 0;  // (host memory: wide, unchecked)
+    if ((m->type != SDY_Q4_K && m->type != SDY_Q6_K) || m->hbase) return 0;  // (host memory: unchecked)
     sdy_mat v = sdy_mat_rows(m, r0, n);
     GemmArgs g = gemm_args(&v);
     const long total = n * (long)g.nb;
@@ -618,7 +621,7 @@ extern "C" int sdy_gemm_ok(const sdy_mat *m, int n_tok) {
 }
 
 // A Q4_K lane reaches both quant planes by one 32-bit offset from its row tile in the first, but where a plane ends just
-// short of 4 GiB (the most sdy_gemm_ok takes): the FAR form.
+// short of 4 GiB (the most sdy_gemm_ok takes): the ALT form.
 static bool gemm_far(const GemmArgs &g) { return (size_t)(g.p[1] - g.p[0]) + (size_t)g.T * 4096 > 0xFFFFFFFFu; }
 
 template <int WT, int RW, int KS, int NT = 1, bool ALT = false>

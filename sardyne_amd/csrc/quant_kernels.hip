@@ -2804,8 +2804,9 @@ static int superblocks_min_tok(const sdy_mat *m, long rows) {
 // launch, five tokens, Q8_0 / Q5_0: 22016 x 2048 20.2 -> 12.8 / 20.8 -> 14.7 us, 2048 x 8192 29.1 -> 20.3 / 28.2 -> 24.1, but
 // 2048 x 2048 7.9 against 8.8 / 8.1 against 10.8 and 2048 x 4096 11.1 against 12.3 / 11.4 against 14.4; 2048 x 4096, six tokens
 // 12.5 against 12.2 / 12.8 against 14.3, seven 14.3 against 12.3 / 14.7 against 14.3), and where a wave of the matvecs has lanes
-// idle: rows of 33 to 63 units of 64 elements (2048 x 3072, five tokens: 12.5 -> 10.3 / 12.6 -> 11.8). Not with very short rows, whose tiles end before they have begun (131072 x 256, five tokens 1.7 / 2.0 times the
-// matvec's time, eight 1.5 / 1.7; 131072 x 800, five 1.12 / 1.07).
+// idle: rows of 33 to 63 units of 64 elements (2048 x 3072, five tokens: 12.5 -> 10.3 / 12.6 -> 11.8). Not with
+// very short rows, whose tiles end before they have begun (131072 x 256, five tokens 1.7 / 2.0 times the matvec's time,
+// eight 1.5 / 1.7; 131072 x 800, five 1.12 / 1.07).
 static bool blocks_take(const sdy_mat *m, int n_tok) {
     if (n_tok < 5 || n_tok > 8) return n_tok > 8;
     if (m->n_units <= 4 || m->n_rows > 128L * m->n_in) return false;

@@ -79,7 +79,7 @@ struct engine_ctx {
     float *attn_part;           /* chunked / split attention: per-span partials */
     unsigned *attn_count;       /* split attention: arrivals per kv head (zero between launches) */
     float *qkv;                 /* q | k | v of one token */
-    void *gemm_ws;              /* scratch of the prefill GEMM (f16 activations of n_batch rows) */
+    void *gemm_ws;              /* scratch of the prefill GEMM (the activations of n_batch rows in planes) */
     /* MoE */
     float *moe_probs, *moe_w, *moe_x, *moe_y, *moe_sum, *moe_gw;
     int32_t *moe_top, *moe_gidx, *moe_top_host, *moe_gidx_host;

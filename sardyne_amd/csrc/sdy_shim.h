@@ -109,7 +109,7 @@ size_t sdy_mat_gemm_layout_bytes(const sdy_mat *m);
 /* Pipelined uploads (upload.hip): a ring of pinned host slots and device slots. A host thread pool
  * copies the next rows from the file mapping into a free pinned slot (advising the kernel to read
  * the rows after them ahead), the DMA engine moves the slot to the device on a copy stream, and the
- * repack runs on the work stream; the three overlap across slots. The GEMM variant checks of the
+ * repack runs on the work stream; the three overlap across slots. The scale checks (gemm_ok) of the
  * uploaded rows run at sdy_uploader_finish, which waits for everything and sets each matrix's
  * gemm_ok. A matrix must stay at its address until then. */
 typedef struct sdy_uploader sdy_uploader;
