@@ -59,13 +59,13 @@ struct FlashArgs {
 
 // LDS: the block's queries, as fragments [3][32][HD + 8] bf16 or as f32 [2][32][QS] (element (query q, dim
 // half * HD/2 + s) at [half][q][s]), then, after the key tiles, the merge area: the waves' O dims, 1/MS of them at a time, as
-// [FW][32][OS] and their m, l as [2][FW][32] (HD 128: 134 KB for MS 1, one workgroup per CU;
+// [FW][32][OS], their m, l as [2][FW][32] and whether their sums hold as [FW] (HD 128: 134 KB for MS 1, one workgroup per CU;
 // 68 KB for MS 2, two).
 template <int HD, int MS>
 struct FlashLds {
     static constexpr int HH = HD / 2, QS = HH + 4, OS = HD / MS + 1;
     static constexpr size_t q_floats = 2 * 32 * QS;
-    static constexpr size_t merge_floats = (size_t)FW * 32 * OS + 2 * FW * 32;
+    static constexpr size_t merge_floats = (size_t)FW * 32 * OS + 2 * FW * 32 + FW;
     static constexpr size_t bytes = 4 * (q_floats > merge_floats ? q_floats : merge_floats);
 };
 
@@ -306,6 +306,7 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
                 o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(VL::at(vv[r], dt), p[r], o[dt], 0, 0, 0);
     }
 
+    bool unfit = false;
     if constexpr (SPLIT) {
         float z = 0.0f * l_run;  // NaN from an infinity or a NaN on
         uint32_t least = ~0u;    // the least |o| but 0, its bits shifted and less one
@@ -317,7 +318,7 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
                 const uint32_t u = (__float_as_uint(o[dt][e]) << 1) - 1;
                 least = u < least ? u : least;
             }
-        if (__syncthreads_or(z != z || least < (127u - 90u) << 24)) return true;
+        unfit = __ballot(z != z || least < (127u - 90u) << 24) != 0;
     }
     // merge of the waves' partials in wave order (the Q^T area is reused), in MS parts of the dims:
     // part x holds the O columns dt in [x NDH, (x + 1) NDH), dims ND * row + dt, at NDH * row + dt - x NDH
@@ -338,7 +339,16 @@ SDY_DEV bool flash_block(const FlashArgs &a, float *lds) {
             ml[wave * 32 + ql] = m_run;
             ml[FW * 32 + wave * 32 + ql] = l_run;
         }
+        int *const fl = reinterpret_cast<int *>(ml + 2 * FW * 32);
+        if (SPLIT && x == 0 && lane == 0) fl[wave] = unfit;
         __syncthreads();
+        if (SPLIT && x == 0) {  // (the other form's queries do not reach the flags)
+            static_assert(LY::q_floats <= (size_t)FW * 32 * LY::OS, "the flags outlive the queries' writes");
+            int any = 0;
+#pragma unroll
+            for (int w = 0; w < FW; w++) any |= fl[w];
+            if (__builtin_amdgcn_readfirstlane(any)) return true;
+        }
         for (int i = tid; i < QB * (HD / MS); i += 64 * FW) {
             const int q = i / (HD / MS), dl = i - q * (HD / MS);
             if (q0 + q >= a.n_tok) continue;
