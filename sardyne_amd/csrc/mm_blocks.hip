@@ -370,16 +370,20 @@ static int launch_mm(const MmArgs &g, hipStream_t st) {
 }
 
 template <int WT>
-static int mm_type(const MmArgs &g, hipStream_t st) {
-    // The split of a row's blocks over KS waves sets the order of its sum, so it is chosen by the row length and the
-    // tokens alone: a row's result does not depend on how many rows a call computes. Two waves for rows of up to
-    // 2048 inputs, four for longer ones (11008 x 2048, 32 tokens: 31.7 us against 41.6 with two), whose error against
+static int mm_type(const MmArgs &g, long mat_rows, hipStream_t st) {
+    // The split of a row's blocks over KS waves sets the order of its sum, so it is chosen by the row length, the
+    // tokens and the matrix' rows: a row's result does not depend on how many rows a call computes. Two waves for rows of
+    // up to 2048 inputs, four for longer ones (11008 x 2048, 32 tokens: 31.7 us against 41.6 with two), whose error against
     // 64 bits then is 2 to 3 % above the one-token kernel's at 4096 (see fold; the four sums added one by one: 1 %
-    // more); from 256 tokens the rows above 4096, where that kernel adds its units one by one, have waves enough with
-    // two (72 against 80 us).
-    // Tiles of 128 rows x 64 tokens where that leaves work for most CUs (22016 x 2048, 512 tokens: 121 us against
-    // 155 with 64 x 32), else 64 x 32 (2048 x 2048, 512 tokens: 20.5 against 25.3).
-    if (g.nb <= 64 || (g.nb > 128 && g.n_tok >= 256)) {
+    // more). Two again where the rows alone are waves enough: from 256 tokens above 4096 inputs (72 against 80 us), and on
+    // more rows than 256 tiles of 32, one to a CU, of 33 to 63 units of 64 inputs, where the four also idle through most of
+    // a row's last stage of 16 blocks (Q8_0, 5 tokens: 121872 x 2080 60 against 95 us, the matvec 67; 16000 x 3072 16.3
+    // against 17.6, but 8000 x 3072 14.7 against 13.0; 64 tokens, 16000 x 2080 19 against 31). The one-token kernel is a chain there (error 1.15e-7,
+    // 1.24e-7 and 1.34e-7 at 2080, 2560 and 3072 inputs, here 7.5e-8, 7.6e-8 and 7.8e-8); of 64 units it is the tree, which
+    // two waves miss by 8 %.
+    if (g.nb <= 64 || (g.T < 64 && mat_rows > 8192) || (g.nb > 128 && g.n_tok >= 256)) {
+        // Tiles of 128 rows x 64 tokens where that leaves work for most CUs (22016 x 2048, 512 tokens: 121 us against
+        // 155 with 64 x 32), else 64 x 32 (2048 x 2048, 512 tokens: 20.5 against 25.3).
         const bool wide = g.n_tok > 32 && ((g.n_tok + 63) / 64) * ((g.n_rows + 127) / 128) >= 160;
         return wide ? launch_mm<WT, 4, 2, 2>(g, st) : launch_mm<WT, 2, 2, 1>(g, st);
     }
@@ -416,8 +420,8 @@ extern "C" int sdy_mm_blocks(const sdy_mat *m, const sdy_mv_args *a, sdy_stream 
     g.swiglu = a->epilogue == SDY_EPI_SWIGLU;
     hipStream_t st = (hipStream_t)s;
     switch (m->type) {
-    case SDY_Q8_0: return mm_type<SDY_Q8_0>(g, st);
-    case SDY_Q4_0: return mm_type<SDY_Q4_0>(g, st);
-    default: return mm_type<SDY_Q5_0>(g, st);
+    case SDY_Q8_0: return mm_type<SDY_Q8_0>(g, m->n_rows, st);
+    case SDY_Q4_0: return mm_type<SDY_Q4_0>(g, m->n_rows, st);
+    default: return mm_type<SDY_Q5_0>(g, m->n_rows, st);
     }
 }

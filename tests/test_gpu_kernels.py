@@ -1563,6 +1563,36 @@ def test_block_mfma_many_tokens(kind, n_in, n_out, n_tok):
     assert np.array_equal(bits(run(tiled, dq.ptr, 0, even, capi.EPI_SWIGLU)), bits(gate))
 
 
+@pytest.mark.parametrize("kind", ["Q8_0", "Q5_0"])
+@pytest.mark.parametrize("n_in,n_out,n_tok,ks", [(2080, 8192, 9, 4), (2080, 8193, 8, 2), (4032, 8193, 40, 2),
+                                                 (4064, 8193, 9, 4), (2048, 70, 9, 2)])
+def test_block_mfma_split_lines(kind, n_in, n_out, n_tok, ks):
+    """Where the block types' many-token kernel splits a row over two waves instead of four: the kernel that runs, against
+    float64 (the bound of test_block_mfma_many_tokens: a wave's chain of sums, in blocks of eight, is at most 8 + nb / 16), and
+    a short row range has the same bits."""
+    t, w, xq = _matvec_case(kind, n_in, n_out, n_tok, seed=n_in + n_tok)
+    nb = n_in // 32
+    wd = O.dequant(w, t, n_in * n_out).astype(np.float64).reshape(n_out, nb, 32)
+    xb = xq.reshape(n_tok, nb, 34)
+    xd = xb[:, :, 2:].copy().view(np.int8).astype(np.float64) * xb[:, :, :2].copy().view(np.float16).astype(np.float64)
+    p = [xd[:, b] @ wd[:, b].T for b in range(nb)]
+    exp, mag = sum(p), sum(np.abs(v) for v in p)
+    L = lib()
+    m, dq = capi.DeviceMatrix(t, n_in, n_out, w), capi.DeviceBuffer.from_array(xq)
+
+    def run(r0, r1):
+        out = capi.DeviceBuffer.from_array(np.full((n_tok, n_out), np.nan, np.float32))
+        a = capi.SdyMvArgs(xq=dq.ptr, n_tok=n_tok, out=out.ptr, out_stride=n_out, row0=r0, row1=r1)
+        capi.check(L.sdy_matvec(ctypes.byref(m.m), ctypes.byref(a), None))
+        name = L.sdy_last_kernel().decode()
+        assert "k_mm_blocks<" in name and name.split("<")[1].split(", ")[2] == str(ks)
+        return out.to_array(np.float32, (n_tok, n_out))
+
+    got = run(0, n_out)
+    assert np.all(np.abs(got - exp) <= (12 + nb / 16) * 2.0 ** -24 * mag + 1e-45)
+    assert np.array_equal(bits(run(3, 60)[:, 3:60]), bits(got[:, 3:60]))
+
+
 @pytest.mark.parametrize("n_in,most", [(2048, 1.052), (4096, 1.046), (11008, 0.6)])
 def test_block_mfma_error_beside_one_token(n_in, most):
     """The rel-L2 error against float64 of the block types' many-token kernel, over that of the one-token kernels. A rounding's
