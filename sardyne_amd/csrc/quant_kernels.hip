@@ -2783,7 +2783,9 @@ static int launch_mv(const sdy_mat *m, const sdy_mv_args *a, int n_tok, const ui
 // quantiser's launch: Q4_K is faster from two tokens on (22016 x 2048: 13.7 -> 6.9 us; 2048 x 2048: 5.6 -> 4.2); so is Q6_K up
 // to 4096 rows (4096 x 8192, two tokens: 15.6 -> 10.7) but for some on few rows (1024 x 8192: two tokens 8.8 against 10.5,
 // three 10.7 against 11.0; 512 x 11008: two 11.3 against 13.3, three 14.5 against 13.9). On more rows Q6_K's arithmetic counts:
-// 151936 x 2048 takes 84 us whatever the tokens, the matvecs 57, 74, 85 and 100 for 2, 3, 4 and 5.
+// 151936 x 2048 takes 84 us whatever the tokens, the matvecs 57, 74, 85 and 100 for 2, 3, 4 and 5; rows of 5 or 6
+// super-blocks leave waves of eight idle (151936 x 1280, five tokens 51.7 against 56.3, six 56.2 against 57.3; 80000 x 1280, five
+// 32.4 against 32.0).
 // From the planes a load instruction meets as many cache lines as rows: Q6_K 1024 x 4096, two tokens 6.2 against 9.2, four 9.1
 // against 9.5, five 11.4 against 9.6; 1024 x 8192, six 16.0 against 18.6, eight 19.3 against 19.3; 2048 x 11008, three 18.8
 // against 18.6; Q4_K 1024 x 8192, three 10.4 against 11.7, five 13.8 against 12.1.
@@ -2793,7 +2795,7 @@ static int superblocks_min_tok(const sdy_mat *m, long rows) {
     const int nb = m->n_in / 256, few = rows <= 1024;
     if (m->hbase) return 9;
     if (m->type == SDY_Q4_K) return m->gbase || !few ? 2 : 2 + nb / 16;
-    if (rows > 4096) return 5;
+    if (rows > 4096) return rows > 65536 && (nb == 5 || nb == 6) ? 6 : 5;
     if (m->gbase) return few ? 2 + nb / 24 : 2;
     return 2 + (int)(nb * 144 / (few ? 1024 : rows));
 }

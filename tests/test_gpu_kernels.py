@@ -1660,7 +1660,8 @@ def test_block_types_few_tokens(kind, n_in, n_out, n_tok, mfma):
 @pytest.mark.parametrize("n_in,n_out,n_tok,planes,mfma", [
     (2048, 1024, 2, "Q-", "KK"), (6144, 1024, 2, "--", "K-"), (6144, 1024, 3, "Q-", "KK"), (4096, 300, 2, "--", "KK"),
     (4096, 1024, 3, "Q-", "KK"), (4096, 300, 4, "QQ", "KK"), (4096, 1025, 3, "Q-", "KK"), (4096, 2049, 2, "Q-", "KK"),
-    (8192, 40, 8, "QQ", "KK"), (1024, 4097, 4, "Q-", "K-"), (1024, 4097, 5, "QQ", "KK"), (256, 40, 8, "QQ", "KK")])
+    (8192, 40, 8, "QQ", "KK"), (1024, 4097, 4, "Q-", "K-"), (1024, 4097, 5, "QQ", "KK"), (256, 40, 8, "QQ", "KK"),
+    (1280, 65537, 5, "Q-", "K-"), (1536, 65537, 6, "QQ", "KK"), (1280, 65536, 5, "QQ", "KK"), (1792, 65537, 5, "QQ", "KK")])
 def test_superblocks_few_tokens_dispatch(kind, n_in, n_out, n_tok, planes, mfma):
     """Both sides of the lines between the matvecs and the matrix cores (first letter Q4_K, second Q6_K; "-" the matvecs),
     from the planes, from the tiled copy, and from pinned host memory, which takes the matvecs up to eight tokens: the
