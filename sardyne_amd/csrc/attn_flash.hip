@@ -20,10 +20,10 @@
 // out are two products of at most about 2^-25 of the whole each and less, together at most 2^-24 (found: 2^-24.01), as
 // much as one rounding of an f32 product. The error against 64 bits is the f32 form's or less (512 tokens over 1024 cached positions, 32 heads of 128: 3.9e-7 against 4.7e-7): there are fewer
 // sums to round. The queries' fragments sit in LDS; K's and V's are made in registers, 3.5 VALU instructions per
-// element. What bounds it: latency at two waves per SIMD (254 registers; the VALU busy in 36 % of the cycles, a
+// element. What bounds it: latency at two waves per SIMD (256 registers; the VALU busy in 37 % of the cycles, a
 // wave ready but not issuing 44 % of its time, waiting for data 26 %), the splits (450 of the tile's 730 VALU
-// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 128 -> 84 us (10.7 GFLOP), f16 138 -> 83;
-// 301 tokens, 32 heads: 34 -> 24; 77 tokens over 3000 positions, 16 heads, f16: 126 -> 66. The XCD order is 6 us of the
+// instructions) and the keys' stream from L2. The 512 tokens above, f32 cache: 129 -> 82 us (10.7 GFLOP), f16 129 -> 70;
+// 301 tokens, 32 heads: 34 -> 24; 77 tokens over 3000 positions, 16 heads, f16: 123 -> 64. The XCD order is 6 us of the
 // first. Two blocks of queries per wave, sharing the splits and the stream: f32 spills (100 us), f16 76, and half the
 // workgroups for the shorter prompts (22 -> 32 us).
 //

@@ -13,7 +13,7 @@
 // What bounds it: VALU work and the waits between it. Per super-block and 32 x 32 outputs Q4_K takes 304 VALU
 // instructions (128 multiply-adds, 96 of the combine) and the f32 outer product's 64 cycles, Q6_K 524, or 424 where a
 // wave unpacks the weights once for two token tiles; the matrix cores' 290 and 540 cycles run beside them. With three
-// or more waves to a SIMD (22016 x 2048 Q4_K, 512 tokens) the VALU is busy in 73 % of the cycles; with two, a wave's
+// or more waves to a SIMD (22016 x 2048 Q4_K, 512 tokens) the VALU is busy in 74 % of the cycles; with two, a wave's
 // waits show (151936 x 2048 Q6_K, 64 tokens, two token tiles to a wave: 51 %; 2048 x 11008 Q6_K, 203 tokens, 448 tiles
 // split over four waves each: 40 %). The weights dequantised to f16 (sc * q, one fragment, two for the scales of real
 // Q6_K files) summed whole super-blocks on the matrix cores with fewer VALU instructions, but its registers and LDS left

@@ -9,7 +9,7 @@
 // Each wave takes one super-block of 16 MT rows and requests all it needs of it at once; the eight waves of a workgroup
 // (four, or two, where a row has no more super-blocks) take as many super-blocks side by side and hand their terms
 // through LDS to the threads that add them in order. What bounds it: the weights' stream and its latency (22016 x 2048
-// Q4_K, 7 tokens: a wave waits 47 % of its time for data, the VALU is busy in 21 % of the cycles); the VALU work of a
+// Q4_K, 7 tokens: a wave waits 47 % of its time for data, the VALU is busy in 22 % of the cycles); the VALU work of a
 // super-block is about 115 instructions per 16 rows whatever the tokens, up to 16, where the 8-token matvec spends 245
 // per token and 64 units. 22016 x 2048 Q4_K (25 MB), 8 tokens, with the quantiser's launch: 33.5 -> 11.2 us; 2048 x 2048
 // 13.0 -> 7.6; Q6_K 2048 x 11008 40.0 -> 19.6.
